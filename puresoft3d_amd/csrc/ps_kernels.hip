@@ -15,10 +15,10 @@
 //  segment : one thread per span walks it and writes its pieces; a wave's
 //            pieces of one tile form one run of consecutive pieces, placed by
 //            one atomic on the tile's counter
-//  raster  : one wave per tile of 64 bins, lane = bin (a row piece of
-//            chunk_w pixels); the wave puts its tile's runs in wave order,
-//            which is submission order, and each lane walks its bin's spans
-//            in triangle order, keeping depth and the winning span in LDS
+//  raster  : one wave per tile of 64 bins (a bin is a row piece of chunk_w
+//            pixels); the wave puts its tile's runs in wave order, which is
+//            submission order, and takes the pieces 64 at a time, one per
+//            lane, keeping each pixel's depth and winner in LDS
 //            (fragthrd.cpp:208-252); depth test -1 < z && z - d < -1e-4
 //  shade   : one thread per pixel whose last colour-writing depth-test pass
 //            is known: re-derives that span's varyings, walks them serially
@@ -58,25 +58,36 @@ __device__ __forceinline__ void ps_commit_pending(PsCounters* c)
     }
 }
 
-__device__ __forceinline__ int ps_view_of_tile(const PsFrame& f, int64_t t)
+// The last view whose base is at most t (t the same in the whole wave, every
+// lane active): 64 bases at a time, one per lane, so that up to 64 views cost
+// one load, where a binary search makes a chain of six.
+template <typename Base>
+__device__ __forceinline__ int ps_find_view(int n, int64_t t, Base base)
 {
-    int lo = 0, hi = f.n_views - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (f.views[mid].tile_base <= t) lo = mid; else hi = mid - 1;
+    const int lane = threadIdx.x & 63;
+    int lo = 0, hi = n;   // views[lo] is at or below t; hi == n or views[hi] above it
+    while (hi - lo > 1) {
+        const int step = (hi - lo + 63) / 64, p = lo + lane * step;
+        const int c = __popcll(__ballot(p < hi && base(p) <= t));
+        lo += (c - 1) * step;
+        hi = min(hi, lo + step);
     }
     return lo;
 }
 
+__device__ __forceinline__ int ps_view_of_tile(const PsFrame& f, int64_t t)
+{
+    return ps_find_view(f.n_views, t, [&](int v) { return f.views[v].tile_base; });
+}
+
 __device__ __forceinline__ int ps_view_of_stile(const PsFrame& f, int64_t t)
 {
-    int lo = 0, hi = f.n_views - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (f.views[mid].stile_base <= t) lo = mid; else hi = mid - 1;
-    }
-    return lo;
+    return ps_find_view(f.n_views, t, [&](int v) { return f.views[v].stile_base; });
 }
+
+// Row pitch of a view's winner plane: rows start 32 bytes aligned, so that a
+// raster lane stores its chunk in one instruction.
+__device__ __forceinline__ int64_t ps_winner_at(const PsView& V, int x, int y) { return (int64_t)y * PS_WINNER_PITCH(V.W) + x; }
 
 // Workgroups are dealt to the 8 XCDs round-robin (workgroup b runs on XCD
 // b % 8), and each XCD has its own L2.  This maps workgroups to logical
@@ -519,7 +530,13 @@ __global__ void __launch_bounds__(128, 3) k_setup(const PsDraw* __restrict__ dra
 // ---------------------------------------------------------------------------
 #define SCAN_ITEMS 16
 #define SCAN_BLOCK (256 * SCAN_ITEMS)
-#define PS_HEAVY_CAP 1024
+
+// Most heavy tiles a flush of n tiles lists: no more than a third of them can
+// hold three times the mean.  At 1,024 a 3840x2160 frame's list was full and
+// half its longest tiles began 30 us into the kernel, which they ended at
+// 64 us; with all of them listed, and whole chunks stored at once, at 45.
+#define PS_HEAVY_MAX 4096
+__host__ __device__ __forceinline__ int64_t ps_heavy_cap(int64_t n) { return n / 3 + 1 < PS_HEAVY_MAX ? n / 3 + 1 : PS_HEAVY_MAX; }
 
 // Pieces that make a tile heavy: three times the flush's mean per tile (at
 // least 96).  The flush's pieces are k_span's 64-bit count in the pending
@@ -650,12 +667,12 @@ __device__ __forceinline__ uint32_t ps_heavy_reserve(uint32_t nh, uint32_t* heav
 
 // The wave's exclusive prefix of its items (from `run` on) into out.  Tile
 // scans (T = uint64, heavy given) also list the tiles of at least heavy_min
-// pieces in heavy[1 ..], the lane's from slot hslot on (up to PS_HEAVY_CAP
-// are listed), and mark the listed ones with bit 63 of their start.
+// pieces in heavy[1 ..], the lane's from slot hslot on (up to hcap are
+// listed), and mark the listed ones with bit 63 of their start.
 template <typename T>
 __device__ __forceinline__ void ps_store_scan(T* out, int64_t wbase, int64_t n, const T* v, T run,
                                               uint32_t heavy_min = 0xffffffffu, uint32_t* heavy = nullptr,
-                                              uint32_t hslot = 0xffffffffu)
+                                              uint32_t hslot = 0xffffffffu, uint32_t hcap = 0)
 {
     constexpr int PER = 16 / sizeof(T);
     const int lane = threadIdx.x & 63;
@@ -673,7 +690,7 @@ __device__ __forceinline__ void ps_store_scan(T* out, int64_t wbase, int64_t n, 
             o[j] = r;
             if constexpr (sizeof(T) == 8) {
                 if (hslot != 0xffffffffu && i + j < n && (uint32_t)v[g * PER + j] >= heavy_min) {
-                    if (hslot < PS_HEAVY_CAP) {
+                    if (hslot < hcap) {
                         heavy[1 + hslot] = (uint32_t)(i + j);
                         o[j] |= 1ull << 63;
                     }
@@ -785,13 +802,14 @@ __global__ void __launch_bounds__(256) k_scan_final(const T* __restrict__ in, co
     // the waves before this one: the block scan of the lane sums, taken at lane 0
     const T wpre = ps_block_excl_scan<T, 4>(s, lds, tot);
     uint32_t hm = 0xffffffffu, hslot = 0xffffffffu;
+    const uint32_t hcap = (uint32_t)ps_heavy_cap(n);
     if constexpr (sizeof(T) == 8) {
         if (heavy) {
             hm = ps_heavy_min(ps_pend_approx(pend), n);
             hslot = ps_heavy_reserve(ps_heavy_count(wbase, n, v, hm), heavy);
         }
     }
-    ps_store_scan(out, wbase, n, v, before + ps_wave_bcast0(wpre), hm, heavy, hslot);
+    ps_store_scan(out, wbase, n, v, before + ps_wave_bcast0(wpre), hm, heavy, hslot, hcap);
 }
 
 // One pass for tile counts up to SCAN_DIRECT_MAX.  Blocks of 16 waves; each
@@ -872,9 +890,10 @@ __global__ void __launch_bounds__(1024) k_scan_direct(const unsigned long long* 
     uint32_t hs = hbefore + hwoff + hown - (ha + hb);      // its first heavy slot
     T oa = r, ob = r + va;
     if (heavy) {
-        if (ha && hs < PS_HEAVY_CAP) { heavy[1 + hs] = (uint32_t)i; oa |= 1ull << 63; }
+        const uint32_t hcap = (uint32_t)ps_heavy_cap(n);
+        if (ha && hs < hcap) { heavy[1 + hs] = (uint32_t)i; oa |= 1ull << 63; }
         hs += ha;
-        if (hb && hs < PS_HEAVY_CAP) { heavy[1 + hs] = (uint32_t)(i + 1); ob |= 1ull << 63; }
+        if (hb && hs < hcap) { heavy[1 + hs] = (uint32_t)(i + 1); ob |= 1ull << 63; }
     }
     if (i + 2 <= n) {
         *(ulonglong2*)(out + i) = make_ulonglong2(oa, ob);
@@ -1314,18 +1333,36 @@ __global__ void __launch_bounds__(256, NVC <= 14 ? 5 : 1) k_segments(const PsSpa
 // ---------------------------------------------------------------------------
 // tile lists: the runs of a tile in submission order
 // ---------------------------------------------------------------------------
-// bitonic sort of one (key, value) pair per lane over lanes [0, np), np a
-// power of two up to 64, ascending by key
-__device__ __forceinline__ void ps_sort_lanes(uint32_t& key, uint32_t& val, int np)
+// For each lane's keys key[0 .. Q): how many of the n keys they are compared
+// with lie below.  Those are held one per lane in `other` (lanes from n on are
+// not looked at); each is read from its lane by a constant index, so a key
+// costs a read lane and Q compares and adds, without a cross-lane round trip
+// (a bitonic network makes two in each of up to 21 dependent steps).
+template <int Q>
+__device__ __forceinline__ void ps_count_below(const uint32_t* key, uint32_t other, uint32_t n, uint32_t* rank)
 {
-    const int lane = threadIdx.x & 63;
-    for (int k = 2; k <= np; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            const uint32_t ok = __shfl_xor(key, j, 64), ov = __shfl_xor(val, j, 64);
-            const bool up = (lane & k) == 0, low = (lane & j) == 0;
-            if (low == up ? ok < key : ok > key) { key = ok; val = ov; }
+#pragma unroll
+    for (int g = 0; g < 64; g += 8) {
+        if ((uint32_t)g >= n) break;
+#pragma unroll
+        for (int i = g; i < g + 8; i++) {
+            const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)other, i);   // 0xffffffff past the last: below none
+#pragma unroll
+            for (int q = 0; q < Q; q++) rank[q] += o < key[q] ? 1u : 0u;
         }
     }
+}
+
+// sorts one (key, value) pair per lane by key over lanes [0, n); the keys are
+// distinct, those of the lanes from n on are 0xffffffff
+__device__ __forceinline__ void ps_sort_lanes(uint32_t& key, uint32_t& val, uint32_t n)
+{
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t rank = 0;
+    ps_count_below<1>(&key, key, n, &rank);
+    const int to = (int)(lane < n ? rank : lane) * 4;
+    key = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)key);
+    val = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)val);
 }
 
 // The runs of a tile are written in the order their atomics happened.  Ordered
@@ -1348,7 +1385,7 @@ __device__ __forceinline__ void ps_run_window(const uint32_t* rl, uint32_t nr, u
     if (nr <= 64) {
         uint32_t key = j < nr ? rl[2 * j + 1] : 0xffffffffu;
         rbase = j < nr ? rl[2 * j] : 0u;
-        ps_sort_lanes(key, rbase, np);
+        ps_sort_lanes(key, rbase, nw);
         const uint32_t c = j < nr ? (key & 0xfffu) + 1u : 0u;
         const uint32_t incl = ps_wave_incl_scan(c);
         rv = j < nr ? incl - c : 0xffffffffu;
@@ -1360,7 +1397,7 @@ __device__ __forceinline__ void ps_run_window(const uint32_t* rl, uint32_t nr, u
     }
 }
 
-// the piece at list position v of the window (rv[0] <= v): the last run that
+// the piece at list position v of the window (rv[0] <= v; the walk that blends): the last run that
 // starts at or before v, found by a binary search over lanes [0, np)
 __device__ __forceinline__ uint32_t ps_run_piece(uint32_t rv, uint32_t rbase, uint32_t v, int np)
 {
@@ -1451,9 +1488,135 @@ __device__ uint32_t* ps_order_runs(uint32_t* a, uint32_t* b, uint32_t nr, uint32
 // counts and offsets
 #define RA_WORDS(cw) ((cw) * 64 * 2 + RA_CHUNK * 7 + 128)
 
-// KCW: the chunk width when it is 1, 2, 4 or 8, else 0.  With a known width
-// each lane keeps its pixels' depth and winner in registers, so the walk has
-// no LDS round trip per pixel; the LDS columns serve wider chunks.
+// LDS of one wave of k_raster: the runs of a tile of 65 to PS_LDS_RUNS runs in
+// order (first piece, list position), which run starts at each position of a
+// batch, a spare pixel per lane, then depth and winner of the tile's pixels, pixel k of lane l's chunk
+// at [k * 64 + l]
+#define PS_LDS_RUNS 256
+#define RA_PIX_WORDS(cw) (PS_LDS_RUNS * 2 + 64 + 64 * 2 + (cw) * 64 * 2)
+
+// keeps the compiler from moving LDS accesses across: the LDS operations of a
+// wave are performed in order
+__device__ __forceinline__ void ps_lds_turn()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The runs of a tile of 65 to PS_LDS_RUNS runs, sorted by wave and with each
+// key replaced by the list position of the run's first piece, into the wave's
+// LDS: every key is counted against all of them (1 us for 128 runs), where
+// sorting them in global memory takes several dependent passes over it
+// (11 to 38 us, the longest part of the tiles that end the kernel).
+__device__ __forceinline__ void ps_sort_runs_lds(const uint32_t* rl, uint32_t nr, uint2* out)
+{
+    constexpr int Q = PS_LDS_RUNS / 64;
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t key[Q], val[Q], rank[Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        const uint32_t j = q * 64 + lane;
+        const uint2 r = j < nr ? *(const uint2*)(rl + 2 * j) : make_uint2(0u, 0xffffffffu);
+        val[q] = r.x;
+        key[q] = r.y;
+        rank[q] = 0;
+    }
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+        if (nr > 64u * q) ps_count_below<Q>(key, key[q], min(nr - 64u * q, 64u), rank);
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+        if (q * 64 + lane < nr) out[rank[q]] = make_uint2(val[q], (key[q] & 0xfffu) + 1u);
+    ps_lds_turn();
+    uint32_t carry = 0;
+    for (uint32_t j0 = 0; j0 < nr; j0 += 64) {
+        const uint32_t j = j0 + lane;
+        const uint2 r = j < nr ? out[j] : make_uint2(0u, 0u);
+        const uint32_t incl = ps_wave_incl_scan(r.y);
+        if (j < nr) out[j].y = carry + incl - r.y;
+        carry += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    }
+    ps_lds_turn();
+}
+
+// inclusive maximum over the lanes
+__device__ __forceinline__ uint32_t ps_wave_incl_max(uint32_t v)
+{
+    v = max(v, (uint32_t)PS_DPP(v, 0x111, 0xf, true));
+    v = max(v, (uint32_t)PS_DPP(v, 0x112, 0xf, true));
+    v = max(v, (uint32_t)PS_DPP(v, 0x114, 0xf, true));
+    v = max(v, (uint32_t)PS_DPP(v, 0x118, 0xf, true));
+    v = max(v, (uint32_t)PS_DPP(v, 0x142, 0xa, false));
+    v = max(v, (uint32_t)PS_DPP(v, 0x143, 0xc, false));
+    return v;
+}
+
+// A lane's run of n (at most N) words at p, in the widest accesses that its
+// length and alignment allow: whole runs of rows 16 bytes aligned (8 for two
+// words) go in one instruction.
+template <int N>
+__device__ __forceinline__ void ps_load_run(const uint32_t* p, int n, uint32_t* v)
+{
+    constexpr int A = N >= 4 ? 16 : 4 * N;
+    if (n == N && ((uintptr_t)p & (A - 1)) == 0) {
+        if constexpr (N >= 4) {
+#pragma unroll
+            for (int k = 0; k < N; k += 4) {
+                const uint4 q = *(const uint4*)(p + k);
+                v[k] = q.x; v[k + 1] = q.y; v[k + 2] = q.z; v[k + 3] = q.w;
+            }
+        } else if constexpr (N == 2) {
+            const uint2 q = *(const uint2*)p;
+            v[0] = q.x; v[1] = q.y;
+        } else {
+            v[0] = p[0];
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < N; k++) v[k] = k < n ? p[k] : 0u;
+    }
+}
+
+template <int N>
+__device__ __forceinline__ void ps_store_run(uint32_t* p, int n, const uint32_t* v)
+{
+    constexpr int A = N >= 4 ? 16 : 4 * N;
+    if (n == N && ((uintptr_t)p & (A - 1)) == 0) {
+        if constexpr (N >= 4) {
+#pragma unroll
+            for (int k = 0; k < N; k += 4) *(uint4*)(p + k) = make_uint4(v[k], v[k + 1], v[k + 2], v[k + 3]);
+        } else if constexpr (N == 2) {
+            *(uint2*)p = make_uint2(v[0], v[1]);
+        } else {
+            p[0] = v[0];
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < N; k++)
+            if (k < n) p[k] = v[k];
+    }
+}
+
+// One wave per tile; the wave takes the tile's pieces 64 at a time, one per
+// lane, in submission order.  Each lane evaluates its own piece's depths, so
+// the divisions run on full waves whatever chunk the pieces fall in, and the
+// order-dependent test is resolved per pixel in rounds: among the lanes whose
+// piece covers pixel k of the same chunk, the one with r such lanes before it
+// goes in round r, against the depth the rounds before it left in LDS.  A
+// batch takes one round unless its pieces overlap.  While every piece of the
+// batch tests depth, a pixel's depth only falls, so a fragment that fails
+// against the depth at the batch's start fails in its turn too and takes no
+// round.
+// The walk this replaced (each lane its chunk's pieces, one after the other,
+// from lists split in LDS) ran as long as the fullest of the 64 chunks.  What
+// bounds it is a wave's chain of LDS and cross-lane latencies, some 3,000
+// cycles a batch; its own work per pixel is small.  Before and after, default
+// tiles: 3840x2160 terrain (2.8M pieces) 113 -> 45 us, 32 views of 256^2 to
+// 1024^2 (3.7M) 158 -> 77, 515x389 (86k, as long as its longest tile) 37 ->
+// 21; 1920x1080 in 16x8 tiles (1.1M) 33 -> 22.
+// KCW: the chunk width when it is 1, 2, 4 or 8 (a batch's pixels are then
+// unrolled and share their rounds), else 0.
 template <bool DEBUG, int KCW>
 __global__ void __launch_bounds__(512, 5) k_raster(const PsSpan* __restrict__ spans, const PsSeg* __restrict__ segs,
                          const PsTri* __restrict__ tris, const PsDraw* __restrict__ draws, PsFrame f, int64_t n_tiles,
@@ -1465,37 +1628,30 @@ __global__ void __launch_bounds__(512, 5) k_raster(const PsSpan* __restrict__ sp
     int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int waves = blockDim.x >> 6;
     // neighbouring tiles share an L2; with a heavy-tile list, the first
-    // PS_HEAVY_CAP waves take the listed tiles (they start first, so the
+    // waves take the listed tiles (they start first, so the
     // longest walks do not end the kernel), the others every unlisted tile
     // (the list and the marks are in bounds, stale or not)
     int64_t tile = ps_xcd_remap<4>(blockIdx.x, gridDim.x) * (int64_t)waves + wave;
     bool skip = false;
     if (f.heavy) {
-        if (tile < PS_HEAVY_CAP) {
-            const uint32_t listed = min(f.heavy[0], (uint32_t)PS_HEAVY_CAP);
+        const int64_t hcap = ps_heavy_cap(n_tiles);
+        if (tile < hcap) {
+            const uint32_t listed = min(f.heavy[0], (uint32_t)hcap);
             const uint32_t t = f.heavy[1 + tile];
             skip = tile >= listed;
             tile = t;
         } else {
-            tile -= PS_HEAVY_CAP;
+            tile -= hcap;
             skip = tile >= n_tiles || (f.tstart[min(tile, n_tiles)] >> 63);
         }
     }
     if (poisoned) return;
     ps_commit_pending(cnt);
     if (skip || tile >= n_tiles) return;
-    uint32_t* wl = lds + (size_t)wave * RA_WORDS(KCW ? 0 : CW);
-    float* dep = (float*)wl;                       // LDS columns: chunks wider than 8 only
-    int* win = (int*)(dep + (KCW ? 0 : CW) * 64);
-    uint32_t* r_s = (uint32_t*)(win + (KCW ? 0 : CW) * 64);   // winner code (triangle, or checkpoint | piece)
-    uint32_t* r_fl = r_s + RA_CHUNK;               // behaviour | writes colour (PsSeg.si high bits)
-    uint32_t* r_x = r_fl + RA_CHUNK;               // xa | xb << 16
-    float* r_cf2 = (float*)(r_x + RA_CHUNK);
-    float* r_pz = r_cf2 + RA_CHUNK;
-    float* r_cst = r_pz + RA_CHUNK;
-    float* r_pst = r_cst + RA_CHUNK;
-    uint32_t* lcnt = (uint32_t*)(r_pst + RA_CHUNK);
-    uint32_t* loff = lcnt + 64;
+    uint2* lruns = (uint2*)(lds + (size_t)wave * RA_PIX_WORDS(CW));
+    uint32_t* starts = (uint32_t*)(lruns + PS_LDS_RUNS);
+    uint2* spare = (uint2*)(starts + 64) + lane;
+    uint2* pix = (uint2*)(starts + 64) + 64;   // x: depth bits, y: winner code
 
     const int cw_shift = __builtin_ctz((unsigned)CW), tc_shift = __builtin_ctz((unsigned)f.tile_cols);
     const PsView& V = f.views[ps_view_of_tile(f, tile)];
@@ -1503,216 +1659,208 @@ __global__ void __launch_bounds__(512, 5) k_raster(const PsSpan* __restrict__ sp
     // a view has fewer than 2^31 tiles; tile_cols is a power of two
     const uint32_t lt32 = (uint32_t)ltile, ntx = (uint32_t)V.n_tiles_x;
     int ty = (int)(lt32 / ntx), tx = (int)(lt32 - (uint32_t)ty * ntx);
-    int ry = lane >> tc_shift, rx = lane & (f.tile_cols - 1);
-    int y = ty * f.tile_rows + ry;
-    int cx = tx * f.tile_cols + rx;
-    int X0 = cx * CW;
+    int y = ty * f.tile_rows + (lane >> tc_shift);
+    int X0 = (tx * f.tile_cols + (lane & (f.tile_cols - 1))) * CW;
     const int VW = V.W;
-    bool inside = y < V.H && X0 < VW;
-    int ncol = inside ? min(CW, VW - X0) : 0;
+    const int ncol = y < V.H && X0 < VW ? min(CW, VW - X0) : 0;
     float* drow = V.depth + (int64_t)y * V.depth_scan;
     // a clear fused into the flush: the tile starts from its value, and the
     // whole tile is written back
     const bool dclear = V.dclear != 0;
-    float dv[KCW ? KCW : 1];
-    int wv[KCW ? KCW : 1];
-    if constexpr (KCW > 0) {
-#pragma unroll
-        for (int k = 0; k < KCW; k++) {
-            dv[k] = k < ncol ? (dclear ? V.dclear_value : drow[X0 + k]) : 1.0f;
-            wv[k] = -1;
-        }
-    } else {
-        for (int c = 0; c < ncol; c++) {
-            dep[c * 64 + lane] = dclear ? V.dclear_value : drow[X0 + c];
-            win[c * 64 + lane] = -1;
-        }
-    }
-    unsigned long long passes = 0;
-    bool dirty = dclear;
-    const uint64_t lt = ps_lt_mask();
     // the tile's runs in submission order, up to 64 at a time (one per lane)
     const unsigned long long ta = PS_TS(f.tstart[tile]), tb = PS_TS(f.tstart[tile + 1]);
     const uint32_t n_list = (uint32_t)tb - (uint32_t)ta;
     const uint32_t r0 = (uint32_t)(ta >> 32), nr = (uint32_t)(tb >> 32) - r0;
     const uint32_t* rl = f.runs + 2 * (size_t)r0;
-    if (nr > 64) rl = ps_order_runs(f.runs + 2 * (size_t)r0, f.runs2 + 2 * (size_t)r0, nr, lcnt);
-    for (uint32_t w0 = 0; w0 < nr; w0 += 64) {
-        uint32_t rbase, rv, vhi;
-        int np;
-        ps_run_window(rl, nr, w0, n_list, rbase, rv, vhi, np);
-        const uint32_t vlo = __builtin_amdgcn_readlane(rv, 0);
-        // software pipeline over chunks of the window: while chunk i is split
-        // and walked, the records of chunk i+1 are in flight
-        uint32_t vn[RA_PER];
-        uint4 ran[RA_PER], rbn[RA_PER];
+    const bool in_lds = nr > 64 && nr <= PS_LDS_RUNS;
+    if (in_lds) ps_sort_runs_lds(rl, nr, lruns);
+    else if (nr > 64) rl = ps_order_runs(f.runs + 2 * (size_t)r0, f.runs2 + 2 * (size_t)r0, nr, (uint32_t*)lruns);
+    if constexpr (KCW > 0) {
+        uint32_t d[KCW];
+        if (dclear) {
 #pragma unroll
-        for (int k = 0; k < RA_PER; k++) {
-            uint32_t e = vlo + k * 64 + lane;
-            uint32_t pp = ps_run_piece(rv, rbase, e, np);
-            vn[k] = e < vhi ? pp : 0u;
-            const uint4* p = (const uint4*)(segs + vn[k]);
-            ran[k] = e < vhi ? p[0] : make_uint4(0, 0, 0, 0);
-            rbn[k] = e < vhi ? p[1] : make_uint4(0, 0, 0, 0);
+            for (int k = 0; k < KCW; k++) d[k] = __float_as_uint(V.dclear_value);
+        } else {
+            ps_load_run<KCW>((const uint32_t*)drow + X0, ncol, d);
         }
-        for (uint32_t cb = vlo; cb < vhi; cb += RA_CHUNK) {
-            uint32_t ce = min(vhi, cb + RA_CHUNK);
-            uint32_t v[RA_PER], key[RA_PER];
-            uint4 ra[RA_PER], rb[RA_PER];
 #pragma unroll
-            for (int k = 0; k < RA_PER; k++) {
-                v[k] = vn[k];
-                ra[k] = ran[k];
-                rb[k] = rbn[k];
+        for (int k = 0; k < KCW; k++) pix[k * 64 + lane] = make_uint2(d[k], 0xffffffffu);
+    } else {
+        for (int k = 0; k < ncol; k++)
+            pix[k * 64 + lane] = make_uint2(__float_as_uint(dclear ? V.dclear_value : drow[X0 + k]), 0xffffffffu);
+    }
+    uint32_t passes = 0;   // the lane's; a list has at most 2^31 pieces of 64 pixels
+    bool dirty = dclear;
+    ps_lds_turn();
+    for (uint32_t w0 = 0; w0 < nr; w0 += 64) {
+        // the window's runs, one per lane: list position of the first piece
+        // (0xffffffff past the last run), and what to add to a list position
+        // in the run to get its piece
+        uint32_t rbase, rv, vhi;
+        if (in_lds) {
+            const uint32_t j = w0 + lane;
+            const uint2 r = j < nr ? lruns[j] : make_uint2(0u, 0xffffffffu);
+            rbase = r.x;
+            rv = r.y;
+            vhi = w0 + 64 < nr ? lruns[w0 + 64].y : n_list;
+        } else {
+            int np;
+            ps_run_window(rl, nr, w0, n_list, rbase, rv, vhi, np);
+        }
+        const uint32_t vlo = (uint32_t)__builtin_amdgcn_readlane((int)rv, 0), delta = rbase - rv;
+        // the records of the next batch are in flight while one is tested.  A
+        // batch's pieces: each run that starts in it marks its first position,
+        // a running maximum over the positions gives every lane its run.
+        uint4 ran, rbn;
+        uint32_t run = 0;   // one more than the run of the last position before the batch
+        auto gather = [&](uint32_t c) {
+            starts[lane] = 0;
+            ps_lds_turn();
+            if (rv - c < 64u) starts[rv - c] = (uint32_t)lane + 1u;
+            ps_lds_turn();
+            const uint32_t m = max(ps_wave_incl_max(starts[lane]), run);
+            ps_lds_turn();
+            run = (uint32_t)__builtin_amdgcn_readlane((int)m, 63);
+            const uint32_t e = c + lane;
+            const uint32_t pp = e + (uint32_t)__builtin_amdgcn_ds_bpermute((int)(m - 1u) * 4, (int)delta);
+            const uint4* p = (const uint4*)(segs + (e < vhi ? pp : 0u));
+            ran = p[0];
+            rbn = p[1];
+        };
+        gather(vlo);
+        for (uint32_t cb = vlo; cb < vhi; cb += 64) {
+            const uint4 ra = ran, rb = rbn;
+            const bool valid = cb + lane < vhi;
+            if (cb + 64 < vhi) gather(cb + 64);
+            // the piece's chunk in the tile and its pixels [a, b] of it
+            const int xa = (int)(ra.y & 0xffffu), pcx = xa >> cw_shift;
+            const int key = (((int)rb.z & (f.tile_rows - 1)) << tc_shift) | (pcx & (f.tile_cols - 1));
+            const int a = xa - (pcx << cw_shift), b = valid ? (int)(ra.y >> 16) - (pcx << cw_shift) : -1;
+            const bool test = (ra.x >> 26) & PSGPU_TEST_DEPTH, upd = (ra.x >> 26) & PSGPU_UPDATE_DEPTH, wc = (ra.x >> 28) & 1;
+            const uint32_t wcode = rb.w;
+            float cf2 = __uint_as_float(ra.z), pz = __uint_as_float(ra.w);
+            const float cst = __uint_as_float(rb.x), pst = __uint_as_float(rb.y);
+            uint32_t th = 0;
+            int tid = 0;
+            if (DEBUG && valid) {
+                int tri = (wcode & PS_SEG_CK) ? spans[segs[wcode & ~PS_SEG_CK].si & PS_SEG_SPAN_MASK].tri : (int)wcode;
+                const PsDraw& d = draws[tris[tri].code >> 8];
+                tid = (int)(d.id_base + (tri - d.tri_start));
+                uint32_t h = (uint32_t)tid;
+                h ^= h >> 16; h *= 0x85ebca6bu; h ^= h >> 13; h *= 0xc2b2ae35u; h ^= h >> 16;
+                th = h;
             }
-            if (cb + RA_CHUNK < vhi) {
+            // lanes of the same chunk
+            uint64_t same = ~0ull;
 #pragma unroll
-                for (int k = 0; k < RA_PER; k++) {
-                    uint32_t e = cb + RA_CHUNK + k * 64 + lane;
-                    uint32_t pp = ps_run_piece(rv, rbase, e, np);
-                    vn[k] = e < vhi ? pp : 0u;
-                    const uint4* p = (const uint4*)(segs + vn[k]);
-                    ran[k] = e < vhi ? p[0] : make_uint4(0, 0, 0, 0);
-                    rbn[k] = e < vhi ? p[1] : make_uint4(0, 0, 0, 0);
+            for (int bit = 0; bit < 6; bit++) {
+                const uint64_t m = __ballot((key >> bit) & 1);
+                same &= ((key >> bit) & 1) ? m : ~m;
+            }
+            const bool all_test = __all(test || !valid);
+            // candidates before this lane at the same pixel
+            auto rank_of = [&](bool cand) {
+                const uint64_t m = same & __ballot(cand);
+                return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+            };
+            // the lane's depth at pixel k, interpolateNextStep (interp.cpp:82-92)
+            auto depth_at = [&](bool in) {
+                const float r = 1.0f / cf2, z = pz * r;
+                cf2 = in ? cf2 + cst : cf2;
+                pz = in ? pz + pst : pz;
+                return z;
+            };
+            // fragthrd.cpp:216-237 against the pixel's depth and winner
+            auto fragment = [&](bool turn, int k, float z, uint2 cur) {
+                const float d = test ? __uint_as_float(cur.x) : 1.0f;
+                const bool pass = turn & (z - d < -0.0001f);
+                if (upd) cur.x = __float_as_uint(z);
+                if (wc) cur.y = wcode;
+                // a fragment that fails, or whose turn it is not, goes to the
+                // lane's own spare slot: selecting the address costs less
+                // than masking the store
+                *(pass ? pix + k * 64 + key : spare) = cur;
+                passes += pass ? 1u : 0u;
+                dirty |= pass & upd;
+                if (DEBUG && pass) {
+                    const int64_t at = (int64_t)(int)rb.z * VW + ((pcx << cw_shift) + k);
+                    atomicAdd(&f.dbg_pcount[at], 1);
+                    atomicXor(&f.dbg_phash[at], th);
+                    f.dbg_last[at] = tid;
                 }
-            }
+            };
+            auto drawn = [&](int k) {   // every rasterised fragment, passing or not
+                const int64_t at = (int64_t)(int)rb.z * VW + ((pcx << cw_shift) + k);
+                atomicAdd(&f.dbg_rcount[at], 1);
+                atomicXor(&f.dbg_rhash[at], th);
+            };
+            if constexpr (KCW > 0) {
+                // every lane evaluates every pixel of the chunk, so that the
+                // divisions and the LDS reads overlap
+                float z[KCW];
+                uint2 cur[KCW];
+                bool cand[KCW];
+                int rank[KCW], last = 0;
 #pragma unroll
-            for (int k = 0; k < RA_PER; k++) {
-                // the piece's lane: its row inside the tile and its chunk inside the row
-                int py = (int)rb[k].z, pcx = (int)(ra[k].y & 0xffffu) >> cw_shift;
-                key[k] = (uint32_t)(((py & (f.tile_rows - 1)) << tc_shift) | (pcx & (f.tile_cols - 1)));
-            }
-            // stable split by lane key: each entry's rank among the equal keys
-            // before it (the same-key lanes of its group of 64 by ballots, plus
-            // the count of earlier groups), then per-key offsets, then placement
-            lcnt[lane] = 0;
-            __builtin_amdgcn_wave_barrier();
-            uint32_t rank[RA_PER];
+                for (int k = 0; k < KCW; k++) cur[k] = pix[k * 64 + key];
 #pragma unroll
-            for (int k = 0; k < RA_PER; k++) {
-                uint32_t e = cb + k * 64 + lane;
-                bool valid = e < ce;
-                uint32_t kk = key[k];
-                uint64_t same = __ballot(valid);
-#pragma unroll
-                for (int bit = 0; bit < 6; bit++) {
-                    uint64_t m = __ballot((kk >> bit) & 1u);
-                    same &= ((kk >> bit) & 1u) ? m : ~m;
+                for (int k = 0; k < KCW; k++) {
+                    const bool in = (k >= a) & (k <= b);
+                    z[k] = depth_at(in);
+                    if (DEBUG && in) drawn(k);
+                    cand[k] = in & (-1.0f < z[k]) & (!all_test | (z[k] - __uint_as_float(cur[k].x) < -0.0001f));
                 }
-                uint32_t before = (uint32_t)__popcll(same & lt);
-                uint32_t cur = lcnt[kk];
-                rank[k] = cur + before;
-                __builtin_amdgcn_wave_barrier();
-                if (valid && before == 0) lcnt[kk] = cur + (uint32_t)__popcll(same);
-                __builtin_amdgcn_wave_barrier();
-            }
-            {
-                uint32_t cntv = lcnt[lane];
-                uint32_t x = cntv;
 #pragma unroll
-                for (int o = 1; o < 64; o <<= 1) {
-                    uint32_t yv = __shfl_up(x, o, 64);
-                    if (lane >= o) x += yv;
+                for (int k = 0; k < KCW; k++) {
+                    rank[k] = rank_of(cand[k]);
+                    last = cand[k] ? max(last, rank[k]) : last;
                 }
-                loff[lane] = x - cntv;
-                __builtin_amdgcn_wave_barrier();
-            }
 #pragma unroll
-            for (int k = 0; k < RA_PER; k++) {
-                uint32_t e = cb + k * 64 + lane;
-                if (e < ce) {
-                    uint32_t q = loff[key[k]] + rank[k];
-                    r_s[q] = rb[k].w;
-                    r_fl[q] = ra[k].x & ~PS_SEG_SPAN_MASK;
-                    r_x[q] = ra[k].y;
-                    r_cf2[q] = __uint_as_float(ra[k].z);
-                    r_pz[q] = __uint_as_float(ra[k].w);
-                    r_cst[q] = __uint_as_float(rb[k].x);
-                    r_pst[q] = __uint_as_float(rb[k].y);
+                for (int k = 0; k < KCW; k++) fragment(cand[k] & (rank[k] == 0), k, z[k], cur[k]);
+                if (DEBUG) __threadfence();   // the last pass of a pixel is stored last
+                ps_lds_turn();
+                for (int r = 1; __any(last >= r); r++) {
+#pragma unroll
+                    for (int k = 0; k < KCW; k++) cur[k] = pix[k * 64 + key];
+#pragma unroll
+                    for (int k = 0; k < KCW; k++) fragment(cand[k] & (rank[k] == r), k, z[k], cur[k]);
+                    if (DEBUG) __threadfence();
+                    ps_lds_turn();
                 }
-            }
-            __builtin_amdgcn_wave_barrier();
-            if (inside) {
-                uint32_t l0 = loff[lane], l1 = l0 + lcnt[lane];
-                for (uint32_t q = l0; q < l1; q++) {
-                    const uint32_t wcode = r_s[q];
-                    uint32_t fl = r_fl[q];
-                    int beh = (fl >> 26) & 3;
-                    bool wc = (fl >> 28) & 1;
-                    uint32_t xab = r_x[q];
-                    int a = (int)(xab & 0xffffu), b = (int)(xab >> 16);
-                    float cf2 = r_cf2[q], pz = r_pz[q];
-                    const float cst = r_cst[q], pst = r_pst[q];
-                    uint32_t th = 0;
-                    int tid = 0;
-                    if (DEBUG) {
-                        int tri = (wcode & PS_SEG_CK) ? spans[segs[wcode & ~PS_SEG_CK].si & PS_SEG_SPAN_MASK].tri : (int)wcode;
-                        const PsTri tr = tris[tri];
-                        const PsDraw& d = draws[tr.code >> 8];
-                        tid = (int)(d.id_base + (tri - d.tri_start));
-                        uint32_t h = (uint32_t)tid;
-                        h ^= h >> 16; h *= 0x85ebca6bu; h ^= h >> 13; h *= 0xc2b2ae35u; h ^= h >> 16;
-                        th = h;
+            } else {
+                for (int k = 0; k < CW; k++) {
+                    const bool in = k >= a && k <= b;
+                    if (!__any(in)) continue;
+                    const float z = depth_at(in);
+                    if (DEBUG && in) drawn(k);
+                    const bool cand = in && -1.0f < z;
+                    const int rank = rank_of(cand);
+                    for (int r = 0; __any(cand && rank >= r); r++) {
+                        fragment(cand && rank == r, k, z, pix[k * 64 + key]);
+                        if (DEBUG) __threadfence();
+                        ps_lds_turn();
                     }
-                    if constexpr (KCW > 0) {
-                        // the chunk's pixels in order, those of [a, b] stepping the accumulators
-#pragma unroll
-                        for (int k = 0; k < KCW; k++) {
-                            const int x = X0 + k;
-                            if (x < a || x > b) continue;
-                            // interpolateNextStep (interp.cpp:82-92)
-                            float r = 1.0f / cf2;
-                            cf2 += cst;
-                            float z = pz * r;
-                            pz += pst;
-                            float cur = (beh & PSGPU_TEST_DEPTH) ? dv[k] : 1.0f;
-                            int64_t pix = (int64_t)y * VW + x;
-                            if (DEBUG) { f.dbg_rcount[pix] += 1; f.dbg_rhash[pix] ^= th; }
-                            // fragthrd.cpp:227
-                            if (-1.0f < z && (z - cur < -0.0001f)) {
-                                passes++;
-                                if (beh & PSGPU_UPDATE_DEPTH) { dv[k] = z; dirty = true; }
-                                if (wc) wv[k] = (int)wcode;
-                                if (DEBUG) { f.dbg_pcount[pix] += 1; f.dbg_phash[pix] ^= th; f.dbg_last[pix] = tid; }
-                            }
-                        }
-                    } else {
-                        for (int x = a; x <= b; x++) {
-                            // interpolateNextStep (interp.cpp:82-92)
-                            float r = 1.0f / cf2;
-                            cf2 += cst;
-                            float z = pz * r;
-                            pz += pst;
-                            int c = x - X0;
-                            float cur = (beh & PSGPU_TEST_DEPTH) ? dep[c * 64 + lane] : 1.0f;
-                            int64_t pix = (int64_t)y * VW + x;
-                            if (DEBUG) { f.dbg_rcount[pix] += 1; f.dbg_rhash[pix] ^= th; }
-                            // fragthrd.cpp:227
-                            if (-1.0f < z && (z - cur < -0.0001f)) {
-                                passes++;
-                                if (beh & PSGPU_UPDATE_DEPTH) { dep[c * 64 + lane] = z; dirty = true; }
-                                if (wc) win[c * 64 + lane] = (int)wcode;
-                                if (DEBUG) { f.dbg_pcount[pix] += 1; f.dbg_phash[pix] ^= th; f.dbg_last[pix] = tid; }
-                            }
-                        }
-                    }
                 }
             }
-            __builtin_amdgcn_wave_barrier();
         }
     }
-    int* wrow = V.winner + (int64_t)y * VW;
+    const bool write_depth = __any(dirty);
+    uint32_t* wrow = (uint32_t*)V.winner + ps_winner_at(V, 0, y);
     if constexpr (KCW > 0) {
+        uint32_t d[KCW], w[KCW];
 #pragma unroll
-        for (int k = 0; k < KCW; k++)
-            if (k < ncol) {
-                if (dirty) drow[X0 + k] = dv[k];
-                wrow[X0 + k] = wv[k];
-            }
+        for (int k = 0; k < KCW; k++) {
+            const uint2 p = pix[k * 64 + lane];
+            d[k] = p.x;
+            w[k] = p.y;
+        }
+        if (write_depth) ps_store_run<KCW>((uint32_t*)drow + X0, ncol, d);
+        ps_store_run<KCW>(wrow + X0, ncol, w);
     } else {
-        for (int c = 0; c < ncol; c++) {
-            if (dirty) drow[X0 + c] = dep[c * 64 + lane];
-            wrow[X0 + c] = win[c * 64 + lane];
+        for (int k = 0; k < ncol; k++) {
+            const uint2 p = pix[k * 64 + lane];
+            if (write_depth) drow[X0 + k] = __uint_as_float(p.x);
+            wrow[X0 + k] = p.y;
         }
     }
     ps_wave_add64(cnt, PS_ST_SHADED, passes);
@@ -1995,7 +2143,7 @@ __global__ void __launch_bounds__(256, 7) k_shade(const PsSpan* __restrict__ spa
     int y = sy * 16 + (threadIdx.x >> 4);
     if (x >= V.W || y >= V.H) return;
     const int64_t crow = V.colour_top_down ? (int64_t)(V.colour_h - 1 - y) : (int64_t)y;
-    int w = V.winner[(int64_t)y * V.W + x];
+    int w = V.winner[ps_winner_at(V, x, y)];
     if (poisoned) return;
     if (w == -1) {   // no fragment colours the pixel: a fused clear of its row, if any, is all it gets
         if (clears && crow < V.cclear_rows) V.colour[crow * V.colour_scan + x] = V.cclear_value;
@@ -2162,7 +2310,7 @@ void psk_scan_parts(hipStream_t s, const uint32_t* in, int64_t n, uint32_t* out,
                        bstart, bcap);
 }
 
-int psk_heavy_cap() { return PS_HEAVY_CAP; }
+int psk_heavy_cap() { return PS_HEAVY_MAX; }
 
 void psk_scan_tiles(hipStream_t s, const unsigned long long* tcnt, int64_t n, unsigned long long* tstart,
                     unsigned long long* partial, uint32_t* total_out, const PsCounters* c, uint32_t* heavy)
@@ -2220,8 +2368,8 @@ void psk_raster(hipStream_t s, bool debug, const PsSpan* spans, const PsSeg* seg
     int64_t n_tiles = f.n_tiles;
     const int cw = f.chunk_w;
     const bool known = cw == 1 || cw == 2 || cw == 4 || cw == 8;
-    size_t lds = psk_raster_lds(known ? 0 : cw, waves_per_group);
-    dim3 g(gsz(n_tiles + (f.heavy ? PS_HEAVY_CAP : 0), waves_per_group)), b(64 * waves_per_group);
+    size_t lds = (size_t)waves_per_group * RA_PIX_WORDS(cw) * 4;
+    dim3 g(gsz(n_tiles + (f.heavy ? ps_heavy_cap(n_tiles) : 0), waves_per_group)), b(64 * waves_per_group);
 #define RA_LAUNCH(D, K) hipLaunchKernelGGL((k_raster<D, K>), g, b, lds, s, spans, segs, tris, draws, f, n_tiles, cnt)
     switch (known ? cw : 0) {
     case 1: if (debug) RA_LAUNCH(true, 1); else RA_LAUNCH(false, 1); break;

@@ -99,6 +99,9 @@ struct PsSeg {
     uint32_t win;
 };
 
+// words per row of a view's winner plane (a multiple of 8)
+#define PS_WINNER_PITCH(w) (((int64_t)(w) + 7) & ~(int64_t)7)
+
 // One view of a flush: a viewport and its colour/depth targets.  A flush
 // renders any number of views with the same kernels; tiles and shading
 // blocks of all views are numbered consecutively.
@@ -110,7 +113,7 @@ struct PsView {
     int64_t stile_base;             // first shading block of the view
     uint32_t* colour; int colour_scan; int colour_top_down; int colour_h;  // scan in uint32
     float* depth; int depth_scan;   // scan in floats
-    // W*H: what shading needs of the last colour-writing pass: its triangle,
+    // H rows of PS_WINNER_PITCH(W): what shading needs of the last colour-writing pass: its triangle,
     // or PS_SEG_CK | its piece when the piece keeps a varying checkpoint;
     // -1 for none
     int* winner;

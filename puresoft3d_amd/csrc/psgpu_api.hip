@@ -473,7 +473,7 @@ int build_blob(psgpu_ctx* c, const Cmd& cmd, Blob& b, PsFrame& f, int64_t& T, in
         pv.cclear_rows = sg.cclear_rows;
         pv.cclear_value = sg.cclear_value;
         pv.winner = (int*)(intptr_t)n_pix;   // offset; rebased once the winner buffer is known
-        n_pix += (int64_t)pv.W * pv.H;
+        n_pix += PS_WINNER_PITCH(pv.W) * pv.H;
         views.push_back(pv);
         for (PsDraw d : sg.draws) {
             d.view = (int)v;
@@ -1197,7 +1197,7 @@ FlushShape flush_shape(psgpu_ctx* c, const Cmd& cmd)
     for (const Segment& sg : cmd.views) {
         int n_chunks = (sg.tg.vpw + cw - 1) / cw;
         sh.n_tiles += (int64_t)((n_chunks + tc - 1) / tc) * ((sg.tg.vph + tr - 1) / tr);
-        sh.n_pix += (int64_t)sg.tg.vpw * sg.tg.vph;
+        sh.n_pix += PS_WINNER_PITCH(sg.tg.vpw) * sg.tg.vph;
         for (const PsDraw& d : sg.draws) {
             sh.T += d.tri_count;
             sh.nvs = std::max(sh.nvs, d.nv);

@@ -918,9 +918,10 @@ struct PsRowWave {
 __global__ void __launch_bounds__(1024) k_scan_parts(const uint32_t* __restrict__ in, int64_t n,
                                                      const uint32_t* __restrict__ partial, int pgran,
                                                      uint32_t* __restrict__ out, uint32_t* total_out,
-                                                     uint32_t* __restrict__ bstart, int64_t bcap)
+                                                     uint32_t* __restrict__ bstart, int64_t bcap, uint32_t* wide)
 {
     __shared__ PsRowWave xw[16];
+    if (blockIdx.x == 0 && threadIdx.x == 0) wide[0] = 0;   // k_span's list of waves with wide spans
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t i = blockIdx.x * (int64_t)SCAN_BLOCK + 4 * (int64_t)threadIdx.x;   // items i .. i + 3
     uint32_t v[4];
@@ -1028,9 +1029,27 @@ __device__ __forceinline__ int ps_row_tri(const uint32_t* __restrict__ row_off, 
 // ---------------------------------------------------------------------------
 // span setup
 // ---------------------------------------------------------------------------
+// Spans at least this long keep varying checkpoints at each later piece, so
+// that shading never replays more than about this many pixels; shorter spans
+// are replayed from x1.
+#define PS_CK_MIN 48
+__device__ __forceinline__ bool ps_span_has_ck(const PsSpan& sp) { return sp.x2 - sp.x1 + 1 >= PS_CK_MIN; }
+
 #define SPAN_BINS 512
-// Also counts, per tile, the span pieces in it and the waves (of 64 span
-// items) that have pieces there: tcnt[t] += pieces | waves << 32.  Eight
+// A wave of span items whose longest span has at least this many pixels gives
+// each of its spans runs of its own, which k_segments then places span by span
+// with a lane per accumulator instead of a span per lane.
+// This is also where spans start to keep varying checkpoints, so only those
+// waves carry varyings (24 to 96 measure alike; below 40 a small sphere's
+// frame, whose spans are mostly that long, loses 3 us).
+#define PS_WIDE_MIN PS_CK_MIN
+// called by every lane of the wave; n: the lane's span's pixels, if it has one
+__device__ __forceinline__ bool ps_wave_own_runs(bool has, uint32_t n) { return __any(has && n >= PS_WIDE_MIN); }
+
+// Also counts, per tile, the span pieces in it and their runs: tcnt[t] +=
+// pieces | runs << 32.  A run holds a wave's (of 64 span items) pieces there,
+// or, in the waves that hold a wide span, one span's; those waves go on the
+// list `wide` ([0] = how many).  Eight
 // waves per SIMD (64 VGPRs, no spill): at seven the 256-view batch's span
 // pass took 1.55 ms instead of 1.21.
 __global__ void __launch_bounds__(256, 8) k_span(const PsTri* __restrict__ tris,
@@ -1038,9 +1057,9 @@ __global__ void __launch_bounds__(256, 8) k_span(const PsTri* __restrict__ tris,
                                               int64_t T, int64_t cap,
                                               PsSpan* __restrict__ spans, unsigned long long* __restrict__ tcnt,
                                               const PsView* __restrict__ views, int n_views, int chunk_w, int tile_rows,
-                                              int tile_cols, uint32_t* heavy, PsCounters* cnt)
+                                              int tile_cols, uint32_t* heavy, uint32_t* wide, PsCounters* cnt)
 {
-    // per wave: piece counts of the tiles [kmin, kmin + SPAN_BINS) its spans touch
+    // per wave: pieces | runs << 16 of the tiles [kmin, kmin + SPAN_BINS) its spans touch
     __shared__ uint32_t bins_all[4][SPAN_BINS];
     uint32_t* bins = bins_all[threadIdx.x >> 6];
     const int lane = threadIdx.x & (PS_WAVE - 1);
@@ -1108,6 +1127,8 @@ __global__ void __launch_bounds__(256, 8) k_span(const PsTri* __restrict__ tris,
         const uint32_t npieces = has ? (uint32_t)(st.cx1 - st.cx0 + 1) : 0u;
         const uint32_t kmin = ps_wave_min(has ? st.g0 : 0xffffffffu);
         const uint32_t kmax = ps_wave_max(has ? st.g1 : 0u);
+        const bool own = ps_wave_own_runs(has, nfrag);
+        if (own && lane == 0) wide[1 + atomicAdd(wide, 1u)] = (uint32_t)(i0 >> 6);
         if (kmin != 0xffffffffu && kmax - kmin < (uint32_t)SPAN_BINS) {
             const uint32_t nbin = kmax - kmin + 1;
             for (uint32_t b = lane; b < nbin; b += PS_WAVE) bins[b] = 0;
@@ -1118,19 +1139,26 @@ __global__ void __launch_bounds__(256, 8) k_span(const PsTri* __restrict__ tris,
                 for (uint32_t k = st.g0; k <= st.g1; k++) {
                     int lo, hi;
                     ps_span_tile_chunks(st, tile_cols, k, lo, hi);
-                    atomicAdd(&bins[k - kmin], (uint32_t)(hi - lo + 1));
+                    atomicAdd(&bins[k - kmin], (uint32_t)(hi - lo + 1) + (own ? 1u << 16 : 0u));
                 }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             for (uint32_t b = lane; b < nbin; b += PS_WAVE) {
                 const uint32_t c = bins[b];
-                if (c) atomicAdd(&tcnt[kmin + b], (unsigned long long)c | (1ull << 32));
+                if (c) atomicAdd(&tcnt[kmin + b], (unsigned long long)(c & 0xffffu) | (unsigned long long)(own ? c >> 16 : 1u) << 32);
             }
             // the next iteration clears the bins only after every lane read them
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        } else if (own) {
+            if (has)
+                for (uint32_t k = st.g0; k <= st.g1; k++) {
+                    int lo, hi;
+                    ps_span_tile_chunks(st, tile_cols, k, lo, hi);
+                    atomicAdd(&tcnt[k], (unsigned long long)(hi - lo + 1) | (1ull << 32));
+                }
         } else {
             uint32_t cur = has ? st.g0 : 0xffffffffu;
             for (;;) {
@@ -1149,41 +1177,190 @@ __global__ void __launch_bounds__(256, 8) k_span(const PsTri* __restrict__ tris,
     ps_wave_add(cnt, PS_ST_FRAGS, all_frags, true);
 }
 
-// Spans at least this long keep varying checkpoints at each later piece, so
-// that shading never replays more than about this many pixels; shorter spans
-// are replayed from x1.
-#define PS_CK_MIN 48
-__device__ __forceinline__ bool ps_span_has_ck(const PsSpan& sp) { return sp.x2 - sp.x1 + 1 >= PS_CK_MIN; }
-
 // ---------------------------------------------------------------------------
 // segments: (bin key, span) pairs
 // ---------------------------------------------------------------------------
 // One thread per span: the span's pieces per bin chunk, in order.  The walk
 // from x1 applies the serial `+= step` of the pixel loop (interp.cpp:82-92)
 // pixel by pixel, so each piece starts with exactly the accumulators the
-// reference holds at its first pixel; spans of colour-writing draws that
-// cross chunks also keep the varying accumulators at each later piece.
-// Placement: the wave visits its tiles in increasing order, SG_BATCH at a
-// time.  Per tile, each lane's pieces go after those of the lanes before it
+// reference holds at its first pixel; wide spans of colour-writing draws also
+// keep the varying accumulators at each later piece.
+// Placement, in the waves without a wide span: the wave visits its tiles in
+// increasing order, SG_BATCH at a time.  Per tile, each lane's pieces go after those of the lanes before it
 // (offsets kept in LDS), and lane j reserves the j-th tile's run of
 // consecutive pieces with one atomic on the tile's counter (counting down
 // from k_span's count), all lanes at once.  Then every lane walks its pieces
 // of the batch's tiles into their slots; a span's tiles are consecutive in
 // the visit order, so each walk goes on from tile to tile.
 #define SG_BATCH 16
-// NVC: room for the flush's widest varying checkpoint (at least its nvs
-// floats); the accumulators live in registers across the walk, so the
-// narrowest instantiation that fits keeps more waves resident (a 1080p
-// Blinn-Phong flush: 117 VGPRs and four waves per SIMD at NVC 14 against
-// 149 and three at 20, pieces 29.2 -> 24.8 us).  Up to NVC 14 the kernel
-// fits 96 VGPRs without spilling, five waves per SIMD (23.6 -> 22.4 us);
-// NVC 20 keeps its registers (a bound of four waves spilled).
-template <int NVC>
-__global__ void __launch_bounds__(256, NVC <= 14 ? 5 : 1) k_segments(const PsSpan* __restrict__ spans, const uint32_t* __restrict__ row_off,
+// Reserves the run of n pieces of tile k (counting its counter down from
+// k_span's count) and writes its record; returns its first piece.  The counts
+// k_span left must cover the run (they always do: both kernels visit the same
+// tiles); 0xffffffff, and the flag set, if they do not: never write outside.
+__device__ __forceinline__ uint32_t ps_reserve_run(const PsFrame& f, unsigned long long* tcnt, uint32_t k, uint32_t n,
+                                                   uint32_t mark, uint32_t key, int64_t cap, PsCounters* cnt)
+{
+    const unsigned long long take = (unsigned long long)n | (1ull << 32);
+    const unsigned long long left = atomicAdd(&tcnt[k], (unsigned long long)0 - take);
+    const unsigned long long end = PS_TS(f.tstart[k + 1]);
+    const uint32_t fp = (uint32_t)end - (uint32_t)left;
+    const uint32_t slot = (uint32_t)(end >> 32) - (uint32_t)(left >> 32);
+    if ((uint32_t)left < n || (uint32_t)(left >> 32) == 0u || (uint64_t)fp + n > (uint64_t)cap) {
+        atomicOr(&cnt->overflow, 2);
+        return 0xffffffffu;
+    }
+    f.runs[2 * (size_t)slot] = fp | mark;
+    f.runs[2 * (size_t)slot + 1] = key | (n - 1u);
+    return fp;
+}
+
+// Spans of the listed waves (those that hold a wide span): G (16 or 32) lanes
+// a span, each carrying one accumulator, so that a span of n pixels takes n
+// dependent adds whatever its varyings, and the spans of a listed wave spread
+// over as many waves of the grid.  With a span per lane, a lane stepped up to
+// 22 accumulators a pixel while the lanes whose spans lie in other tile rows
+// waited: 24 objects and a full-view quad at 1366x768 took 2,830 us, now 38
+// (1920x1080 terrain with spans of over 1,000 pixels, 8-pixel tiles: 93 -> 33);
+// what is left is the chain of a span's loads, reservations and adds.
+// Lane j of the group holds word j of the span's piece records (PsSeg: 2 is
+// cf2, 3 the depth numerator) and, from 8 on, varying j - 8, so a piece is one
+// store.  The group first places the span's pieces, one run per tile: its
+// lanes reserve as many tiles at once.
+template <int G>
+__device__ __forceinline__ void ps_wide_spans(const PsSpan* __restrict__ spans, int64_t R, const PsFrame& f,
+                                              const PsTri* __restrict__ tris, const PsDraw* __restrict__ draws,
+                                              const float* __restrict__ vary, int nvs, const uint32_t* __restrict__ wide,
+                                              unsigned long long* __restrict__ tcnt, PsSeg* __restrict__ segs,
+                                              float* __restrict__ ck, int64_t cap, PsCounters* cnt)
+{
+    constexpr int SPW = 64 / G;
+    const int lane = threadIdx.x & (PS_WAVE - 1), j = lane & (G - 1), grp = lane & ~(G - 1);
+    const int CW = f.chunk_w, TC = f.tile_cols;
+    const uint32_t units = wide[0] * G, stride = gridDim.x * (blockDim.x / PS_WAVE);
+    for (uint32_t u = blockIdx.x * (blockDim.x / PS_WAVE) + threadIdx.x / PS_WAVE; u < units; u += stride) {
+        const uint32_t wave_id = wide[1 + u / G], in_wave = (u % G) * SPW + (uint32_t)grp / G;
+        const int64_t i = (int64_t)wave_id * PS_WAVE + in_wave;
+        PsSpan sp;
+        sp.tri = -1;
+        if (i < R) sp = spans[i];
+        const bool has = sp.tri >= 0;
+        if (!__any(has)) continue;
+        PsSpanTiles st = {};
+        int nv = 0, nt = 0;
+        bool need_ck = false;
+        uint32_t word = 0;          // what the lane stores of each piece, where it does not change
+        float v = 0.0f, step = 0.0f;
+        if (has) {
+            const int y = sp.y & 0xffffff;
+            const PsTri tr = tris[sp.tri];
+            const PsView& V = f.views[tr.view];
+            st = ps_span_tiles(V.tile_base, V.n_tiles_x, f.tile_rows, TC, CW, y, sp.x1, sp.x2);
+            nt = (int)(st.g1 - st.g0) + 1;
+            need_ck = st.cx1 > st.cx0 && ((sp.y >> 28) & 1) && ps_span_has_ck(sp);
+            const uint32_t flags = ((uint32_t)(sp.y >> 24) & 3u) << 26 | ((uint32_t)(sp.y >> 28) & 1u) << 28;
+            if (j == 0) word = (uint32_t)i | flags;
+            if (j == 2) { v = sp.cf2; step = sp.cf2_step; }
+            if (j == 3) { v = sp.pz; step = sp.pz_step; }
+            if (j == 4) word = __float_as_uint(sp.cf2_step);
+            if (j == 5) word = __float_as_uint(sp.pz_step);
+            if (j == 6) word = (uint32_t)y;
+            if (need_ck) {
+                const PsDraw& d = draws[tr.code >> 8];
+                nv = d.nv;
+                PsEdge L, Rr;
+                ps_row_edges(tr, y, L, Rr);
+                int left = ps_cvt_i32(ps_edge_eval(L, (float)y) + 0.5f);
+                int right = ps_cvt_i32(ps_edge_eval(Rr, (float)y) + 0.5f);
+                PsSpanGeom g;
+                ps_span_geom(tr, y, left, right, L, Rr, g);
+                if (j >= 8 && j - 8 < nv) {
+                    const float* u0 = vary + (int64_t)ps_vary_index(d, sp.tri) * 3 * nvs + (j - 8);
+                    ps_span_varyings_n<1>(g, u0, u0 + nvs, u0 + 2 * nvs, &v, &step, 1);
+                }
+            }
+        }
+        const bool acc = j == 2 || j == 3 || j >= 8;
+        // the lane's words of consecutive pieces lie `next` words apart; a
+        // whole chunk further, the pixel range and the checkpointed piece's
+        // own index move by `move`
+        const int64_t next = j < 8 ? (int64_t)(sizeof(PsSeg) / 4) : f.ck_stride;
+        const uint32_t move = j == 1 ? (uint32_t)CW * 0x10001u : (j == 7 && need_ck) ? 1u : 0u;
+        const int maxnt = (int)ps_wave_max((uint32_t)nt);
+        for (int q0 = 0; q0 < maxnt; q0 += G) {
+            uint32_t first = 0xffffffffu;
+            if (q0 + j < nt) {
+                const uint32_t k = st.g0 + (uint32_t)(q0 + j);
+                int lo, hi;
+                ps_span_tile_chunks(st, TC, k, lo, hi);
+                first = ps_reserve_run(f, tcnt, k, (uint32_t)(hi - lo + 1), PS_RUN_OWN, wave_id << 12 | in_wave << 6, cap, cnt);
+            }
+            for (int q = q0; q < min(q0 + G, maxnt); q++) {
+                const uint32_t s = (uint32_t)__shfl((int)first, grp + (q - q0), PS_WAVE);
+                if (q >= nt) continue;
+                int lo, hi;
+                ps_span_tile_chunks(st, TC, st.g0 + (uint32_t)q, lo, hi);
+                const bool lost = s == 0xffffffffu;   // not placed: step over the tile
+                uint32_t* at = j < 8 ? (uint32_t*)(segs + (lost ? 0u : s)) + j
+                                     : (uint32_t*)ck + (int64_t)(lost ? 0u : s) * f.ck_stride + (j - 8);
+                const bool begins = lo == st.cx0;
+                bool on = !lost && (j < 8 || (j - 8 < nv && !begins));   // the span's first piece keeps no checkpoint
+                if (j == 1) word = (uint32_t)max(sp.x1, lo * CW) | (uint32_t)min(sp.x2, lo * CW + CW - 1) << 16;
+                if (j == 7) word = need_ck && !begins ? (s | PS_SEG_CK) : (uint32_t)sp.tri;
+                int n = hi - lo + 1;
+                if (begins) {   // on to the next chunk's first pixel
+                    if (on) *at = acc ? __float_as_uint(v) : word;
+                    const int x = (st.cx0 + 1) * CW;
+                    for (int k = sp.x1; k < x; k++) v += step;
+                    at += next;
+                    on = !lost && (j < 8 || j - 8 < nv);
+                    if (j == 1) word = (uint32_t)x | (uint32_t)(x + CW - 1) << 16;
+                    if (j == 7 && need_ck) word = (s + 1u) | PS_SEG_CK;
+                    n--;
+                }
+                const bool ends = n > 0 && hi == st.cx1;
+                if (ends) n--;
+                if (lost) {
+                    for (int k = n * CW; k > 0; k--) v += step;
+                } else if (on) {   // the other lanes carry nothing
+                    auto whole = [&](int adds) {
+                        *at = acc ? __float_as_uint(v) : word;
+                        at += next;
+                        word += move;
+#pragma unroll
+                        for (int k = 0; k < adds; k++) v += step;
+                    };
+                    auto tile = [&](int adds) {
+                        for (; n >= 4; n -= 4) { whole(adds); whole(adds); whole(adds); whole(adds); }
+                        for (; n > 0; n--) whole(adds);
+                    };
+                    if (CW == 2) tile(2);
+                    else if (CW == 4) tile(4);
+                    else if (CW == 8) tile(8);
+                    else
+                        for (; n > 0; n--) {
+                            whole(1);
+                            for (int k = 1; k < CW; k++) v += step;
+                        }
+                }
+                if (ends) {
+                    if (j == 1) word = (word & 0xffffu) | (uint32_t)sp.x2 << 16;
+                    if (on) *at = acc ? __float_as_uint(v) : word;
+                }
+            }
+        }
+    }
+}
+
+// G: lanes of a wide span, 8 and one per varying float.  Spans per lane carry
+// two accumulators: with the varyings beside them the kernel took 96 VGPRs
+// (five waves per SIMD) for 14 floats and 149 for 20.
+template <int G>
+__global__ void __launch_bounds__(256) k_segments(const PsSpan* __restrict__ spans, const uint32_t* __restrict__ row_off,
                                                   int64_t T, PsFrame f, const PsTri* __restrict__ tris,
                                                   const PsDraw* __restrict__ draws, const float* __restrict__ vary, int nvs,
                                                   unsigned long long* __restrict__ tcnt, PsSeg* __restrict__ segs,
-                                                  float* __restrict__ ck, int64_t cap, PsCounters* cnt)
+                                                  float* __restrict__ ck, int64_t cap, const uint32_t* __restrict__ wide,
+                                                  PsCounters* cnt)
 {
     __shared__ uint32_t rel_all[4][SG_BATCH][PS_WAVE];   // per wave: [iteration][lane] offset in the run
     const bool poisoned = ps_poisoned(cnt);
@@ -1194,6 +1371,7 @@ __global__ void __launch_bounds__(256, NVC <= 14 ? 5 : 1) k_segments(const PsSpa
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&cnt->overflow, 1);
         return;
     }
+    ps_wide_spans<G>(spans, R, f, tris, draws, vary, nvs, wide, tcnt, segs, ck, cap, cnt);
     const int CW = f.chunk_w, TC = f.tile_cols;
     int64_t tb1 = 0;   // the only view of a one-view flush, read once
     int ntx1 = 0;
@@ -1207,40 +1385,22 @@ __global__ void __launch_bounds__(256, NVC <= 14 ? 5 : 1) k_segments(const PsSpa
         sp.tri = -1;
         if (i < R) sp = spans[i];
         const bool has = sp.tri >= 0;
+        if (ps_wave_own_runs(has, (uint32_t)(sp.x2 - sp.x1 + 1))) continue;   // placed above
         PsSpanTiles st = {};
-        int nv = 0, y = 0;
+        int y = 0;
         uint32_t flags = 0;
-        bool need_ck = false;
-        float vs[NVC], vt[NVC];
         if (has) {
-            // the triangle only for a flush of several views (its view) or
-            // for varying checkpoints
-            PsTri tr;
+            // the triangle only for a flush of several views (its view)
             int64_t vtb = tb1;
             int vntx = ntx1;
             if (f.n_views != 1) {
-                tr = tris[sp.tri];
-                const PsView& v = f.views[tr.view];
+                const PsView& v = f.views[tris[sp.tri].view];
                 vtb = v.tile_base;
                 vntx = v.n_tiles_x;
             }
             y = sp.y & 0xffffff;
             flags = ((uint32_t)(sp.y >> 24) & 3u) << 26 | ((uint32_t)(sp.y >> 28) & 1u) << 28;
             st = ps_span_tiles(vtb, vntx, f.tile_rows, TC, CW, y, sp.x1, sp.x2);
-            need_ck = (st.cx1 > st.cx0) && ((sp.y >> 28) & 1) && ps_span_has_ck(sp);
-            if (need_ck) {
-                if (f.n_views == 1) tr = tris[sp.tri];
-                const PsDraw& d = draws[tr.code >> 8];
-                nv = d.nv;
-                PsEdge L, Rr;
-                ps_row_edges(tr, y, L, Rr);
-                int left = ps_cvt_i32(ps_edge_eval(L, (float)y) + 0.5f);
-                int right = ps_cvt_i32(ps_edge_eval(Rr, (float)y) + 0.5f);
-                PsSpanGeom g;
-                ps_span_geom(tr, y, left, right, L, Rr, g);
-                const float* u0 = vary + (int64_t)ps_vary_index(d, sp.tri) * 3 * nvs;
-                ps_span_varyings_n<NVC>(g, u0, u0 + nvs, u0 + 2 * nvs, vs, vt, nv);
-            }
         }
         float cf2 = sp.cf2, pz = sp.pz;
         int x = sp.x1;
@@ -1271,22 +1431,7 @@ __global__ void __launch_bounds__(256, NVC <= 14 ? 5 : 1) k_segments(const PsSpa
             }
             if (nb == 0) break;
             uint32_t first = 0xffffffffu;
-            if (lane < nb) {
-                const unsigned long long take = (unsigned long long)bn | (1ull << 32);
-                const unsigned long long left = atomicAdd(&tcnt[bk], (unsigned long long)0 - take);
-                const unsigned long long end = PS_TS(f.tstart[bk + 1]);
-                const uint32_t fp = (uint32_t)end - (uint32_t)left;
-                const uint32_t slot = (uint32_t)(end >> 32) - (uint32_t)(left >> 32);
-                // the counts k_span left must cover this run (they always do:
-                // both kernels visit the same tiles); never write outside
-                if ((uint32_t)left < bn || (uint32_t)(left >> 32) == 0u || (uint64_t)fp + bn > (uint64_t)cap) {
-                    atomicOr(&cnt->overflow, 2);
-                } else {
-                    first = fp;
-                    f.runs[2 * (size_t)slot] = fp;
-                    f.runs[2 * (size_t)slot + 1] = (wave_id << 12) | (bn - 1u);
-                }
-            }
+            if (lane < nb) first = ps_reserve_run(f, tcnt, bk, bn, 0u, wave_id << 12, cap, cnt);
             // every lane walks its pieces of the batch's tiles
             const int maxtb = __builtin_amdgcn_readfirstlane(ps_wave_max((uint32_t)ntb));
             for (int q = 0; q < maxtb; q++) {
@@ -1300,11 +1445,6 @@ __global__ void __launch_bounds__(256, NVC <= 14 ? 5 : 1) k_segments(const PsSpa
                         for (; x < xa; x++) {
                             cf2 += sp.cf2_step;
                             pz += sp.pz_step;
-                            if (need_ck) {
-#pragma unroll
-                                for (int k = 0; k < NVC; k++)
-                                    if (k < nv) vs[k] = vs[k] + vt[k];
-                            }
                         }
                         PsSeg sg;
                         sg.si = (uint32_t)i | flags;
@@ -1314,14 +1454,8 @@ __global__ void __launch_bounds__(256, NVC <= 14 ? 5 : 1) k_segments(const PsSpa
                         sg.cst = sp.cf2_step;
                         sg.pst = sp.pz_step;
                         sg.y = y;
-                        sg.win = need_ck && xa > sp.x1 ? (s | PS_SEG_CK) : (uint32_t)sp.tri;
+                        sg.win = (uint32_t)sp.tri;
                         segs[s] = sg;
-                        if (need_ck && xa > sp.x1) {
-                            float* c = ck + (int64_t)s * f.ck_stride;
-#pragma unroll
-                            for (int k = 0; k < NVC; k++)
-                                if (k < nv) c[k] = vs[k];
-                        }
                     }
                 }
             }
@@ -1333,6 +1467,12 @@ __global__ void __launch_bounds__(256, NVC <= 14 ? 5 : 1) k_segments(const PsSpa
 // ---------------------------------------------------------------------------
 // tile lists: the runs of a tile in submission order
 // ---------------------------------------------------------------------------
+// pieces of a run (PsFrame.runs: first piece and mark, key)
+__device__ __forceinline__ uint32_t ps_run_count(uint32_t first, uint32_t key)
+{
+    return (key & ((first & PS_RUN_OWN) ? 0x3fu : 0xfffu)) + 1u;
+}
+
 // For each lane's keys key[0 .. Q): how many of the n keys they are compared
 // with lie below.  Those are held one per lane in `other` (lanes from n on are
 // not looked at); each is read from its lane by a constant index, so a key
@@ -1386,7 +1526,8 @@ __device__ __forceinline__ void ps_run_window(const uint32_t* rl, uint32_t nr, u
         uint32_t key = j < nr ? rl[2 * j + 1] : 0xffffffffu;
         rbase = j < nr ? rl[2 * j] : 0u;
         ps_sort_lanes(key, rbase, nw);
-        const uint32_t c = j < nr ? (key & 0xfffu) + 1u : 0u;
+        const uint32_t c = j < nr ? ps_run_count(rbase, key) : 0u;
+        rbase &= ~PS_RUN_OWN;
         const uint32_t incl = ps_wave_incl_scan(c);
         rv = j < nr ? incl - c : 0xffffffffu;
         vhi = n_list;
@@ -1408,8 +1549,9 @@ __device__ __forceinline__ uint32_t ps_run_piece(uint32_t rv, uint32_t rbase, ui
     return __shfl(rbase, pos, 64) + (v - __shfl(rv, pos, 64));
 }
 
-// A tile with more than 64 runs: one wave sorts them stably by wave (LSD
-// radix, 7-bit digits of the wave index above the smallest, ping-ponging
+// A tile with more than PS_LDS_RUNS runs (more than 64 in the walk that
+// blends): one wave sorts them by their keys from bit 6 up, which tell any two
+// runs of a tile apart (LSD radix, 7-bit digits above the smallest, ping-ponging
 // between the tile's parts a and b of the two run arrays), then replaces each
 // run's key by the list position of its first piece.  cnt128: 128 words of
 // the wave's LDS.  Returns the array that holds the result.
@@ -1419,7 +1561,7 @@ __device__ uint32_t* ps_order_runs(uint32_t* a, uint32_t* b, uint32_t nr, uint32
     const uint64_t lt = ps_lt_mask();
     uint32_t mn = 0xffffffffu, mx = 0;
     for (uint32_t j = lane; j < nr; j += 64) {
-        const uint32_t w = a[2 * j + 1] >> 12;
+        const uint32_t w = a[2 * j + 1] >> 6;
         mn = min(mn, w);
         mx = max(mx, w);
     }
@@ -1431,7 +1573,7 @@ __device__ uint32_t* ps_order_runs(uint32_t* a, uint32_t* b, uint32_t nr, uint32
         cnt128[lane + 64] = 0;
         __builtin_amdgcn_wave_barrier();
         for (uint32_t j = lane; j < nr; j += 64)
-            atomicAdd(&cnt128[(((a[2 * j + 1] >> 12) - mn) >> shift) & 127u], 1u);
+            atomicAdd(&cnt128[(((a[2 * j + 1] >> 6) - mn) >> shift) & 127u], 1u);
         __builtin_amdgcn_wave_barrier();
         {
             const uint32_t c0 = cnt128[2 * lane], c1 = cnt128[2 * lane + 1];
@@ -1445,7 +1587,7 @@ __device__ uint32_t* ps_order_runs(uint32_t* a, uint32_t* b, uint32_t nr, uint32
             const uint32_t j = j0 + lane;
             const bool valid = j < nr;
             const uint32_t e0 = valid ? a[2 * j] : 0u, e1 = valid ? a[2 * j + 1] : 0u;
-            const uint32_t dig = valid ? (((e1 >> 12) - mn) >> shift) & 127u : 0u;
+            const uint32_t dig = valid ? (((e1 >> 6) - mn) >> shift) & 127u : 0u;
             uint64_t same = __ballot(valid);
 #pragma unroll
             for (int bit = 0; bit < 7; bit++) {
@@ -1468,9 +1610,13 @@ __device__ uint32_t* ps_order_runs(uint32_t* a, uint32_t* b, uint32_t nr, uint32
     uint32_t carry = 0;
     for (uint32_t j0 = 0; j0 < nr; j0 += 64) {
         const uint32_t j = j0 + lane;
-        const uint32_t c = j < nr ? (a[2 * j + 1] & 0xfffu) + 1u : 0u;
+        const uint32_t first = j < nr ? a[2 * j] : 0u;
+        const uint32_t c = j < nr ? ps_run_count(first, a[2 * j + 1]) : 0u;
         const uint32_t incl = ps_wave_incl_scan(c);
-        if (j < nr) a[2 * j + 1] = carry + incl - c;
+        if (j < nr) {
+            a[2 * j] = first & ~PS_RUN_OWN;
+            a[2 * j + 1] = carry + incl - c;
+        }
         carry += __builtin_amdgcn_readlane(incl, 63);
     }
     __threadfence();
@@ -1527,7 +1673,7 @@ __device__ __forceinline__ void ps_sort_runs_lds(const uint32_t* rl, uint32_t nr
         if (nr > 64u * q) ps_count_below<Q>(key, key[q], min(nr - 64u * q, 64u), rank);
 #pragma unroll
     for (int q = 0; q < Q; q++)
-        if (q * 64 + lane < nr) out[rank[q]] = make_uint2(val[q], (key[q] & 0xfffu) + 1u);
+        if (q * 64 + lane < nr) out[rank[q]] = make_uint2(val[q] & ~PS_RUN_OWN, ps_run_count(val[q], key[q]));
     ps_lds_turn();
     uint32_t carry = 0;
     for (uint32_t j0 = 0; j0 < nr; j0 += 64) {
@@ -2304,10 +2450,10 @@ int psk_scan_blocks(int64_t cap) { return gsz(cap, SCAN_BLOCK); }
 
 
 void psk_scan_parts(hipStream_t s, const uint32_t* in, int64_t n, uint32_t* out, const uint32_t* parts, int pgran,
-                    uint32_t* total_out, uint32_t* bstart, int64_t bcap)
+                    uint32_t* total_out, uint32_t* bstart, int64_t bcap, uint32_t* wide)
 {
     hipLaunchKernelGGL(k_scan_parts, dim3(psk_scan_blocks(n)), dim3(1024), 0, s, in, n, parts, pgran, out, total_out,
-                       bstart, bcap);
+                       bstart, bcap, wide);
 }
 
 int psk_heavy_cap() { return PS_HEAVY_MAX; }
@@ -2329,34 +2475,33 @@ void psk_scan_tiles(hipStream_t s, const unsigned long long* tcnt, int64_t n, un
 
 void psk_span(hipStream_t s, const PsTri* tris, const uint32_t* row_off, const uint32_t* bstart, int64_t T,
               PsSpan* spans, unsigned long long* tcnt, const PsView* views, int n_views, int chunk_w, int tile_rows,
-              int64_t cap, uint32_t* heavy, PsCounters* cnt)
+              int64_t cap, uint32_t* heavy, uint32_t* wide, PsCounters* cnt)
 {
     int g = gsz(cap, 256); if (g > 2048) g = 2048;
     const int tile_cols = 64 / tile_rows;
     hipLaunchKernelGGL(k_span, dim3(g), dim3(256), 0, s, tris, row_off, bstart, T, cap, spans, tcnt, views, n_views,
-                       chunk_w, tile_rows, tile_cols, heavy, cnt);
+                       chunk_w, tile_rows, tile_cols, heavy, wide, cnt);
 }
 
 void psk_scan_rows(hipStream_t s, const uint32_t* in, int64_t n, uint32_t* out, uint32_t* partial, uint32_t* total_out,
-                   uint32_t* bstart, int64_t bcap)
+                   uint32_t* bstart, int64_t bcap, uint32_t* wide)
 {
     hipLaunchKernelGGL(k_scan_reduce<uint32_t>, dim3(psk_scan_blocks(n)), dim3(256), 0, s, in, (const uint32_t*)nullptr, n,
                        partial, (const PsCounters*)nullptr);
-    psk_scan_parts(s, in, n, out, partial, SCAN_BLOCK, total_out, bstart, bcap);
+    psk_scan_parts(s, in, n, out, partial, SCAN_BLOCK, total_out, bstart, bcap, wide);
 }
 
 void psk_segments(hipStream_t s, const PsSpan* spans, const uint32_t* row_off, int64_t T, const PsFrame& f,
                   const PsTri* tris, const PsDraw* draws, const float* vary, int nvs, unsigned long long* tcnt, PsSeg* segs,
-                  float* ck, int64_t span_cap, int64_t seg_cap, PsCounters* cnt)
+                  float* ck, int64_t span_cap, int64_t seg_cap, const uint32_t* wide, PsCounters* cnt)
 {
     int g = gsz(span_cap, 256); if (g > 2048) g = 2048;
-#define SG_LAUNCH(NVC)                                                                                                \
-    hipLaunchKernelGGL(k_segments<NVC>, dim3(g), dim3(256), 0, s, spans, row_off, T, f, tris, draws, vary, nvs, tcnt, \
-                       segs, ck, seg_cap, cnt)
-    if (nvs <= 4) SG_LAUNCH(4);
-    else if (nvs <= 8) SG_LAUNCH(8);
-    else if (nvs <= 14) SG_LAUNCH(14);
-    else SG_LAUNCH(PS_MAX_NV);
+#define SG_LAUNCH(G)                                                                                                  \
+    hipLaunchKernelGGL(k_segments<G>, dim3(g), dim3(256), 0, s, spans, row_off, T, f, tris, draws, vary, nvs, tcnt,   \
+                       segs, ck, seg_cap, wide, cnt)
+    static_assert(PS_MAX_NV <= 24, "a lane per varying float beside the 8 of the record");
+    if (nvs <= 8) SG_LAUNCH(16);
+    else SG_LAUNCH(32);
 #undef SG_LAUNCH
 }
 

@@ -126,6 +126,8 @@ struct PsView {
     int cclear_rows; uint32_t cclear_value;
 };
 
+#define PS_RUN_OWN 0x80000000u
+
 // Flush-wide parameters passed by value to kernels.
 struct PsFrame {
     int chunk_w, tile_rows, tile_cols;   // raster tiling
@@ -134,9 +136,13 @@ struct PsFrame {
     int64_t n_tiles, n_stiles;
     const PsView* views;
     // tile lists.  Each wave of 64 span items writes its pieces of a tile as
-    // one run of consecutive pieces.  tstart[t] holds the first piece (low 32
-    // bits) and the first run (bits 32-62) of tile t (n_tiles + 1 entries);
-    // run r is runs[2r] = its first piece, runs[2r+1] = wave << 12 | pieces - 1.
+    // one run of consecutive pieces, in span order; a wave that holds a wide
+    // span writes one run per span instead.  tstart[t] holds the first piece
+    // (low 32 bits) and the first run (bits 32-62) of tile t (n_tiles + 1
+    // entries); run r is runs[2r] = its first piece, with PS_RUN_OWN set in a
+    // run of one span, and runs[2r+1] = its key: wave << 12 | pieces - 1, or
+    // wave << 12 | span in the wave << 6 | pieces - 1.  Ordered by key, the
+    // runs of a tile are in submission order.
     // runs2 is scratch of the same size for ordering long run lists.
     const unsigned long long* tstart;
     uint32_t* runs;

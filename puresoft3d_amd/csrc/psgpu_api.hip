@@ -143,6 +143,7 @@ struct FlushBufs {
     DevBuf<float> grad;   // per triangle: screen gradients for the mip level (8 floats)
     DevBuf<uint32_t> nrows, rowoff, partial;
     DevBuf<uint32_t> bstart;   // triangle of every 64th row item, written by the row scan
+    DevBuf<uint32_t> wide;     // count and list of the span waves that hold a wide span
     DevBuf<PsSpan> spans;
     // tile lists: per-tile piece and run counts (zero between flushes: the
     // piece kernel counts them back down), their scan, the scan's block sums,
@@ -559,7 +560,7 @@ int size_flush_scratch(psgpu_ctx* c, int64_t T, int nvs, int64_t n_tiles)
         return fail(c, PSGPU_ERR_NOMEM, "more than %lld spans or %lld pieces in one flush", (long long)c->max_spans,
                     (long long)c->max_segs);
     if ((rc = ensure(c, b.partial, row_partials(T))) ||
-        (rc = ensure(c, b.bstart, b.span_cap / 64 + 2)) || (rc = ensure(c, b.spans, b.span_cap)) ||
+        (rc = ensure(c, b.bstart, b.span_cap / 64 + 2)) || (rc = ensure(c, b.wide, b.span_cap / 64 + 3)) || (rc = ensure(c, b.spans, b.span_cap)) ||
         (rc = ensure(c, b.segs, b.seg_cap)) || (rc = ensure(c, b.ck, (size_t)b.seg_cap * nvs)) ||
         (rc = ensure(c, b.runs, (size_t)b.seg_cap * 2)) || (rc = ensure(c, b.runs2, (size_t)b.seg_cap * 2)) ||
         (rc = ensure(c, b.tstart, n_tiles + 1)) || (rc = ensure(c, b.tpartial, psk_scan_blocks(n_tiles) + 1)) ||
@@ -628,10 +629,10 @@ int run_flush(psgpu_ctx* c, const Cmd& cmd, uint8_t* staged)
         const int sb = psk_setup_block();
         if (row_part)
             psk_scan_parts(s, c->fb.nrows.p, T, c->fb.rowoff.p, row_part, sb, c->d_sizes + 0, c->fb.bstart.p,
-                           c->fb.span_cap / 64 + 2);
+                           c->fb.span_cap / 64 + 2, c->fb.wide.p);
         else
             psk_scan_rows(s, c->fb.nrows.p, T, c->fb.rowoff.p, c->fb.partial.p, c->d_sizes + 0, c->fb.bstart.p,
-                          c->fb.span_cap / 64 + 2);
+                          c->fb.span_cap / 64 + 2, c->fb.wide.p);
     }
     // k_span finds each row's triangle by a search in the row offsets,
     // started from the row scan's table of every 64th item's triangle and
@@ -647,7 +648,7 @@ int run_flush(psgpu_ctx* c, const Cmd& cmd, uint8_t* staged)
     {
         ProfScope p(c, "span");
         psk_span(s, c->fb.tris.p, c->fb.rowoff.p, c->fb.bstart.p, T, c->fb.spans.p, c->fb.tcnt.p, dv,
-                 f.n_views, f.chunk_w, f.tile_rows, c->fb.span_cap, heavy, c->d_cnt);
+                 f.n_views, f.chunk_w, f.tile_rows, c->fb.span_cap, heavy, c->fb.wide.p, c->d_cnt);
     }
     {
         ProfScope p(c, "scan_tiles");
@@ -660,7 +661,7 @@ int run_flush(psgpu_ctx* c, const Cmd& cmd, uint8_t* staged)
     {
         ProfScope p(c, "segments");
         psk_segments(s, c->fb.spans.p, c->fb.rowoff.p, T, f, c->fb.tris.p, dd, c->fb.vary.p, nvs, c->fb.tcnt.p,
-                     c->fb.segs.p, c->fb.ck.p, c->fb.span_cap, c->fb.seg_cap, c->d_cnt);
+                     c->fb.segs.p, c->fb.ck.p, c->fb.span_cap, c->fb.seg_cap, c->fb.wide.p, c->d_cnt);
     }
     if (imm) {
         ProfScope p(c, "raster");
@@ -1218,9 +1219,9 @@ bool carve_flush(Arena& a, const FlushShape& sh, FlushBufs& b)
         !a.take(b.tstart, sh.n_tiles + 1) || !a.take(b.tpartial, psk_scan_blocks(sh.n_tiles) + 1) ||
         !a.take(b.heavy, psk_heavy_cap() + 1))
         return false;
-    // bytes per span: record and row-start table entry, and 1.5 pieces of
+    // bytes per span: record, entries of the row-start table and the list of wide waves, and 1.5 pieces of
     // record, checkpoint and two run records
-    const double per_span = 32 + 4.0 / 64 + 1.5 * (sizeof(PsSeg) + 4.0 * sh.nvs + 16);
+    const double per_span = 32 + 8.0 / 64 + 1.5 * (sizeof(PsSeg) + 4.0 * sh.nvs + 16);
     size_t left = a.cap - a.used;
     int64_t spans = (int64_t)((double)left / per_span);
     spans = std::min<int64_t>(spans, (int64_t)1 << 26);
@@ -1229,7 +1230,7 @@ bool carve_flush(Arena& a, const FlushShape& sh, FlushBufs& b)
         FlushBufs x = b;
         x.span_cap = spans;
         x.seg_cap = spans * 3 / 2;
-        if (t.take(x.bstart, x.span_cap / 64 + 2) &&
+        if (t.take(x.bstart, x.span_cap / 64 + 2) && t.take(x.wide, x.span_cap / 64 + 3) &&
             t.take(x.spans, x.span_cap) && t.take(x.segs, x.seg_cap) &&
             t.take(x.ck, (size_t)x.seg_cap * sh.nvs) && t.take(x.runs, (size_t)x.seg_cap * 2) &&
             t.take(x.runs2, (size_t)x.seg_cap * 2)) {
@@ -1314,7 +1315,7 @@ int psgpu_destroy(psgpu_ctx* c)
     for (auto& t : c->tex) fr(t.d);
     for (auto& v : c->vbo) fr(v.d);
     fr(c->d_blob.p); fr(c->fb.tris.p); fr(c->fb.vary.p); fr(c->fb.nrows.p); fr(c->fb.rowoff.p); fr(c->fb.partial.p);
-    fr(c->fb.bstart.p); fr(c->fb.spans.p); fr(c->fb.tcnt.p); fr(c->fb.tstart.p); fr(c->fb.tpartial.p);
+    fr(c->fb.bstart.p); fr(c->fb.wide.p); fr(c->fb.spans.p); fr(c->fb.tcnt.p); fr(c->fb.tstart.p); fr(c->fb.tpartial.p);
     fr(c->fb.runs.p); fr(c->fb.runs2.p); fr(c->fb.heavy.p); fr(c->fb.winner.p);
     fr(c->fb.segs.p); fr(c->fb.ck.p); fr(c->fb.grad.p);
     fr(c->dbg_last); fr(c->dbg_rcount); fr(c->dbg_rhash); fr(c->dbg_pcount); fr(c->dbg_phash);

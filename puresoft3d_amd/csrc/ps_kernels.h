@@ -49,5 +49,12 @@ void psk_raster_imm(hipStream_t s, int prog, bool debug, const PsSpan* spans, co
 void psk_shade(hipStream_t s, int prog, const PsSpan* spans, const PsSeg* segs, const float* ck, const PsTri* tris,
                const float* vary, int nvs, const float* grads, const PsDraw* draws, const PsFrame& f,
                const PsCounters* cnt, bool clears);
-void psk_mip(hipStream_t s, const uint8_t* src, int ws, int hs, int ss, uint8_t* dst, int wd, int hd, int elem);
+// up to six levels of the mip chains of `layers` layers, from a source level of
+// w x h texels: off[0] its offset in the layer, off[1 .. levels] those to write;
+// rows are tight
+struct PsMips {
+    int w, h, levels;
+    int64_t off[7];
+};
+void psk_mips(hipStream_t s, uint8_t* data, int64_t layer_bytes, int layers, int elem, const PsMips& m);
 void psk_selftest(hipStream_t s, int op, const float* a, const float* b, float* out, int n);

@@ -1432,14 +1432,14 @@ int psgpu_texture_generate_mips(psgpu_ctx* c, int tex)
     int rc = do_sync(c);
     if (rc) return rc;
     Tex& t = c->tex[tex];
-    for (int L = 0; L < t.layers; L++)
-        for (int l = 1; l < t.levels; l++) {
-            int ws, hs, ss, wd, hd, sd;
-            level_bytes(t, l - 1, &ws, &hs, &ss);
-            level_bytes(t, l, &wd, &hd, &sd);
-            psk_mip(c->stream, t.d + t.layer_bytes * L + t.level_off[l - 1], ws, hs, ss, t.d + t.layer_bytes * L + t.level_off[l],
-                    wd, hd, t.elem);
-        }
+    for (int l = 0; l + 1 < t.levels; l += 6) {
+        PsMips m;
+        int scan;
+        level_bytes(t, l, &m.w, &m.h, &scan);
+        m.levels = std::min(6, t.levels - 1 - l);
+        for (int k = 0; k <= m.levels; k++) m.off[k] = t.level_off[l + k];
+        psk_mips(c->stream, t.d, t.layer_bytes, t.layers, t.elem, m);
+    }
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return PSGPU_OK;

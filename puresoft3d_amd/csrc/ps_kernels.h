@@ -7,6 +7,10 @@ void psk_fill_u32(hipStream_t s, uint32_t* p, int64_t n, uint32_t v, const PsCou
 // work pieces of a fill (1024 values of a row); psk_fills takes the largest
 int64_t psk_fill_pieces(int64_t rows, int64_t width);
 void psk_fills(hipStream_t s, const PsFill* fills, int n, int64_t max_pieces, const PsCounters* c);
+void psk_few_fills(hipStream_t s, const PsFewFills& fills, int n, int64_t max_pieces, const PsCounters* c);
+// the log's overflow flag, sizes and statistics to the host, and all zero again
+// (after an overflow only with reset)
+void psk_finish(hipStream_t s, PsCounters* c, uint32_t* sizes, PsFinish* out, bool reset);
 // row_part (optional, flushes of one programme): each block of psk_setup_block()
 // triangles writes its row total there
 int psk_setup_block();
@@ -24,19 +28,20 @@ void psk_scan_rows(hipStream_t s, const uint32_t* in, int64_t n, uint32_t* out, 
 // exclusive scan of the per-tile counts (pieces | runs << 32) into tstart
 // (n + 1 entries); the piece total into *total_out, its running maximum at
 // total_out[2]
+// flag: the host's word for the command (pinned), set where the kernel finds an overflow
 // heavy (optional, 1 + psk_heavy_cap() words): the heavy-tile list of PsFrame.heavy
 int psk_heavy_cap();
 void psk_scan_tiles(hipStream_t s, const unsigned long long* tcnt, int64_t n, unsigned long long* tstart,
-                    unsigned long long* partial, uint32_t* total_out, const PsCounters* c, uint32_t* heavy);
+                    unsigned long long* partial, uint32_t* total_out, PsCounters* c, uint32_t* heavy, int* flag);
 // spans of every row item; tcnt[t] += the pieces in tile t | their runs << 32; wide: the
 // waves of 64 items that hold a wide span ([0] = how many)
 void psk_span(hipStream_t s, const PsTri* tris, const uint32_t* row_off, const uint32_t* bstart, int64_t T,
               PsSpan* spans, unsigned long long* tcnt, const PsView* views, int n_views, int chunk_w, int tile_rows,
-              int64_t cap, uint32_t* heavy, uint32_t* wide, PsCounters* cnt);
+              int64_t cap, uint32_t* heavy, uint32_t* wide, PsCounters* cnt, int* flag);
 // the pieces, into runs of the tile lists f.tstart / f.runs; counts tcnt back down to zero.
 void psk_segments(hipStream_t s, const PsSpan* spans, const uint32_t* row_off, int64_t T, const PsFrame& f,
                   const PsTri* tris, const PsDraw* draws, const float* vary, int nvs, unsigned long long* tcnt, PsSeg* segs,
-                  float* ck, int64_t span_cap, int64_t seg_cap, const uint32_t* wide, PsCounters* cnt);
+                  float* ck, int64_t span_cap, int64_t seg_cap, const uint32_t* wide, PsCounters* cnt, int* flag);
 size_t psk_raster_lds(int chunk_w, int waves);
 void psk_raster(hipStream_t s, bool debug, const PsSpan* spans, const PsSeg* segs, const PsTri* tris, const PsDraw* draws,
                 const PsFrame& f, int waves_per_group, PsCounters* cnt);

@@ -30,6 +30,15 @@
 
 #define PS_WAVE 64
 
+// An overflow is noted twice: in the counters, where it stops the later kernels
+// of the log, and in the host's word for the logged command (pinned memory),
+// so that no copy has to follow every flush.
+__device__ __forceinline__ void ps_overflow(PsCounters* c, int bits, int* flag)
+{
+    atomicOr(&c->overflow, bits);
+    __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __device__ __forceinline__ bool ps_poisoned(const PsCounters* c)
 {
     return *((volatile const int*)&c->overflow) != 0;
@@ -265,10 +274,8 @@ __global__ void k_fill_u32(uint32_t* p, int64_t n, uint32_t v, const PsCounters*
 // row's alignment), and inside a piece the 16-byte aligned middle is stored
 // four values per thread.
 #define FILL_PIECE 1024
-__global__ void __launch_bounds__(256) k_fills(const PsFill* __restrict__ fills, const PsCounters* c)
+__device__ __forceinline__ void ps_fill(const PsFill& fl)
 {
-    if (c && ps_poisoned(c)) return;
-    const PsFill fl = fills[blockIdx.y];
     const uint4 v4 = make_uint4(fl.value, fl.value, fl.value, fl.value);
     if (fl.scan == fl.width) {
         // rows without padding are one run: four values per thread, grid-stride
@@ -298,6 +305,45 @@ __global__ void __launch_bounds__(256) k_fills(const PsFill* __restrict__ fills,
         if ((int64_t)threadIdx.x < nvec) ((uint4*)(p + head))[threadIdx.x] = v4;
         if (tail0 + threadIdx.x < n) p[tail0 + threadIdx.x] = fl.value;
     }
+}
+
+__global__ void __launch_bounds__(256) k_fills(const PsFill* __restrict__ fills, const PsCounters* c)
+{
+    if (c && ps_poisoned(c)) return;
+    ps_fill(fills[blockIdx.y]);
+}
+
+// a few fills come as kernel arguments, without a copy of their records
+__global__ void __launch_bounds__(256) k_few_fills(PsFewFills fills, const PsCounters* c)
+{
+    if (c && ps_poisoned(c)) return;
+    ps_fill(fills.f[blockIdx.y]);
+}
+
+// The end of the log, one wave: what the host waits for (the overflow flag, the
+// sizes and the sums of the statistics) goes to its pinned memory, and unless
+// the log is to be replayed everything is zero again for the next one.
+__global__ void __launch_bounds__(64) k_finish(PsCounters* c, uint32_t* sizes, PsFinish* out, int reset)
+{
+    const int lane = threadIdx.x;
+    const int overflow = c->overflow;
+    unsigned long long sum[PS_ST_N];
+#pragma unroll
+    for (int f = 0; f < PS_ST_N; f++) {
+        sum[f] = c->stat[lane][f];
+        for (int o = 32; o > 0; o >>= 1) sum[f] += __shfl_xor(sum[f], o, 64);
+    }
+    if (lane < 4) out->sizes[lane] = sizes[lane];
+    if (lane == 0) {
+        out->overflow = overflow;
+#pragma unroll
+        for (int f = 0; f < PS_ST_N; f++) out->sum[f] = (long long)sum[f];
+    }
+    if (overflow && !reset) return;
+#pragma unroll
+    for (int f = 0; f < PS_ST_N; f++) c->stat[lane][f] = c->pend[lane][f] = 0;
+    if (lane == 0) c->overflow = 0;
+    if (lane < 4) sizes[lane] = 0;
 }
 
 
@@ -719,7 +765,7 @@ __device__ __forceinline__ void ps_store_scan(T* out, int64_t wbase, int64_t n, 
 // the flush is split.  Called by the 64 lanes of one wave.
 template <typename T>
 __device__ __forceinline__ void ps_scan_total(T tot, int64_t n, int64_t cap, T* out, uint32_t* total_out,
-                                              const PsCounters* c, unsigned long long pieces = 0)
+                                              PsCounters* c, int* flag, unsigned long long pieces = 0)
 {
     const int lane = threadIdx.x & 63;
     if (lane == 0 && n <= cap) {
@@ -732,7 +778,7 @@ __device__ __forceinline__ void ps_scan_total(T tot, int64_t n, int64_t cap, T* 
     if constexpr (sizeof(T) == 8) {
         if (lane == 0 && pieces != (uint32_t)tot) {
             if (total_out) atomicMax(total_out + 2, 0xffffffffu);
-            atomicOr((int*)&c->overflow, 1);
+            ps_overflow(c, 1, flag);
         }
     }
 }
@@ -776,8 +822,8 @@ __device__ __forceinline__ T ps_block_sum_prefix(const T* partial, int end, T* l
 template <typename T>
 __global__ void __launch_bounds__(256) k_scan_final(const T* __restrict__ in, const uint32_t* n_ptr, int64_t n_host,
                                                     const T* __restrict__ partial, int nb, int pgran, T* __restrict__ out,
-                                                    uint32_t* total_out, int64_t cap, const PsCounters* c,
-                                                    uint32_t* heavy)
+                                                    uint32_t* total_out, int64_t cap, PsCounters* c,
+                                                    uint32_t* heavy, int* flag)
 {
     __shared__ T lds[4];
     const bool poisoned = c && ps_poisoned(c);
@@ -793,7 +839,7 @@ __global__ void __launch_bounds__(256) k_scan_final(const T* __restrict__ in, co
     else if (mine) before = ps_block_sum_prefix(partial, blockIdx.x * (SCAN_BLOCK / pgran), lds);
     if (poisoned) return;
     const unsigned long long pieces = ps_wave_sum64(pend);
-    if (blockIdx.x == 0 && threadIdx.x < 64) ps_scan_total(total, n, cap, out, total_out, c, pieces);
+    if (blockIdx.x == 0 && threadIdx.x < 64) ps_scan_total(total, n, cap, out, total_out, c, flag, pieces);
     if (!mine) return;
     T s = 0;
 #pragma unroll
@@ -828,7 +874,7 @@ struct PsDirectWave {
 };
 __global__ void __launch_bounds__(1024) k_scan_direct(const unsigned long long* __restrict__ in, int64_t n,
                                                       unsigned long long* __restrict__ out, uint32_t* total_out,
-                                                      const PsCounters* c, uint32_t* heavy)
+                                                      PsCounters* c, uint32_t* heavy, int* flag)
 {
     typedef unsigned long long T;
     __shared__ PsDirectWave xw[16];
@@ -901,7 +947,7 @@ __global__ void __launch_bounds__(1024) k_scan_direct(const unsigned long long* 
         out[i] = oa;
     }
     if (blockIdx.x == gridDim.x - 1 && wave == 0) {
-        ps_scan_total(before + btot, n, n, out, total_out, c, ps_wave_sum64(pend));
+        ps_scan_total(before + btot, n, n, out, total_out, c, flag, ps_wave_sum64(pend));
         if (heavy && lane == 0) heavy[0] = hbefore + hbtot;
     }
 }
@@ -971,7 +1017,7 @@ __global__ void __launch_bounds__(1024) k_scan_parts(const uint32_t* __restrict_
         for (int j = 0; j < 4; j++)
             if (i + j < n) out[i + j] = o[j];
     }
-    if (blockIdx.x == gridDim.x - 1 && wave == 0) ps_scan_total(before + btot, n, n, out, total_out, (const PsCounters*)nullptr);
+    if (blockIdx.x == gridDim.x - 1 && wave == 0) ps_scan_total(before + btot, n, n, out, total_out, (PsCounters*)nullptr, nullptr);
 }
 
 // Triangle of row item i: the t with row_off[t] <= i < row_off[t + 1]
@@ -1057,7 +1103,7 @@ __global__ void __launch_bounds__(256, 8) k_span(const PsTri* __restrict__ tris,
                                               int64_t T, int64_t cap,
                                               PsSpan* __restrict__ spans, unsigned long long* __restrict__ tcnt,
                                               const PsView* __restrict__ views, int n_views, int chunk_w, int tile_rows,
-                                              int tile_cols, uint32_t* heavy, uint32_t* wide, PsCounters* cnt)
+                                              int tile_cols, uint32_t* heavy, uint32_t* wide, PsCounters* cnt, int* flag)
 {
     // per wave: pieces | runs << 16 of the tiles [kmin, kmin + SPAN_BINS) its spans touch
     __shared__ uint32_t bins_all[4][SPAN_BINS];
@@ -1072,7 +1118,7 @@ __global__ void __launch_bounds__(256, 8) k_span(const PsTri* __restrict__ tris,
     if (poisoned) return;
     if (heavy && blockIdx.x == 0 && threadIdx.x == 0) heavy[0] = 0;   // the two-pass tile scan lists heavy tiles atomically
     if (R > cap) {   // more rows than span records: flag it, write nothing
-        if (threadIdx.x == 0 && blockIdx.x == 0) atomicOr(&cnt->overflow, 1);
+        if (threadIdx.x == 0 && blockIdx.x == 0) ps_overflow(cnt, 1, flag);
         return;
     }
     uint32_t all_spans = 0, all_pieces = 0, all_frags = 0;   // the lane's statistics, added up once per wave
@@ -1198,7 +1244,7 @@ __global__ void __launch_bounds__(256, 8) k_span(const PsTri* __restrict__ tris,
 // k_span left must cover the run (they always do: both kernels visit the same
 // tiles); 0xffffffff, and the flag set, if they do not: never write outside.
 __device__ __forceinline__ uint32_t ps_reserve_run(const PsFrame& f, unsigned long long* tcnt, uint32_t k, uint32_t n,
-                                                   uint32_t mark, uint32_t key, int64_t cap, PsCounters* cnt)
+                                                   uint32_t mark, uint32_t key, int64_t cap, PsCounters* cnt, int* flag)
 {
     const unsigned long long take = (unsigned long long)n | (1ull << 32);
     const unsigned long long left = atomicAdd(&tcnt[k], (unsigned long long)0 - take);
@@ -1206,7 +1252,7 @@ __device__ __forceinline__ uint32_t ps_reserve_run(const PsFrame& f, unsigned lo
     const uint32_t fp = (uint32_t)end - (uint32_t)left;
     const uint32_t slot = (uint32_t)(end >> 32) - (uint32_t)(left >> 32);
     if ((uint32_t)left < n || (uint32_t)(left >> 32) == 0u || (uint64_t)fp + n > (uint64_t)cap) {
-        atomicOr(&cnt->overflow, 2);
+        ps_overflow(cnt, 2, flag);
         return 0xffffffffu;
     }
     f.runs[2 * (size_t)slot] = fp | mark;
@@ -1231,7 +1277,7 @@ __device__ __forceinline__ void ps_wide_spans(const PsSpan* __restrict__ spans, 
                                               const PsTri* __restrict__ tris, const PsDraw* __restrict__ draws,
                                               const float* __restrict__ vary, int nvs, const uint32_t* __restrict__ wide,
                                               unsigned long long* __restrict__ tcnt, PsSeg* __restrict__ segs,
-                                              float* __restrict__ ck, int64_t cap, PsCounters* cnt)
+                                              float* __restrict__ ck, int64_t cap, PsCounters* cnt, int* flag)
 {
     constexpr int SPW = 64 / G;
     const int lane = threadIdx.x & (PS_WAVE - 1), j = lane & (G - 1), grp = lane & ~(G - 1);
@@ -1292,7 +1338,7 @@ __device__ __forceinline__ void ps_wide_spans(const PsSpan* __restrict__ spans, 
                 const uint32_t k = st.g0 + (uint32_t)(q0 + j);
                 int lo, hi;
                 ps_span_tile_chunks(st, TC, k, lo, hi);
-                first = ps_reserve_run(f, tcnt, k, (uint32_t)(hi - lo + 1), PS_RUN_OWN, wave_id << 12 | in_wave << 6, cap, cnt);
+                first = ps_reserve_run(f, tcnt, k, (uint32_t)(hi - lo + 1), PS_RUN_OWN, wave_id << 12 | in_wave << 6, cap, cnt, flag);
             }
             for (int q = q0; q < min(q0 + G, maxnt); q++) {
                 const uint32_t s = (uint32_t)__shfl((int)first, grp + (q - q0), PS_WAVE);
@@ -1360,7 +1406,7 @@ __global__ void __launch_bounds__(256) k_segments(const PsSpan* __restrict__ spa
                                                   const PsDraw* __restrict__ draws, const float* __restrict__ vary, int nvs,
                                                   unsigned long long* __restrict__ tcnt, PsSeg* __restrict__ segs,
                                                   float* __restrict__ ck, int64_t cap, const uint32_t* __restrict__ wide,
-                                                  PsCounters* cnt)
+                                                  PsCounters* cnt, int* flag)
 {
     __shared__ uint32_t rel_all[4][SG_BATCH][PS_WAVE];   // per wave: [iteration][lane] offset in the run
     const bool poisoned = ps_poisoned(cnt);
@@ -1368,10 +1414,10 @@ __global__ void __launch_bounds__(256) k_segments(const PsSpan* __restrict__ spa
     const int64_t S = (uint32_t)f.tstart[f.n_tiles];
     if (poisoned) return;
     if (S > cap) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&cnt->overflow, 1);
+        if (blockIdx.x == 0 && threadIdx.x == 0) ps_overflow(cnt, 1, flag);
         return;
     }
-    ps_wide_spans<G>(spans, R, f, tris, draws, vary, nvs, wide, tcnt, segs, ck, cap, cnt);
+    ps_wide_spans<G>(spans, R, f, tris, draws, vary, nvs, wide, tcnt, segs, ck, cap, cnt, flag);
     const int CW = f.chunk_w, TC = f.tile_cols;
     int64_t tb1 = 0;   // the only view of a one-view flush, read once
     int ntx1 = 0;
@@ -1431,7 +1477,7 @@ __global__ void __launch_bounds__(256) k_segments(const PsSpan* __restrict__ spa
             }
             if (nb == 0) break;
             uint32_t first = 0xffffffffu;
-            if (lane < nb) first = ps_reserve_run(f, tcnt, bk, bn, 0u, wave_id << 12, cap, cnt);
+            if (lane < nb) first = ps_reserve_run(f, tcnt, bk, bn, 0u, wave_id << 12, cap, cnt, flag);
             // every lane walks its pieces of the batch's tiles
             const int maxtb = __builtin_amdgcn_readfirstlane(ps_wave_max((uint32_t)ntb));
             for (int q = 0; q < maxtb; q++) {
@@ -2489,6 +2535,18 @@ void psk_fills(hipStream_t s, const PsFill* fills, int n, int64_t max_pieces, co
     hipLaunchKernelGGL(k_fills, dim3((unsigned)g, n), dim3(256), 0, s, fills, c);
 }
 
+void psk_few_fills(hipStream_t s, const PsFewFills& fills, int n, int64_t max_pieces, const PsCounters* c)
+{
+    if (n <= 0) return;
+    int64_t g = max_pieces < 1 ? 1 : max_pieces; if (g > 4096) g = 4096;
+    hipLaunchKernelGGL(k_few_fills, dim3((unsigned)g, n), dim3(256), 0, s, fills, c);
+}
+
+void psk_finish(hipStream_t s, PsCounters* c, uint32_t* sizes, PsFinish* out, bool reset)
+{
+    hipLaunchKernelGGL(k_finish, dim3(1), dim3(64), 0, s, c, sizes, out, reset ? 1 : 0);
+}
+
 
 int psk_setup_block() { return 128; }
 
@@ -2525,28 +2583,28 @@ void psk_scan_parts(hipStream_t s, const uint32_t* in, int64_t n, uint32_t* out,
 int psk_heavy_cap() { return PS_HEAVY_MAX; }
 
 void psk_scan_tiles(hipStream_t s, const unsigned long long* tcnt, int64_t n, unsigned long long* tstart,
-                    unsigned long long* partial, uint32_t* total_out, const PsCounters* c, uint32_t* heavy)
+                    unsigned long long* partial, uint32_t* total_out, PsCounters* c, uint32_t* heavy, int* flag)
 {
     if (n <= SCAN_DIRECT_MAX) {
         hipLaunchKernelGGL(k_scan_direct, dim3(gsz(n, DIRECT_BLOCK)), dim3(1024), 0, s, tcnt, n, tstart,
-                           total_out, c, heavy);
+                           total_out, c, heavy, flag);
         return;
     }
     int nb = psk_scan_blocks(n);
     hipLaunchKernelGGL(k_scan_reduce<unsigned long long>, dim3(nb), dim3(256), 0, s, tcnt, nullptr, n, partial, c);
     hipLaunchKernelGGL(k_scan_final<unsigned long long>, dim3(nb), dim3(256), 0, s, tcnt, nullptr, n, partial, nb,
-                       SCAN_BLOCK, tstart, total_out, n, c, heavy);
+                       SCAN_BLOCK, tstart, total_out, n, c, heavy, flag);
 }
 
 
 void psk_span(hipStream_t s, const PsTri* tris, const uint32_t* row_off, const uint32_t* bstart, int64_t T,
               PsSpan* spans, unsigned long long* tcnt, const PsView* views, int n_views, int chunk_w, int tile_rows,
-              int64_t cap, uint32_t* heavy, uint32_t* wide, PsCounters* cnt)
+              int64_t cap, uint32_t* heavy, uint32_t* wide, PsCounters* cnt, int* flag)
 {
     int g = gsz(cap, 256); if (g > 2048) g = 2048;
     const int tile_cols = 64 / tile_rows;
     hipLaunchKernelGGL(k_span, dim3(g), dim3(256), 0, s, tris, row_off, bstart, T, cap, spans, tcnt, views, n_views,
-                       chunk_w, tile_rows, tile_cols, heavy, wide, cnt);
+                       chunk_w, tile_rows, tile_cols, heavy, wide, cnt, flag);
 }
 
 void psk_scan_rows(hipStream_t s, const uint32_t* in, int64_t n, uint32_t* out, uint32_t* partial, uint32_t* total_out,
@@ -2559,12 +2617,12 @@ void psk_scan_rows(hipStream_t s, const uint32_t* in, int64_t n, uint32_t* out, 
 
 void psk_segments(hipStream_t s, const PsSpan* spans, const uint32_t* row_off, int64_t T, const PsFrame& f,
                   const PsTri* tris, const PsDraw* draws, const float* vary, int nvs, unsigned long long* tcnt, PsSeg* segs,
-                  float* ck, int64_t span_cap, int64_t seg_cap, const uint32_t* wide, PsCounters* cnt)
+                  float* ck, int64_t span_cap, int64_t seg_cap, const uint32_t* wide, PsCounters* cnt, int* flag)
 {
     int g = gsz(span_cap, 256); if (g > 2048) g = 2048;
 #define SG_LAUNCH(G)                                                                                                  \
     hipLaunchKernelGGL(k_segments<G>, dim3(g), dim3(256), 0, s, spans, row_off, T, f, tris, draws, vary, nvs, tcnt,   \
-                       segs, ck, seg_cap, wide, cnt)
+                       segs, ck, seg_cap, wide, cnt, flag)
     static_assert(PS_MAX_NV <= 24, "a lane per varying float beside the 8 of the record");
     if (nvs <= 8) SG_LAUNCH(16);
     else SG_LAUNCH(32);

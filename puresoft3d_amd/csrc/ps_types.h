@@ -162,6 +162,10 @@ struct PsFill {
     int pad;
 };
 
+// fills passed as kernel arguments
+#define PS_FEW_FILLS 8
+struct PsFewFills { PsFill f[PS_FEW_FILLS]; };
+
 // Device-side counters.  Statistics are striped over 64 slots (by block
 // index) so that waves of many blocks do not serialise on one address.  The
 // kernels before a flush's raster pass count into `pend`; the raster pass,
@@ -178,4 +182,12 @@ struct PsCounters {
     int overflow;
     int pad[63];
     unsigned long long pend[PS_STRIPES][PS_ST_N];
+};
+
+// What a sync reads, in pinned host memory: the overflow flag, the row and piece
+// totals with their maxima over the log, and the statistics' sums.
+struct PsFinish {
+    int overflow, pad;
+    uint32_t sizes[4];
+    long long sum[PS_ST_N];
 };

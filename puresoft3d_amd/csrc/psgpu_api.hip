@@ -216,12 +216,15 @@ struct psgpu_ctx {
     // flush that needs more is split in two and re-run
     int64_t max_spans = ((int64_t)1 << 26) - 64, max_segs = ((int64_t)1 << 31) - 64;
     uint32_t* d_sizes = nullptr;
-    uint32_t* h_sizes = nullptr;
-    // per logged command: the overflow flag as it stood after the command ran
+    // per logged command (pinned; kernels of an eager flush set their command's
+    // word where it overflows its scratch), and one more word for flushes that
+    // are not logged: captured ones and psgpu_sync_noalloc's
     static const int kFlagCap = 16384;
     int* h_flags = nullptr;
+    int* flush_flag = nullptr;     // the word of the command being run
     PsCounters* d_cnt = nullptr;
-    PsCounters* h_cnt = nullptr;
+    PsFinish* h_fin = nullptr;     // what a sync reads (pinned)
+    bool copies_pending = false;   // the copy stream has work since the last sync
     // command staging (pinned), ring of slots
     static const int kStage = 4;
     uint8_t* h_stage[kStage] = {nullptr};
@@ -608,6 +611,7 @@ int run_flush(psgpu_ctx* c, const Cmd& cmd, uint8_t* staged)
     }
 
     hipStream_t s = c->stream;
+    int* flag = c->in_stream_capture || c->fixed_scratch ? c->h_flags + psgpu_ctx::kFlagCap : c->flush_flag;
     int nd = blob.nd;
     const PsView* dv = f.views;
     // a flush of one programme has one setup launch, which also leaves the
@@ -648,11 +652,11 @@ int run_flush(psgpu_ctx* c, const Cmd& cmd, uint8_t* staged)
     {
         ProfScope p(c, "span");
         psk_span(s, c->fb.tris.p, c->fb.rowoff.p, c->fb.bstart.p, T, c->fb.spans.p, c->fb.tcnt.p, dv,
-                 f.n_views, f.chunk_w, f.tile_rows, c->fb.span_cap, heavy, c->fb.wide.p, c->d_cnt);
+                 f.n_views, f.chunk_w, f.tile_rows, c->fb.span_cap, heavy, c->fb.wide.p, c->d_cnt, flag);
     }
     {
         ProfScope p(c, "scan_tiles");
-        psk_scan_tiles(s, c->fb.tcnt.p, f.n_tiles, c->fb.tstart.p, c->fb.tpartial.p, c->d_sizes + 1, c->d_cnt, heavy);
+        psk_scan_tiles(s, c->fb.tcnt.p, f.n_tiles, c->fb.tstart.p, c->fb.tpartial.p, c->d_sizes + 1, c->d_cnt, heavy, flag);
     }
     f.tstart = c->fb.tstart.p;
     f.runs = c->fb.runs.p;
@@ -661,7 +665,7 @@ int run_flush(psgpu_ctx* c, const Cmd& cmd, uint8_t* staged)
     {
         ProfScope p(c, "segments");
         psk_segments(s, c->fb.spans.p, c->fb.rowoff.p, T, f, c->fb.tris.p, dd, c->fb.vary.p, nvs, c->fb.tcnt.p,
-                     c->fb.segs.p, c->fb.ck.p, c->fb.span_cap, c->fb.seg_cap, c->fb.wide.p, c->d_cnt);
+                     c->fb.segs.p, c->fb.ck.p, c->fb.span_cap, c->fb.seg_cap, c->fb.wide.p, c->d_cnt, flag);
     }
     if (imm) {
         ProfScope p(c, "raster");
@@ -693,6 +697,16 @@ int run_flush(psgpu_ctx* c, const Cmd& cmd, uint8_t* staged)
 int run_clears(psgpu_ctx* c, const Cmd& cmd, uint8_t* staged)
 {
     if (cmd.fills.empty()) return PSGPU_OK;
+    int64_t mx = 1;
+    for (const PsFill& fl : cmd.fills) mx = std::max<int64_t>(mx, psk_fill_pieces(fl.rows, fl.width));
+    if (cmd.fills.size() <= PS_FEW_FILLS) {
+        PsFewFills few = {};
+        std::copy(cmd.fills.begin(), cmd.fills.end(), few.f);
+        ProfScope p(c, "clear");
+        psk_few_fills(c->stream, few, (int)cmd.fills.size(), mx, c->d_cnt);
+        HIPCHK(c, hipGetLastError());
+        return PSGPU_OK;
+    }
     Blob blob;
     blob.off_views = blob.off_fills = 0;
     blob.nf = (int)cmd.fills.size();
@@ -701,8 +715,6 @@ int run_clears(psgpu_ctx* c, const Cmd& cmd, uint8_t* staged)
     uint8_t* dev = staged;
     int rc;
     if (!dev && (rc = stage_blob(c, blob, &dev))) return rc;
-    int64_t mx = 1;
-    for (const PsFill& fl : cmd.fills) mx = std::max<int64_t>(mx, psk_fill_pieces(fl.rows, fl.width));
     ProfScope p(c, "clear");
     for (size_t i = 0; i < cmd.fills.size(); i += 65535)
         psk_fills(c->stream, (const PsFill*)dev + i, (int)std::min<size_t>(65535, cmd.fills.size() - i), mx, c->d_cnt);
@@ -716,6 +728,7 @@ int run_copy(psgpu_ctx* c, const CopyRegion& r)
 {
     HIPCHK(c, hipEventRecord(c->copy_ev, c->stream));
     HIPCHK(c, hipStreamWaitEvent(c->copy_stream, c->copy_ev, 0));
+    c->copies_pending = true;
     HIPCHK(c, hipMemcpy2DAsync(r.dst, r.dst_pitch, r.src, r.src_pitch, r.width_bytes, r.rows, hipMemcpyDeviceToHost,
                                c->copy_stream));
     return PSGPU_OK;
@@ -822,20 +835,16 @@ bool split_flush(psgpu_ctx* c, size_t idx)
     return true;
 }
 
-// remember whether the overflow flag was already set when command i finished:
-// the first command that finished with it set is where a replay starts.
-// Only an eager flush can set it (clears, copies and post-processes have no
-// intermediate buffers, and a graph replay fits the buffers it was sized
-// for), so the first command found set is always a flush and the others are
-// marked clear without a copy.
-int mark_done(psgpu_ctx* c, int i)
+// run logged command i.  Its flag word says whether it overflowed its scratch:
+// the first command found with it set is where a replay starts.  Only an eager
+// flush can set it (clears, copies and post-processes have no intermediate
+// buffers, and a graph replay fits the buffers it was sized for); commands
+// after one that overflowed do nothing until they are replayed.
+int run_logged(psgpu_ctx* c, size_t i)
 {
-    if (c->log[i].type != CMD_FLUSH) {
-        c->h_flags[i] = 0;
-        return PSGPU_OK;
-    }
-    HIPCHK(c, hipMemcpyAsync(c->h_flags + i, &c->d_cnt->overflow, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    return PSGPU_OK;
+    c->h_flags[i] = 0;
+    c->flush_flag = c->h_flags + i;
+    return run_cmd(c, c->log[i]);
 }
 
 // a command is either recorded (between capture begin/end) or logged and run
@@ -850,9 +859,7 @@ int submit(psgpu_ctx* c, Cmd&& cmd)
         if (rc) return rc;
     }
     c->log.push_back(std::move(cmd));
-    int rc = run_cmd(c, c->log.back());
-    if (rc) return rc;
-    return mark_done(c, (int)c->log.size() - 1);
+    return run_logged(c, c->log.size() - 1);
 }
 
 // Clears that a flush can apply itself: a clear of a view's whole depth
@@ -956,44 +963,54 @@ int add_fill(psgpu_ctx* c, void* ptr, int64_t rows, int64_t width, int64_t scan,
     return PSGPU_OK;
 }
 
+// the statistics of the log that ended
+void add_stats(psgpu_ctx* c)
+{
+    const long long* sum = c->h_fin->sum;
+    c->stats.tris_culled += sum[PS_ST_CULLED];
+    c->stats.tris_zrejected += sum[PS_ST_ZREJ];
+    c->stats.tris_dropped += sum[PS_ST_DROPPED];
+    c->stats.spans += sum[PS_ST_SPANS];
+    c->stats.frags_rasterised += sum[PS_ST_FRAGS];
+    c->stats.frags_shaded += sum[PS_ST_SHADED];
+    c->stats.segments += sum[PS_ST_SEGS];
+}
+
 int do_sync(psgpu_ctx* c)
 {
     if (c->capturing) return fail(c, PSGPU_ERR_STATE, "not allowed while recording a command list");
     int rc = queue_to_log(c);
     if (rc) return rc;
-    const int64_t span_cap0 = c->fb.span_cap, seg_cap0 = c->fb.seg_cap;
-    for (int attempt = 0; attempt < 64; attempt++) {
-        HIPCHK(c, hipMemcpyAsync(c->h_cnt, c->d_cnt, sizeof(PsCounters), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipMemcpyAsync(c->h_sizes, c->d_sizes, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+    if (c->log.empty() && c->fences.empty()) {
+        // nothing logged since the last sync, which left the counters at zero;
+        // the caller may have put work of its own on the stream
         HIPCHK(c, hipStreamSynchronize(c->stream));
         HIPCHK(c, hipStreamSynchronize(c->copy_stream));
+        return PSGPU_OK;
+    }
+    const int64_t span_cap0 = c->fb.span_cap, seg_cap0 = c->fb.seg_cap;
+    for (int attempt = 0; attempt < 64; attempt++) {
+        psk_finish(c->stream, c->d_cnt, c->d_sizes, c->h_fin, false);
+        HIPCHK(c, hipGetLastError());
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        if (c->copies_pending) HIPCHK(c, hipStreamSynchronize(c->copy_stream));
+        c->copies_pending = false;
         if (c->profiling) prof_collect(c);
-        if (!c->h_cnt->overflow) {
-            int64_t sum[PS_ST_N] = {0};
-            for (int k = 0; k < PS_STRIPES; k++)
-                for (int f = 0; f < PS_ST_N; f++) sum[f] += (int64_t)c->h_cnt->stat[k][f];
-            c->stats.tris_culled += sum[PS_ST_CULLED];
-            c->stats.tris_zrejected += sum[PS_ST_ZREJ];
-            c->stats.tris_dropped += sum[PS_ST_DROPPED];
-            c->stats.spans += sum[PS_ST_SPANS];
-            c->stats.frags_rasterised += sum[PS_ST_FRAGS];
-            c->stats.frags_shaded += sum[PS_ST_SHADED];
-            c->stats.segments += sum[PS_ST_SEGS];
+        if (!c->h_fin->overflow) {
+            add_stats(c);
             c->log.clear();
             for (const Fence& fe : c->fences) {
                 c->fence_ev_pool.push_back(fe.main_ev);
                 c->fence_ev_pool.push_back(fe.copy_ev);
             }
             c->fences.clear();
-            HIPCHK(c, hipMemsetAsync(c->d_cnt, 0, sizeof(PsCounters), c->stream));
-            HIPCHK(c, hipMemsetAsync(c->d_sizes, 0, 4 * sizeof(uint32_t), c->stream));
             return PSGPU_OK;
         }
-        if (c->h_cnt->overflow & 2)
+        if (c->h_fin->overflow & 2)
             return fail(c, PSGPU_ERR_STATE, "internal: a tile list did not match its counts");
         // grow and replay the log; a flush that needs more than one flush may
         // hold is split in two (and again, if a half still does)
-        int64_t need_spans = (int64_t)c->h_sizes[2], need_segs = (int64_t)c->h_sizes[3];
+        int64_t need_spans = (int64_t)c->h_fin->sizes[2], need_segs = (int64_t)c->h_fin->sizes[3];
         size_t first = 0;
         while (first < c->log.size() && !c->h_flags[first]) first++;
         // only eager flushes carry a copied flag; the others cannot overflow
@@ -1024,10 +1041,8 @@ int do_sync(psgpu_ctx* c)
         // a flush cut short leaves tile counts behind
         if (c->fb.tcnt.p)
             HIPCHK(c, hipMemsetAsync(c->fb.tcnt.p, 0, c->fb.tcnt.cap * sizeof(unsigned long long), c->stream));
-        for (size_t i = 0; i < c->log.size(); i++) {
-            if ((rc = run_cmd(c, c->log[i]))) return rc;
-            if ((rc = mark_done(c, (int)i))) return rc;
-        }
+        for (size_t i = 0; i < c->log.size(); i++)
+            if ((rc = run_logged(c, i))) return rc;
     }
     // give up with the capacities as they were, so later flushes stay usable
     c->fb.span_cap = span_cap0;
@@ -1102,8 +1117,7 @@ int graph_prepare(psgpu_ctx* c, Graph& g)
     for (const Cmd& cmd : g.cmds) {
         Cmd copy = cmd;
         c->log.push_back(std::move(copy));
-        if ((rc = run_cmd(c, c->log.back()))) return rc;
-        if ((rc = mark_done(c, (int)c->log.size() - 1))) return rc;
+        if ((rc = run_logged(c, c->log.size() - 1))) return rc;
     }
     if ((rc = do_sync(c))) return rc;
     if (c->stats.splits != splits) return graph_too_large(c);
@@ -1284,10 +1298,9 @@ int psgpu_create(int device, int width, int height, unsigned flags, psgpu_ctx** 
               hipMalloc((void**)&c->display, (size_t)width * height * 4) == hipSuccess &&
               hipMalloc((void**)&c->depth, (size_t)dscan * height * 4) == hipSuccess &&
               hipMalloc((void**)&c->d_cnt, sizeof(PsCounters)) == hipSuccess &&
-              hipHostMalloc((void**)&c->h_cnt, sizeof(PsCounters)) == hipSuccess &&
+              hipHostMalloc((void**)&c->h_fin, sizeof(PsFinish)) == hipSuccess &&
               hipMalloc((void**)&c->d_sizes, 4 * sizeof(uint32_t)) == hipSuccess &&
-              hipHostMalloc((void**)&c->h_sizes, 4 * sizeof(uint32_t)) == hipSuccess &&
-              hipHostMalloc((void**)&c->h_flags, psgpu_ctx::kFlagCap * sizeof(int)) == hipSuccess &&
+              hipHostMalloc((void**)&c->h_flags, (psgpu_ctx::kFlagCap + 1) * sizeof(int)) == hipSuccess &&
               hipMemsetAsync(c->display, 0, (size_t)width * height * 4, c->stream) == hipSuccess &&
               hipMemsetAsync(c->depth, 0, (size_t)dscan * height * 4, c->stream) == hipSuccess &&
               hipMemsetAsync(c->d_cnt, 0, sizeof(PsCounters), c->stream) == hipSuccess &&
@@ -1297,7 +1310,9 @@ int psgpu_create(int device, int width, int height, unsigned flags, psgpu_ctx** 
         psgpu_destroy(c);
         return PSGPU_ERR_DEVICE;
     }
-    memset(c->h_cnt, 0, sizeof(PsCounters));
+    memset(c->h_fin, 0, sizeof(PsFinish));
+    memset(c->h_flags, 0, (psgpu_ctx::kFlagCap + 1) * sizeof(int));
+    c->flush_flag = c->h_flags + psgpu_ctx::kFlagCap;
     *out = c;
     return PSGPU_OK;
 }
@@ -1309,8 +1324,7 @@ int psgpu_destroy(psgpu_ctx* c)
     if (c->copy_stream) hipStreamSynchronize(c->copy_stream);
     auto fr = [](void* p) { if (p) hipFree(p); };
     fr(c->display); fr(c->depth); fr(c->d_cnt); fr(c->d_sizes);
-    if (c->h_cnt) hipHostFree(c->h_cnt);
-    if (c->h_sizes) hipHostFree(c->h_sizes);
+    if (c->h_fin) hipHostFree(c->h_fin);
     if (c->h_flags) hipHostFree(c->h_flags);
     for (auto& t : c->tex) fr(t.d);
     for (auto& v : c->vbo) fr(v.d);
@@ -2256,8 +2270,7 @@ int psgpu_capture_end(psgpu_ctx* c, int* out_graph)
     for (const Cmd& cmd : g.cmds) {
         Cmd copy = cmd;
         c->log.push_back(std::move(copy));
-        if ((rc = run_cmd(c, c->log.back()))) return rc;
-        if ((rc = mark_done(c, (int)c->log.size() - 1))) return rc;
+        if ((rc = run_logged(c, c->log.size() - 1))) return rc;
     }
     if ((rc = do_sync(c))) return rc;
     if (c->stats.splits != splits) return graph_too_large(c);
@@ -2403,29 +2416,16 @@ int psgpu_sync_noalloc(psgpu_ctx* c)
                                  : run_flush(c, flush, blob_dev);
         }
     }
-    // wait, then read and reset the counters as psgpu_sync does
-    hipError_t e = hipMemcpyAsync(c->h_cnt, c->d_cnt, sizeof(PsCounters), hipMemcpyDeviceToHost, c->stream);
+    // wait; read and reset the counters as psgpu_sync does, after an overflow too
+    psk_finish(c->stream, c->d_cnt, c->d_sizes, c->h_fin, true);
+    hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     std::swap(c->fb, sb);
     c->fixed_scratch = false;
     if (rc) return rc;
     if (e != hipSuccess) return fail(c, PSGPU_ERR_DEVICE, "%s", hipGetErrorString(e));
-    bool overflow = c->h_cnt->overflow != 0;
-    if (!overflow) {
-        int64_t sum[PS_ST_N] = {0};
-        for (int k = 0; k < PS_STRIPES; k++)
-            for (int f = 0; f < PS_ST_N; f++) sum[f] += (int64_t)c->h_cnt->stat[k][f];
-        c->stats.tris_culled += sum[PS_ST_CULLED];
-        c->stats.tris_zrejected += sum[PS_ST_ZREJ];
-        c->stats.tris_dropped += sum[PS_ST_DROPPED];
-        c->stats.spans += sum[PS_ST_SPANS];
-        c->stats.frags_rasterised += sum[PS_ST_FRAGS];
-        c->stats.frags_shaded += sum[PS_ST_SHADED];
-        c->stats.segments += sum[PS_ST_SEGS];
-    }
-    HIPCHK(c, hipMemsetAsync(c->d_cnt, 0, sizeof(PsCounters), c->stream));
-    HIPCHK(c, hipMemsetAsync(c->d_sizes, 0, 4 * sizeof(uint32_t), c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    const bool overflow = c->h_fin->overflow != 0;
+    if (!overflow) add_stats(c);
     if (overflow)
         return fail(c, PSGPU_ERR_NOMEM,
                     "the flush's spans or pieces exceed what the %zu-byte static scratch array holds (%lld spans, "

@@ -113,8 +113,8 @@ __device__ __forceinline__ int64_t ps_xcd_remap(int64_t b, int64_t n)
     return s * (8 * G) + (j & 7) * G + (j >> 3);
 }
 
-// where triangle tri of draw d finds its three vertices' varyings
-__device__ __forceinline__ int ps_vary_index(const PsDraw& d, int tri) { return tri + d.vary_delta; }
+// the programme of a triangle's draw
+__device__ __forceinline__ int ps_tri_prog(const PsTri& t) { return (int)(t.vflags >> 4); }
 
 // the first of the two texcoord varyings the mip-level gradients use (-1: none)
 template <class P> __device__ constexpr int ps_grad_iu()
@@ -498,8 +498,9 @@ __global__ void __launch_bounds__(128, 3) k_setup(const PsDraw* __restrict__ dra
                 tr.split = split;
                 tr.code = code | ((uint32_t)di << 8);
                 tr.view = d.view;
-                tr.vflags = (uint32_t)(d.behavior & 3) | (d.writes_colour ? 4u : 0u);
-                tr.pad[0] = tr.pad[1] = 0;
+                tr.vflags = (uint32_t)(d.behavior & 3) | (d.writes_colour ? 4u : 0u) | (uint32_t)PROG << 4;
+                tr.vary = (int)t + d.vary_delta;
+                tr.pad = 0;
                 n = (uint32_t)(last - first + 1);
                 // a triangle without rows has no spans: nothing reads its records
                 // (rows can lie outside the vertices' y range, where edges
@@ -1320,7 +1321,7 @@ __device__ __forceinline__ void ps_wide_spans(const PsSpan* __restrict__ spans, 
                 PsSpanGeom g;
                 ps_span_geom(tr, y, left, right, L, Rr, g);
                 if (j >= 8 && j - 8 < nv) {
-                    const float* u0 = vary + (int64_t)ps_vary_index(d, sp.tri) * 3 * nvs + (j - 8);
+                    const float* u0 = vary + (int64_t)tr.vary * 3 * nvs + (j - 8);
                     ps_span_varyings_n<1>(g, u0, u0 + nvs, u0 + 2 * nvs, &v, &step, 1);
                 }
             }
@@ -2255,7 +2256,7 @@ __global__ void __launch_bounds__(512) k_raster_imm(const PsSpan* __restrict__ s
                         int right = ps_cvt_i32(ps_edge_eval(Re, (float)y) + 0.5f);
                         PsSpanGeom g;
                         ps_span_geom(tr, y, left, right, Le, Re, g);
-                        const float* u0 = vary + (int64_t)ps_vary_index(d, sp.tri) * 3 * nvs;
+                        const float* u0 = vary + (int64_t)tr.vary * 3 * nvs;
                         ps_span_varyings<P::NV>(g, u0, u0 + nvs, u0 + 2 * nvs, vs, vt);
                         int xs = sp.x1;
                         if (a > sp.x1 && ps_span_has_ck(sp) && wc) {
@@ -2318,7 +2319,7 @@ __global__ void __launch_bounds__(512) k_raster_imm(const PsSpan* __restrict__ s
 // triangle exactly as k_span did; only pixels of a piece with a varying
 // checkpoint read that piece and its span first.
 template <int PROG>
-__global__ void __launch_bounds__(256, 7) k_shade(const PsSpan* __restrict__ spans, const PsSeg* __restrict__ segs,
+__global__ void __launch_bounds__(256, 6) k_shade(const PsSpan* __restrict__ spans, const PsSeg* __restrict__ segs,
                                                const float* __restrict__ ck, const PsTri* __restrict__ tris,
                                                const float* __restrict__ vary, int nvs, const float* __restrict__ grads,
                                                const PsDraw* __restrict__ draws, PsFrame f, const PsCounters* cnt, int clears)
@@ -2354,8 +2355,8 @@ __global__ void __launch_bounds__(256, 7) k_shade(const PsSpan* __restrict__ spa
         cfa = sg.cf2;
     }
     const PsTri tr = tris[tri];
-    ps_with_draw(draws, (int)(tr.code >> 8), [&](const PsDraw& d) {
-    if (d.prog != PROG) return;
+    if (ps_tri_prog(tr) != PROG) return;
+    const int di = (int)(tr.code >> 8);
     PsEdge L, R;
     ps_row_edges(tr, y, L, R);
     int left = ps_cvt_i32(ps_edge_eval(L, (float)y) + 0.5f);
@@ -2364,7 +2365,7 @@ __global__ void __launch_bounds__(256, 7) k_shade(const PsSpan* __restrict__ spa
     ps_span_geom(tr, y, left, right, L, R, g);
     float cf2, cf2_step, pz, pz_step;
     ps_span_vis(tr, g, cf2, cf2_step, pz, pz_step);
-    const float* u0 = vary + (int64_t)ps_vary_index(d, tri) * 3 * nvs;
+    const float* u0 = vary + (int64_t)tr.vary * 3 * nvs;
     float vs[P::NV > 0 ? P::NV : 1], vt[P::NV > 0 ? P::NV : 1];
     ps_span_varyings<P::NV>(g, u0, u0 + nvs, u0 + 2 * nvs, vs, vt);
     // from the span's first pixel (leftClamped), or from the checkpoint,
@@ -2400,10 +2401,27 @@ __global__ void __launch_bounds__(256, 7) k_shade(const PsSpan* __restrict__ spa
         float4 g0 = gi[0], g1 = gi[1];
         grad[0] = g0.x; grad[1] = g0.y; grad[2] = g0.z; grad[3] = g0.w; grad[4] = g1.x; grad[5] = g1.y;
     }
+    // The programme, with the draw of the whole wave where it has only one: the
+    // record's fields then come in with scalar loads and the branches on them
+    // are scalar.  The index is opaque before it is made uniform: knowing it
+    // equal to di, the compiler would index with di after all.  The geometry
+    // stays out of the two branches, which spill with it.  Six waves per SIMD:
+    // seven spill three registers for Blinn-Phong, 13 for its shadowed form.
+    // Terrain 3840x2160 190 -> 176 us, 1920x1080 50 -> 46, 32 views 288 -> 267,
+    // shadowed 1280x720 31.5 -> 27.9 (a loop over the wave's draws, one copy of
+    // the code: 168, 50, 265, 38; waves of several draws on a list for a second
+    // kernel: 168 + 20, 45 + 11, 270, 29 + 10).
     uint32_t c;
-    if (P::fp(d, in, r, grad, c)) V.colour[crow * V.colour_scan + x] = c;
+    bool hit;
+    if (__ballot(di != __builtin_amdgcn_readfirstlane(di)) == 0) {
+        int du = di;
+        asm volatile("" : "+v"(du));
+        hit = P::fp(draws[__builtin_amdgcn_readfirstlane(du)], in, r, grad, c);
+    } else {
+        hit = P::fp(draws[di], in, r, grad, c);
+    }
+    if (hit) V.colour[crow * V.colour_scan + x] = c;
     else if (crow < V.cclear_rows) V.colour[crow * V.colour_scan + x] = V.cclear_value;
-    });
 }
 
 // ---------------------------------------------------------------------------

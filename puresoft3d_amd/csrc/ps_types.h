@@ -68,11 +68,12 @@ struct PsTri {
     int nrows;     // drawn rows (0 = no rows)
     int split;     // last row of the lower half (standing triangles)
     uint32_t code; // edge code | draw index << 8
-    // what the span and piece kernels need of the draw, without reading it:
-    // its view, and its depth behaviour bits | writes colour << 2
+    // what the later kernels need of the draw, without reading it:
+    // its view, and its depth behaviour bits | writes colour << 2 | programme << 4
     int view;
     uint32_t vflags;
-    int pad[2];
+    int vary;      // the triangle whose slot holds the three vertices' varyings (PsDraw::vary_delta)
+    int pad;
 };
 
 // One scanline span with at least one pixel (drawvao.cpp:66-110, interp.cpp:26-80).

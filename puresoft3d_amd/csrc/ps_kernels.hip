@@ -1558,17 +1558,14 @@ __device__ __forceinline__ void ps_sort_lanes(uint32_t& key, uint32_t& val, uint
 //
 // Window of up to 64 runs from run w0 on, one per lane: rbase = the run's
 // first piece, rv = the list position of that piece (0xffffffff past the last
-// run), vhi = the list position where the window ends, np = the smallest
-// power of two at least the window's runs.  A tile of at most 64 runs is
-// sorted here; longer lists come ordered by ps_order_runs, with each run's
-// key replaced by its list position.
+// run), vhi = the list position where the window ends.  A tile of at most 64
+// runs is sorted here; longer lists come ordered by ps_order_runs, with each
+// run's key replaced by its list position.
 __device__ __forceinline__ void ps_run_window(const uint32_t* rl, uint32_t nr, uint32_t w0, uint32_t n_list,
-                                              uint32_t& rbase, uint32_t& rv, uint32_t& vhi, int& np)
+                                              uint32_t& rbase, uint32_t& rv, uint32_t& vhi)
 {
     const uint32_t j = w0 + (threadIdx.x & 63);
     const uint32_t nw = min(nr - w0, 64u);
-    np = 1;
-    while ((uint32_t)np < nw) np <<= 1;
     if (nr <= 64) {
         uint32_t key = j < nr ? rl[2 * j + 1] : 0xffffffffu;
         rbase = j < nr ? rl[2 * j] : 0u;
@@ -1585,19 +1582,7 @@ __device__ __forceinline__ void ps_run_window(const uint32_t* rl, uint32_t nr, u
     }
 }
 
-// the piece at list position v of the window (rv[0] <= v; the walk that blends): the last run that
-// starts at or before v, found by a binary search over lanes [0, np)
-__device__ __forceinline__ uint32_t ps_run_piece(uint32_t rv, uint32_t rbase, uint32_t v, int np)
-{
-    if (np == 1) return (uint32_t)__builtin_amdgcn_readlane(rbase, 0) + (v - (uint32_t)__builtin_amdgcn_readlane(rv, 0));
-    int pos = 0;
-    for (int st = np >> 1; st >= 1; st >>= 1)
-        if (__shfl(rv, pos + st, 64) <= v) pos += st;
-    return __shfl(rbase, pos, 64) + (v - __shfl(rv, pos, 64));
-}
-
-// A tile with more than PS_LDS_RUNS runs (more than 64 in the walk that
-// blends): one wave sorts them by their keys from bit 6 up, which tell any two
+// A tile with more than PS_LDS_RUNS runs: one wave sorts them by their keys from bit 6 up, which tell any two
 // runs of a tile apart (LSD radix, 7-bit digits above the smallest, ping-ponging
 // between the tile's parts a and b of the two run arrays), then replaces each
 // run's key by the list position of its first piece.  cnt128: 128 words of
@@ -1673,18 +1658,10 @@ __device__ uint32_t* ps_order_runs(uint32_t* a, uint32_t* b, uint32_t nr, uint32
 // ---------------------------------------------------------------------------
 // raster: ordered depth test per bin
 // ---------------------------------------------------------------------------
-#define RA_CHUNK 128    // tile-list entries staged in LDS per pass
-#define RA_PER (RA_CHUNK / 64)
-
-// LDS of one wave: depth and winner columns [c][lane] (bank = lane), then the
-// staged pieces of the current chunk (SoA, in per-lane order), then per-lane
-// counts and offsets
-#define RA_WORDS(cw) ((cw) * 64 * 2 + RA_CHUNK * 7 + 128)
-
-// LDS of one wave of k_raster: the runs of a tile of 65 to PS_LDS_RUNS runs in
-// order (first piece, list position), which run starts at each position of a
-// batch, a spare pixel per lane, then depth and winner of the tile's pixels, pixel k of lane l's chunk
-// at [k * 64 + l]
+// LDS of one wave of the raster kernels: the runs of a tile of 65 to
+// PS_LDS_RUNS runs in order (first piece, list position), which run starts at
+// each position of a batch, a spare pixel per lane, then depth and winner (or
+// colour) of the tile's pixels, pixel k of lane l's chunk at [k * 64 + l]
 #define PS_LDS_RUNS 256
 #define RA_PIX_WORDS(cw) (PS_LDS_RUNS * 2 + 64 + 64 * 2 + (cw) * 64 * 2)
 
@@ -1897,8 +1874,7 @@ __global__ void __launch_bounds__(512, 5) k_raster(const PsSpan* __restrict__ sp
             rv = r.y;
             vhi = w0 + 64 < nr ? lruns[w0 + 64].y : n_list;
         } else {
-            int np;
-            ps_run_window(rl, nr, w0, n_list, rbase, rv, vhi, np);
+            ps_run_window(rl, nr, w0, n_list, rbase, rv, vhi);
         }
         const uint32_t vlo = (uint32_t)__builtin_amdgcn_readlane((int)rv, 0), delta = rbase - rv;
         // the records of the next batch are in flight while one is tested.  A
@@ -2064,34 +2040,39 @@ __global__ void __launch_bounds__(512, 5) k_raster(const PsSpan* __restrict__ sp
 // ---------------------------------------------------------------------------
 // A discarded fragment leaves the depth unchanged and a blended one depends
 // on the colour beneath it, so neither can be deferred to one shading pass
-// per pixel.  The same tile walk runs the programme's FP on every depth-test
-// pass, in submission order, and writes (or blends) the colour at once.
-template <int PROG, bool DEBUG>
+// per pixel.  As in k_raster the wave takes the tile's pieces 64 at a time,
+// one per lane; depth and colour of the tile stay in LDS.  What the programme
+// gives for a fragment does not depend on the order, only whether it counts
+// does: each lane runs the programme for the pixels of its piece, if a fragment
+// of the batch can pass, and the order is resolved per pixel in rounds
+// afterwards.
+// What bounds it is issue on the SIMDs that hold the layer's tiles, some
+// 25,000 cycles a batch with two waves each: a fragment takes five texture
+// reads and 400 instructions, and the pieces fill 2.3 of their 4 pixels.  Before
+// (each lane its chunk's pieces, one after the other, and a piece's pixels one
+// after the other) and after, a layer over a 960x540 scene: blended 57 -> 30
+// us, discarding 35 -> 17.  Unrolled over the chunk (KCW) the texture reads of
+// its pixels overlap: 34 -> 30 and 21 -> 17; other widths walk it.
+template <int PROG, bool DEBUG, int KCW>
 __global__ void __launch_bounds__(512) k_raster_imm(const PsSpan* __restrict__ spans, const PsSeg* __restrict__ segs,
                          const PsTri* __restrict__ tris, const PsDraw* __restrict__ draws, PsFrame f, int64_t n_tiles,
                          PsCounters* cnt, const float* __restrict__ vary, int nvs, const float* __restrict__ ck)
 {
     typedef PsProc<PROG> P;
+    constexpr int NV = P::NV;
+    constexpr bool COLOUR = PROG == PSGPU_PROC_CLOUD;   // the other one only discards
     extern __shared__ uint32_t lds[];
     if (ps_poisoned(cnt)) return;
     ps_commit_pending(cnt);
-    const int CW = f.chunk_w;
+    const int CW = KCW ? KCW : f.chunk_w;
     int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int waves = blockDim.x >> 6;
     int64_t tile = ps_xcd_remap<4>(blockIdx.x, gridDim.x) * (int64_t)waves + wave;   // neighbouring tiles share an L2
     if (tile >= n_tiles) return;
-    uint32_t* wl = lds + (size_t)wave * RA_WORDS(CW);
-    float* dep = (float*)wl;
-    int* win = (int*)(dep + CW * 64);
-    uint32_t* r_s = (uint32_t*)(win + CW * 64);   // segment index
-    uint32_t* r_fl = r_s + RA_CHUNK;               // behaviour | writes colour (PsSeg.si high bits)
-    uint32_t* r_x = r_fl + RA_CHUNK;               // xa | xb << 16
-    float* r_cf2 = (float*)(r_x + RA_CHUNK);
-    float* r_pz = r_cf2 + RA_CHUNK;
-    float* r_cst = r_pz + RA_CHUNK;
-    float* r_pst = r_cst + RA_CHUNK;
-    uint32_t* lcnt = (uint32_t*)(r_pst + RA_CHUNK);
-    uint32_t* loff = lcnt + 64;
+    uint2* lruns = (uint2*)(lds + (size_t)wave * RA_PIX_WORDS(CW));
+    uint32_t* starts = (uint32_t*)(lruns + PS_LDS_RUNS);
+    uint2* spare = (uint2*)(starts + 64) + lane;
+    uint2* pix = (uint2*)(starts + 64) + 64;   // x: depth bits, y: colour
 
     const int cw_shift = __builtin_ctz((unsigned)CW), tc_shift = __builtin_ctz((unsigned)f.tile_cols);
     const PsView& V = f.views[ps_view_of_tile(f, tile)];
@@ -2099,215 +2080,256 @@ __global__ void __launch_bounds__(512) k_raster_imm(const PsSpan* __restrict__ s
     // a view has fewer than 2^31 tiles; tile_cols is a power of two
     const uint32_t lt32 = (uint32_t)ltile, ntx = (uint32_t)V.n_tiles_x;
     int ty = (int)(lt32 / ntx), tx = (int)(lt32 - (uint32_t)ty * ntx);
-    int ry = lane >> tc_shift, rx = lane & (f.tile_cols - 1);
-    int y = ty * f.tile_rows + ry;
-    int cx = tx * f.tile_cols + rx;
-    int X0 = cx * CW;
+    int y = ty * f.tile_rows + (lane >> tc_shift);
+    int X0 = (tx * f.tile_cols + (lane & (f.tile_cols - 1))) * CW;
     const int VW = V.W;
-    bool inside = y < V.H && X0 < VW;
-    int ncol = inside ? min(CW, VW - X0) : 0;
+    const int ncol = y < V.H && X0 < VW ? min(CW, VW - X0) : 0;
     float* drow = V.depth + (int64_t)y * V.depth_scan;
+    uint32_t* crow = V.colour + (V.colour_top_down ? (int64_t)(V.colour_h - 1 - y) : (int64_t)y) * V.colour_scan;
     // a clear fused into the flush: the tile starts from its value, and the
     // whole tile is written back
     const bool dclear = V.dclear != 0;
-    for (int c = 0; c < ncol; c++) {
-        dep[c * 64 + lane] = dclear ? V.dclear_value : drow[X0 + c];
-        win[c * 64 + lane] = -1;
-    }
-    unsigned long long passes = 0;
-    bool dirty = dclear;
-    const uint64_t lt = ps_lt_mask();
     // the tile's runs in submission order, up to 64 at a time (one per lane)
     const unsigned long long ta = PS_TS(f.tstart[tile]), tb = PS_TS(f.tstart[tile + 1]);
     const uint32_t n_list = (uint32_t)tb - (uint32_t)ta;
     const uint32_t r0 = (uint32_t)(ta >> 32), nr = (uint32_t)(tb >> 32) - r0;
+    if (nr == 0 && !dclear) return;
     const uint32_t* rl = f.runs + 2 * (size_t)r0;
-    if (nr > 64) rl = ps_order_runs(f.runs + 2 * (size_t)r0, f.runs2 + 2 * (size_t)r0, nr, lcnt);
+    const bool in_lds = nr > 64 && nr <= PS_LDS_RUNS;
+    if (in_lds) ps_sort_runs_lds(rl, nr, lruns);
+    else if (nr > 64) rl = ps_order_runs(f.runs + 2 * (size_t)r0, f.runs2 + 2 * (size_t)r0, nr, (uint32_t*)lruns);
+    // the chunk as the flush finds it, to write back what it changes
+    uint32_t d0[KCW > 0 ? KCW : 1], c0[KCW > 0 ? KCW : 1];
+    if constexpr (KCW > 0) {
+        ps_load_run<KCW>((const uint32_t*)drow + X0, ncol, d0);
+#pragma unroll
+        for (int k = 0; k < KCW; k++) c0[k] = 0;
+        if (COLOUR) ps_load_run<KCW>(crow + X0, ncol, c0);
+#pragma unroll
+        for (int k = 0; k < KCW; k++) pix[k * 64 + lane] = make_uint2(dclear ? __float_as_uint(V.dclear_value) : d0[k], c0[k]);
+    } else {
+        for (int k = 0; k < ncol; k++)
+            pix[k * 64 + lane] = make_uint2(__float_as_uint(dclear ? V.dclear_value : drow[X0 + k]), COLOUR ? crow[X0 + k] : 0u);
+    }
+    uint32_t passes = 0;   // the lane's; a list has at most 2^31 pieces of 64 pixels
+    ps_lds_turn();
     for (uint32_t w0 = 0; w0 < nr; w0 += 64) {
+        // the window's runs, one per lane: list position of the first piece
+        // (0xffffffff past the last run), and what to add to a list position
+        // in the run to get its piece
         uint32_t rbase, rv, vhi;
-        int np;
-        ps_run_window(rl, nr, w0, n_list, rbase, rv, vhi, np);
-        const uint32_t vlo = __builtin_amdgcn_readlane(rv, 0);
-        // software pipeline over chunks of the window: while chunk i is split
-        // and walked, the records of chunk i+1 are in flight
-        uint32_t vn[RA_PER];
-        uint4 ran[RA_PER], rbn[RA_PER];
-#pragma unroll
-        for (int k = 0; k < RA_PER; k++) {
-            uint32_t e = vlo + k * 64 + lane;
-            uint32_t pp = ps_run_piece(rv, rbase, e, np);
-            vn[k] = e < vhi ? pp : 0u;
-            const uint4* p = (const uint4*)(segs + vn[k]);
-            ran[k] = e < vhi ? p[0] : make_uint4(0, 0, 0, 0);
-            rbn[k] = e < vhi ? p[1] : make_uint4(0, 0, 0, 0);
+        if (in_lds) {
+            const uint32_t j = w0 + lane;
+            const uint2 r = j < nr ? lruns[j] : make_uint2(0u, 0xffffffffu);
+            rbase = r.x;
+            rv = r.y;
+            vhi = w0 + 64 < nr ? lruns[w0 + 64].y : n_list;
+        } else {
+            ps_run_window(rl, nr, w0, n_list, rbase, rv, vhi);
         }
-        for (uint32_t cb = vlo; cb < vhi; cb += RA_CHUNK) {
-            uint32_t ce = min(vhi, cb + RA_CHUNK);
-            uint32_t v[RA_PER], key[RA_PER];
-            uint4 ra[RA_PER], rb[RA_PER];
+        const uint32_t vlo = (uint32_t)__builtin_amdgcn_readlane((int)rv, 0), delta = rbase - rv;
+        uint32_t run = 0;   // one more than the run of the last position before the batch
+        for (uint32_t cb = vlo; cb < vhi; cb += 64) {
+            // the batch's pieces, as k_raster gathers them
+            starts[lane] = 0;
+            ps_lds_turn();
+            if (rv - cb < 64u) starts[rv - cb] = (uint32_t)lane + 1u;
+            ps_lds_turn();
+            const uint32_t m = max(ps_wave_incl_max(starts[lane]), run);
+            ps_lds_turn();
+            run = (uint32_t)__builtin_amdgcn_readlane((int)m, 63);
+            const uint32_t e = cb + lane;
+            const bool valid = e < vhi;
+            const uint32_t pp = e + (uint32_t)__builtin_amdgcn_ds_bpermute((int)(m - 1u) * 4, (int)delta);
+            uint4 ra = make_uint4(0, 0, 0, 0), rb = make_uint4(0, 0, 0, 0);
+            float vs[NV > 0 ? NV : 1], vt[NV > 0 ? NV : 1];
 #pragma unroll
-            for (int k = 0; k < RA_PER; k++) {
-                v[k] = vn[k];
-                ra[k] = ran[k];
-                rb[k] = rbn[k];
-            }
-            if (cb + RA_CHUNK < vhi) {
+            for (int i = 0; i < NV; i++) vs[i] = vt[i] = 0.0f;
+            int di = 0, tri = 0;
+            if (valid) {
+                const uint4* p = (const uint4*)(segs + pp);
+                ra = p[0];
+                rb = p[1];
+                // the span's varyings at the piece's first pixel: from its
+                // checkpoint or by the serial walk from x1 (interp.cpp:82-92),
+                // as the deferred shading does
+                const PsSpan sp = spans[ra.x & PS_SEG_SPAN_MASK];
+                tri = sp.tri;
+                const PsTri tr = tris[tri];
+                di = (int)(tr.code >> 8);
+                const int py = (int)rb.z, xa = (int)(ra.y & 0xffffu);
+                PsEdge Le, Re;
+                ps_row_edges(tr, py, Le, Re);
+                int left = ps_cvt_i32(ps_edge_eval(Le, (float)py) + 0.5f);
+                int right = ps_cvt_i32(ps_edge_eval(Re, (float)py) + 0.5f);
+                PsSpanGeom g;
+                ps_span_geom(tr, py, left, right, Le, Re, g);
+                const float* u0 = vary + (int64_t)tr.vary * 3 * nvs;
+                ps_span_varyings<NV>(g, u0, u0 + nvs, u0 + 2 * nvs, vs, vt);
+                int xs = sp.x1;
+                if (xa > sp.x1 && ps_span_has_ck(sp) && ((ra.x >> 28) & 1)) {
+                    const float* cp = ck + (int64_t)pp * f.ck_stride;
 #pragma unroll
-                for (int k = 0; k < RA_PER; k++) {
-                    uint32_t e = cb + RA_CHUNK + k * 64 + lane;
-                    uint32_t pp = ps_run_piece(rv, rbase, e, np);
-                    vn[k] = e < vhi ? pp : 0u;
-                    const uint4* p = (const uint4*)(segs + vn[k]);
-                    ran[k] = e < vhi ? p[0] : make_uint4(0, 0, 0, 0);
-                    rbn[k] = e < vhi ? p[1] : make_uint4(0, 0, 0, 0);
+                    for (int i = 0; i < NV; i++) vs[i] = cp[i];
+                    xs = xa;
+                }
+                for (int xx = xs; xx < xa; xx++) {
+#pragma unroll
+                    for (int i = 0; i < NV; i++) vs[i] = vs[i] + vt[i];
                 }
             }
-#pragma unroll
-            for (int k = 0; k < RA_PER; k++) {
-                // the piece's lane: its row inside the tile and its chunk inside the row
-                int py = (int)rb[k].z, pcx = (int)(ra[k].y & 0xffffu) >> cw_shift;
-                key[k] = (uint32_t)(((py & (f.tile_rows - 1)) << tc_shift) | (pcx & (f.tile_cols - 1)));
+            // the piece's chunk in the tile and its pixels [a, b] of it
+            const int xa = (int)(ra.y & 0xffffu), pcx = xa >> cw_shift;
+            const int key = (((int)rb.z & (f.tile_rows - 1)) << tc_shift) | (pcx & (f.tile_cols - 1));
+            const int a = xa - (pcx << cw_shift), b = valid ? (int)(ra.y >> 16) - (pcx << cw_shift) : -1;
+            const bool test = (ra.x >> 26) & PSGPU_TEST_DEPTH, upd = (ra.x >> 26) & PSGPU_UPDATE_DEPTH, wc = (ra.x >> 28) & 1;
+            float cf2 = __uint_as_float(ra.z), pz = __uint_as_float(ra.w);
+            const float cst = __uint_as_float(rb.x), pst = __uint_as_float(rb.y);
+            const PsDraw& d = draws[di];
+            const bool blend = COLOUR && (d.behavior & PSGPU_ALPHABLEND) != 0;
+            uint32_t th = 0;
+            int tid = 0;
+            if (DEBUG && valid) {
+                tid = (int)(d.id_base + (tri - d.tri_start));
+                uint32_t h = (uint32_t)tid;
+                h ^= h >> 16; h *= 0x85ebca6bu; h ^= h >> 13; h *= 0xc2b2ae35u; h ^= h >> 16;
+                th = h;
             }
-            // stable split by lane key: each entry's rank among the equal keys
-            // before it (the same-key lanes of its group of 64 by ballots, plus
-            // the count of earlier groups), then per-key offsets, then placement
-            lcnt[lane] = 0;
-            __builtin_amdgcn_wave_barrier();
-            uint32_t rank[RA_PER];
+            // lanes of the same chunk
+            uint64_t same = ~0ull;
 #pragma unroll
-            for (int k = 0; k < RA_PER; k++) {
-                uint32_t e = cb + k * 64 + lane;
-                bool valid = e < ce;
-                uint32_t kk = key[k];
-                uint64_t same = __ballot(valid);
+            for (int bit = 0; bit < 6; bit++) {
+                const uint64_t bm = __ballot((key >> bit) & 1);
+                same &= ((key >> bit) & 1) ? bm : ~bm;
+            }
+            const bool all_test = __all(test || !valid);
+            // candidates before this lane at the same pixel
+            auto rank_of = [&](bool cand) {
+                const uint64_t cm = same & __ballot(cand);
+                return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(cm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)cm, 0));
+            };
+            // the lane's depth at pixel k, interpolateNextStep (interp.cpp:82-92)
+            auto depth_at = [&](bool in, float& r) {
+                r = 1.0f / cf2;
+                const float z = pz * r;
+                cf2 = in ? cf2 + cst : cf2;
+                pz = in ? pz + pst : pz;
+                return z;
+            };
+            auto can_pass = [&](bool in, float z, uint2 cur) {
+                return in & (-1.0f < z) & (!all_test | (z - __uint_as_float(cur.x) < -0.0001f));
+            };
+            // the programme at the lane's pixel, and the step to the next.
+            // Texture reads clamp their coordinates, so lanes without a
+            // fragment run along.
+            auto shade = [&](bool in, float r, uint32_t& col) {
+                float v[NV > 0 ? NV : 1];
 #pragma unroll
-                for (int bit = 0; bit < 6; bit++) {
-                    uint64_t m = __ballot((kk >> bit) & 1u);
-                    same &= ((kk >> bit) & 1u) ? m : ~m;
+                for (int i = 0; i < NV; i++) {
+                    v[i] = vs[i] * r;
+                    vs[i] = in ? vs[i] + vt[i] : vs[i];
                 }
-                uint32_t before = (uint32_t)__popcll(same & lt);
-                uint32_t cur = lcnt[kk];
-                rank[k] = cur + before;
-                __builtin_amdgcn_wave_barrier();
-                if (valid && before == 0) lcnt[kk] = cur + (uint32_t)__popcll(same);
-                __builtin_amdgcn_wave_barrier();
-            }
-            {
-                uint32_t cntv = lcnt[lane];
-                uint32_t x = cntv;
-#pragma unroll
-                for (int o = 1; o < 64; o <<= 1) {
-                    uint32_t yv = __shfl_up(x, o, 64);
-                    if (lane >= o) x += yv;
+                col = 0;
+                return P::fpi(d, v, col);
+            };
+            auto drawn = [&](int k) {   // every rasterised fragment, passing or not
+                const int64_t at = (int64_t)(int)rb.z * VW + ((pcx << cw_shift) + k);
+                atomicAdd(&f.dbg_rcount[at], 1);
+                atomicXor(&f.dbg_rhash[at], th);
+            };
+            // fragthrd.cpp:216-237 against the pixel as the rounds before left
+            // it; the FP runs on a pass, and a discarded fragment leaves depth
+            // as it was (fragthrd.cpp:227-236)
+            auto fragment = [&](bool turn, int k, float z, int fr, uint32_t col, uint2 cur) {
+                const float dd = test ? __uint_as_float(cur.x) : 1.0f;
+                const bool pass = turn & (z - dd < -0.0001f);
+                const bool depth = pass & upd & (fr != 2), paint = COLOUR & pass & wc & (fr == 1);
+                if (depth) cur.x = __float_as_uint(z);
+                if (paint) cur.y = blend ? ps_blend4(cur.y, col) : col;   // FBOBridge::write4 (fragthrd.cpp:70-82)
+                *(depth | paint ? pix + k * 64 + key : spare) = cur;
+                passes += pass ? 1u : 0u;
+                if (DEBUG && pass) {
+                    const int64_t at = (int64_t)(int)rb.z * VW + ((pcx << cw_shift) + k);
+                    atomicAdd(&f.dbg_pcount[at], 1);
+                    atomicXor(&f.dbg_phash[at], th);
+                    f.dbg_last[at] = tid;
                 }
-                loff[lane] = x - cntv;
-                __builtin_amdgcn_wave_barrier();
-            }
+            };
+            if constexpr (KCW > 0) {
+                float z[KCW], r[KCW];
+                uint2 cur[KCW];
+                bool cand[KCW], some = false;
+                int rank[KCW], fr[KCW], last = 0;
+                uint32_t col[KCW];
 #pragma unroll
-            for (int k = 0; k < RA_PER; k++) {
-                uint32_t e = cb + k * 64 + lane;
-                if (e < ce) {
-                    uint32_t q = loff[key[k]] + rank[k];
-                    r_s[q] = v[k];
-                    r_fl[q] = ra[k].x & ~PS_SEG_SPAN_MASK;
-                    r_x[q] = ra[k].y;
-                    r_cf2[q] = __uint_as_float(ra[k].z);
-                    r_pz[q] = __uint_as_float(ra[k].w);
-                    r_cst[q] = __uint_as_float(rb[k].x);
-                    r_pst[q] = __uint_as_float(rb[k].y);
+                for (int k = 0; k < KCW; k++) cur[k] = pix[k * 64 + key];
+#pragma unroll
+                for (int k = 0; k < KCW; k++) {
+                    const bool in = (k >= a) & (k <= b);
+                    z[k] = depth_at(in, r[k]);
+                    if (DEBUG && in) drawn(k);
+                    cand[k] = can_pass(in, z[k], cur[k]);
+                    some |= cand[k];
                 }
-            }
-            __builtin_amdgcn_wave_barrier();
-            if (inside) {
-                uint32_t l0 = loff[lane], l1 = l0 + lcnt[lane];
-                for (uint32_t q = l0; q < l1; q++) {
-                    int sidx = (int)r_s[q];
-                    uint32_t fl = r_fl[q];
-                    int beh = (fl >> 26) & 3;
-                    bool wc = (fl >> 28) & 1;
-                    uint32_t xab = r_x[q];
-                    int a = (int)(xab & 0xffffu), b = (int)(xab >> 16);
-                    float cf2 = r_cf2[q], pz = r_pz[q];
-                    const float cst = r_cst[q], pst = r_pst[q];
-                    uint32_t th = 0;
-                    int tid = 0;
-                    if (DEBUG) {
-                        int si = (int)(segs[sidx].si & PS_SEG_SPAN_MASK);
-                        int tri = spans[si].tri;
-                        const PsTri tr = tris[tri];
-                        const PsDraw& d = draws[tr.code >> 8];
-                        tid = (int)(d.id_base + (tri - d.tri_start));
-                        uint32_t h = (uint32_t)tid;
-                        h ^= h >> 16; h *= 0x85ebca6bu; h ^= h >> 13; h *= 0xc2b2ae35u; h ^= h >> 16;
-                        th = h;
+                if (!__any(some)) continue;
+#pragma unroll
+                for (int k = 0; k < KCW; k++) fr[k] = shade((k >= a) & (k <= b), r[k], col[k]);
+#pragma unroll
+                for (int k = 0; k < KCW; k++) {
+                    rank[k] = rank_of(cand[k]);
+                    last = cand[k] ? max(last, rank[k]) : last;
+                }
+                for (int q = 0;;) {
+#pragma unroll
+                    for (int k = 0; k < KCW; k++) fragment(cand[k] & (rank[k] == q), k, z[k], fr[k], col[k], cur[k]);
+                    if (DEBUG) __threadfence();   // the last pass of a pixel is stored last
+                    ps_lds_turn();
+                    q++;
+                    if (!__any(last >= q)) break;
+#pragma unroll
+                    for (int k = 0; k < KCW; k++) cur[k] = pix[k * 64 + key];
+                }
+            } else {
+                for (int k = 0; k < CW; k++) {
+                    const bool in = k >= a && k <= b;
+                    if (!__any(in)) continue;
+                    float r;
+                    uint32_t col;
+                    const float z = depth_at(in, r);
+                    if (DEBUG && in) drawn(k);
+                    const bool cand = can_pass(in, z, pix[k * 64 + key]);
+                    const int fr = shade(in, r, col);
+                    const int rank = rank_of(cand);
+                    for (int q = 0; __any(cand && rank >= q); q++) {
+                        fragment(cand && rank == q, k, z, fr, col, pix[k * 64 + key]);
+                        if (DEBUG) __threadfence();
+                        ps_lds_turn();
                     }
-                    // the span's varyings at pixel a: from the piece's checkpoint or
-                    // by the serial walk from x1 (interp.cpp:82-92), as the deferred
-                    // shading does
-                    const int si = (int)(segs[sidx].si & PS_SEG_SPAN_MASK);
-                    const PsSpan sp = spans[si];
-                    const PsTri tr = tris[sp.tri];
-                    const PsDraw& d = draws[tr.code >> 8];
-                    float vs[P::NV > 0 ? P::NV : 1], vt[P::NV > 0 ? P::NV : 1];
-                    {
-                        PsEdge Le, Re;
-                        ps_row_edges(tr, y, Le, Re);
-                        int left = ps_cvt_i32(ps_edge_eval(Le, (float)y) + 0.5f);
-                        int right = ps_cvt_i32(ps_edge_eval(Re, (float)y) + 0.5f);
-                        PsSpanGeom g;
-                        ps_span_geom(tr, y, left, right, Le, Re, g);
-                        const float* u0 = vary + (int64_t)tr.vary * 3 * nvs;
-                        ps_span_varyings<P::NV>(g, u0, u0 + nvs, u0 + 2 * nvs, vs, vt);
-                        int xs = sp.x1;
-                        if (a > sp.x1 && ps_span_has_ck(sp) && wc) {
-                            const float* cp = ck + (int64_t)sidx * f.ck_stride;
-#pragma unroll
-                            for (int i = 0; i < P::NV; i++) vs[i] = cp[i];
-                            xs = a;
-                        }
-                        for (int xx = xs; xx < a; xx++) {
-#pragma unroll
-                            for (int i = 0; i < P::NV; i++) vs[i] = vs[i] + vt[i];
-                        }
-                    }
-                    const bool blend = (d.behavior & PSGPU_ALPHABLEND) != 0;
-                    const int64_t crow = (V.colour_top_down ? (int64_t)(V.colour_h - 1 - y) : (int64_t)y) * V.colour_scan;
-                    for (int x = a; x <= b; x++) {
-                        // interpolateNextStep (interp.cpp:82-92)
-                        float r = 1.0f / cf2;
-                        cf2 += cst;
-                        float z = pz * r;
-                        pz += pst;
-                        int c = x - X0;
-                        float cur = (beh & PSGPU_TEST_DEPTH) ? dep[c * 64 + lane] : 1.0f;
-                        int64_t pix = (int64_t)y * VW + x;
-                        if (DEBUG) { f.dbg_rcount[pix] += 1; f.dbg_rhash[pix] ^= th; }
-                        // fragthrd.cpp:227-236: the FP runs on a pass; a discarded
-                        // fragment leaves depth as it was
-                        if (-1.0f < z && (z - cur < -0.0001f)) {
-                            passes++;
-                            float in[P::NV > 0 ? P::NV : 1];
-#pragma unroll
-                            for (int i = 0; i < P::NV; i++) in[i] = vs[i] * r;
-                            uint32_t col = 0;
-                            int fr = P::fpi(d, in, col);
-                            if (fr != 2 && (beh & PSGPU_UPDATE_DEPTH)) { dep[c * 64 + lane] = z; dirty = true; }
-                            if (fr == 1 && wc) {   // FBOBridge::write4 (fragthrd.cpp:70-82)
-                                uint32_t* cp = V.colour + crow + x;
-                                *cp = blend ? ps_blend4(*cp, col) : col;
-                            }
-                            if (DEBUG) { f.dbg_pcount[pix] += 1; f.dbg_phash[pix] ^= th; f.dbg_last[pix] = tid; }
-                        }
-#pragma unroll
-                        for (int i = 0; i < P::NV; i++) vs[i] = vs[i] + vt[i];
-                    }
                 }
             }
-            __builtin_amdgcn_wave_barrier();
         }
     }
-    for (int c = 0; c < ncol; c++)
-        if (dirty) drow[X0 + c] = dep[c * 64 + lane];
+    // the colours that changed, then the depths of chunks in which one did
+    bool dirty = dclear;
+    if constexpr (KCW > 0) {
+        uint32_t dv[KCW];
+#pragma unroll
+        for (int k = 0; k < KCW; k++) {
+            const uint2 q = pix[k * 64 + lane];
+            dv[k] = q.x;
+            dirty |= k < ncol && q.x != d0[k];
+            if (COLOUR && k < ncol && q.y != c0[k]) crow[X0 + k] = q.y;
+        }
+        if (dirty) ps_store_run<KCW>((uint32_t*)drow + X0, ncol, dv);
+    } else {
+        for (int k = 0; k < ncol; k++) {
+            const uint2 q = pix[k * 64 + lane];
+            dirty |= q.x != __float_as_uint(drow[X0 + k]);
+            if (COLOUR && q.y != crow[X0 + k]) crow[X0 + k] = q.y;
+        }
+        if (dirty)
+            for (int k = 0; k < ncol; k++) drow[X0 + k] = __uint_as_float(pix[k * 64 + lane].x);
+    }
     ps_wave_add64(cnt, PS_ST_SHADED, passes);
 }
 
@@ -2647,7 +2669,13 @@ void psk_segments(hipStream_t s, const PsSpan* spans, const uint32_t* row_off, i
 #undef SG_LAUNCH
 }
 
-size_t psk_raster_lds(int chunk_w, int waves) { return (size_t)waves * RA_WORDS(chunk_w) * 4; }
+// the tilings taken and refused go by 1,024 words a wave beside the pixels,
+// which the kernels stay below
+size_t psk_raster_lds(int chunk_w, int waves)
+{
+    static_assert(RA_PIX_WORDS(0) <= 1024, "a tiling that is taken fits");
+    return (size_t)waves * (chunk_w * 64 * 2 + 1024) * 4;
+}
 
 void psk_raster(hipStream_t s, bool debug, const PsSpan* spans, const PsSeg* segs, const PsTri* tris, const PsDraw* draws,
                 const PsFrame& f, int waves_per_group, PsCounters* cnt)
@@ -2673,22 +2701,22 @@ void psk_raster_imm(hipStream_t s, int prog, bool debug, const PsSpan* spans, co
                     const float* ck)
 {
     int64_t n_tiles = f.n_tiles;
-    size_t lds = psk_raster_lds(f.chunk_w, waves_per_group);
+    size_t lds = (size_t)waves_per_group * RA_PIX_WORDS(f.chunk_w) * 4;
     dim3 g(gsz(n_tiles, waves_per_group)), b(64 * waves_per_group);
-#define RI_CASE(K)                                                                                                   \
-    case K:                                                                                                          \
-        if (debug)                                                                                                   \
-            hipLaunchKernelGGL((k_raster_imm<K, true>), g, b, lds, s, spans, segs, tris, draws, f, n_tiles, cnt,     \
-                               vary, nvs, ck);                                                                       \
-        else                                                                                                         \
-            hipLaunchKernelGGL((k_raster_imm<K, false>), g, b, lds, s, spans, segs, tris, draws, f, n_tiles, cnt,    \
-                               vary, nvs, ck);                                                                       \
+#define RI_LAUNCH(P, D, K)                                                                                           \
+    hipLaunchKernelGGL((k_raster_imm<P, D, K>), g, b, lds, s, spans, segs, tris, draws, f, n_tiles, cnt, vary, nvs, ck)
+#define RI_CASE(P)                                                                                                   \
+    case P:                                                                                                          \
+        if (debug) RI_LAUNCH(P, true, 0);                                                                            \
+        else if (f.chunk_w == 4) RI_LAUNCH(P, false, 4);                                                             \
+        else RI_LAUNCH(P, false, 0);                                                                                 \
         break;
     switch (prog) {
     RI_CASE(PSGPU_PROC_CLOUD) RI_CASE(PSGPU_PROC_CLOUD_SHADOW)
     default: break;
     }
 #undef RI_CASE
+#undef RI_LAUNCH
 }
 
 void psk_shade(hipStream_t s, int prog, const PsSpan* spans, const PsSeg* segs, const float* ck, const PsTri* tris,

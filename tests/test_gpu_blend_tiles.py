@@ -1,0 +1,67 @@
+"""Programmes shaded in the raster walk on crowded tiles: viewports of one to
+a few tiles under hundreds of overlapping triangles, blended, opaque and
+discarded, whose draws test and update depth in every combination, in tiles of
+every chunk width.  Bit-exact against the oracle."""
+import numpy as np
+import pytest
+
+from conftest import announce
+import scenegen
+from test_gpu_parity import assert_same, gpu_render
+
+pytestmark = pytest.mark.gpu
+
+N = pytest.importorskip("puresoft3d_amd.native")
+from puresoft3d_amd import scenes as S  # noqa: E402
+
+
+def crowded_layers(prog, n, width, height, seed, mixed):
+    """a Blinn-Phong ground, then n triangles a draw of prog, blended where it
+    may; mixed: four draws, one of each combination of depth test and update,
+    the blended ones between opaque ones"""
+    sc = scenegen.micro_scene(N.PROC_BLINN, seed, width, height, n=12)
+    rng = np.random.default_rng(seed)
+    scenegen.add_depth_map(sc, rng, 32, 15, 16)
+    sc.name = "layers_p%d_%d_%dx%d_s%d_%d" % (prog, n, width, height, seed, mixed)
+    sc.draws = [S.DrawSpec("m", N.PROC_BLINN)]
+    full = N.UPDATE_DEPTH | N.TEST_DEPTH
+    order = [full, N.TEST_DEPTH, N.UPDATE_DEPTH, full] if mixed else [full]
+    for k, beh in enumerate(order):
+        pos = np.concatenate([scenegen.random_clip_triangles(rng, n - n // 3, kind=0),
+                              scenegen.random_clip_triangles(rng, n // 3, kind=1)], 0).reshape(-1, 3, 4)
+        pos = pos[rng.permutation(n)].reshape(-1, 4)
+        sc.meshes["l%d" % k] = scenegen._slots_for(prog, pos, rng)
+        blend = N.ALPHABLEND if prog == N.PROC_CLOUD and k % 2 == 0 else 0
+        sc.draws.append(S.DrawSpec("l%d" % k, prog, behavior=beh | blend))
+    return sc
+
+
+def assert_both(sc, oracle, tiling=None):
+    """with the debug planes, whose kernels are their own, and without"""
+    assert_same(sc, oracle, tiling=tiling)
+    col, dep, _, st = gpu_render(sc, tiling, debug=False)
+    f, ost = oracle.render_scene(sc)
+    np.testing.assert_array_equal(dep.view(np.uint32), f.depth.view(np.uint32))
+    np.testing.assert_array_equal(col, f.colour)
+    assert st["frags_shaded"] == ost.frags_shaded
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("n", [12, 40, 700, 3000])
+@pytest.mark.parametrize("prog", [N.PROC_CLOUD, N.PROC_CLOUD_SHADOW])
+def test_crowded_layers(oracle, prog, n, mixed):
+    assert_both(crowded_layers(prog, n, 31, 8, n, mixed), oracle)
+
+
+@pytest.mark.parametrize("tiling", [(1, 8, 8), (2, 16, 1), (4, 8, 2), (8, 8, 8), (8, 64, 3), (16, 4, 5), (32, 2, 3), (64, 1, 1)])
+@pytest.mark.parametrize("prog", [N.PROC_CLOUD, N.PROC_CLOUD_SHADOW])
+def test_layer_tilings(oracle, prog, tiling):
+    announce("layers %d %s" % (prog, tiling))
+    assert_both(crowded_layers(prog, 300, 131, 35, 9, True), oracle, tiling=tiling)
+
+
+def test_layer_without_pieces_keeps_the_ground(oracle):
+    """every triangle of the layer lies behind the ground or off screen"""
+    sc = crowded_layers(N.PROC_CLOUD, 40, 131, 35, 3, False)
+    sc.meshes["l0"][0][:, 0] += 50.0
+    assert_both(sc, oracle)

@@ -309,7 +309,9 @@ int psgpu_sync_noalloc(psgpu_ctx* ctx);
  *      5:(int)(unsigned)x86(a), 6:log2 approximation of the trilinear LOD, 7:a (a plain copy kernel,
  *      the calibration point for HBM traffic counters), 8 and 9: the wrapped texel coordinates of v and
  *      v + 1 modulo m (v, m and the result are int32 bit patterns in the float arrays a, b, out),
- *      10: one lane of FP_Cloud's cvtps2dq/packusdw/packuswb tail (testproc.cpp:562-568) as a float} ---- */
+ *      10: one lane of FP_Cloud's cvtps2dq/packusdw/packuswb tail (testproc.cpp:562-568) as a float,
+ *      11: 1 / sqrt(a), each rounded, 12 and 13: the texels of the whole coordinates a and a + 1 in a row
+ *      whose last texel is b (int32 bits, the sign bit asking for wrap; the result is int32 bits)} ---- */
 int psgpu_selftest_math(psgpu_ctx* ctx, int op, const float* a, const float* b, float* out, int n);
 
 #ifdef __cplusplus

@@ -43,6 +43,25 @@ PS_DEV void ps_m4v4(float* r, const float* m, const float* v)
     }
 }
 
+// 1.0f / sqrtf(x), both correctly rounded, in 8 instructions and two tests where
+// x is far from the ends of the range (the two operations are 25): the
+// hardware's reciprocal root h is within an ulp, and one step each with the
+// exact residuals x - s s and 1 - s h (fused) rounds the root s and its
+// reciprocal as the two operations do (Markstein, IBM J. Res. Dev. 34, 1990),
+// but for an s whose bits are all ones: 1 / s lies next to the midpoint of two
+// floats.  That is the root of the last two floats below a power of four.
+// Every float has been compared.
+PS_DEV float ps_rsqrt(float x)
+{
+    if (x >= 0x1p-100f && x <= 0x1p+100f && (__float_as_uint(x) & 0x7ffffeu) != 0x7ffffeu) {
+        const float h = __builtin_amdgcn_rsqf(x);
+        float s = x * h;
+        s = __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * h, s);
+        return __builtin_fmaf(__builtin_fmaf(-s, h, 1.0f), h, h);
+    }
+    return 1.0f / sqrtf(x);
+}
+
 // dot_3_4, vector.cpp:85-112
 PS_DEV float ps_dot4(const float* a, const float* b)
 {
@@ -52,7 +71,7 @@ PS_DEV float ps_dot4(const float* a, const float* b)
 
 PS_DEV void ps_norm4(float* a)   // norm_3_4
 {
-    float r = 1.0f / sqrtf(ps_dot4(a, a));
+    float r = ps_rsqrt(ps_dot4(a, a));
     a[0] *= r; a[1] *= r; a[2] *= r; a[3] *= r;
 }
 
@@ -64,7 +83,7 @@ PS_DEV float ps_dot3(const float* a, const float* b)
 
 PS_DEV void ps_norm3(float* a)
 {
-    float r = 1.0f / sqrtf(ps_dot3(a, a));
+    float r = ps_rsqrt(ps_dot3(a, a));
     a[0] *= r; a[1] *= r; a[2] *= r;
 }
 
@@ -272,19 +291,17 @@ PS_DEV int ps_lvl_h(const PsTex& t, int l) { int h = t.height >> l; return h < 1
 // quotient comes from the 1-ulp hardware reciprocal: |v * rcp(m) - v/m| <
 // 2^21 * 1.5 * 2^-23 < 1, so the floored estimate is within one of the true
 // quotient and a single correction each way makes the remainder exact.
-// Larger |v| (and INT_MIN, the conversion of NaN) take the integer remainder.
+// A larger |v| (and INT_MIN, the conversion of NaN) is first brought within
+// 512 + 2 m of 0 by such an estimate, off by at most 2^31 * 2^-22 + 1.
 // Textures have at most 2^22 texels a side (psgpu_texture_create), so m and
 // |q| fit the 24-bit multiplier, whose low 32 bits equal the 32-bit product.
 PS_DEV int ps_floor_mod(int v, int m, float rm)
 {
-    if ((unsigned)v + (1u << 21) < (2u << 21)) {
-        int q = (int)floorf((float)v * rm);
-        int r = v - __mul24(q, m);
-        r = r < 0 ? r + m : r;
-        return r >= m ? r - m : r;
-    }
-    int r = v % m;
-    return r < 0 ? r + m : r;
+    if ((unsigned)v + (1u << 21) >= (2u << 21)) v = (int)((unsigned)v - (unsigned)(int)floorf((float)v * rm) * (unsigned)m);
+    int q = (int)floorf((float)v * rm);
+    int r = v - __mul24(q, m);
+    r = r < 0 ? r + m : r;
+    return r >= m ? r - m : r;
 }
 
 PS_DEV float ps_rcp_approx(int m) { return __builtin_amdgcn_rcpf((float)m); }
@@ -408,6 +425,25 @@ PS_DEV void ps_clamp_pair(int wrap, int maxv, int v, int& a, int& b)
     else b = ps_floor_mod(v1, maxv, rm);
 }
 
+// The same of the coordinates x and x + 1 for a whole x, kept in floats where
+// they are exact: |x| < 2^21, and the remainder (fused, so rounded once) is a
+// whole number below 2^23.
+PS_DEV void ps_texel_pair(int wrap, int maxv, float x, int& a, int& b)
+{
+    if (!(fabsf(x) < 2097152.0f)) { ps_clamp_pair(wrap, maxv, ps_cvt_i32(x), a, b); return; }
+    const float m = (float)maxv;
+    if (!wrap) {
+        a = (int)__builtin_amdgcn_fmed3f(x, 0.0f, m);
+        b = (int)__builtin_amdgcn_fmed3f(x + 1.0f, 0.0f, m);
+        return;
+    }
+    float r = __builtin_fmaf(-floorf(x * __builtin_amdgcn_rcpf(m)), m, x);
+    r = r < 0.0f ? r + m : r;
+    r = r >= m ? r - m : r;
+    a = maxv > 0 ? (int)r : 0;
+    b = a + 1 >= maxv ? 0 : a + 1;
+}
+
 // bilinear filter: texel j covers u = j/W (the nearest sampler's rounding rule).
 // Rows and columns are addressed once each; the four texels share them.  The
 // built-in programmes use the B, G, R channels only (NCH = 3).
@@ -418,10 +454,9 @@ PS_DEV void ps_sample_bilinear(const PsTex& t, int level, float u, float v, floa
     float fx = (float)w * u, fy = (float)h * v;
     float x0 = floorf(fx), y0 = floorf(fy);
     float ax = fx - x0, ay = fy - y0;
-    int ix = ps_cvt_i32(x0), iy = ps_cvt_i32(y0);
     int r0, r1, c0, c1;
-    ps_clamp_pair(t.wrap, h - 1, iy, r0, r1);
-    ps_clamp_pair(t.wrap, w - 1, ix, c0, c1);
+    ps_texel_pair(t.wrap, h - 1, y0, r0, r1);
+    ps_texel_pair(t.wrap, w - 1, x0, c0, c1);
     int scan = level == 0 ? t.scanline : w * t.elem_len;
     // a layer stays below 4 GiB (psgpu_texture_create): 32-bit texel offsets
     const uint32_t lo = (uint32_t)t.level_off[level];
@@ -517,10 +552,9 @@ PS_DEV void ps_sample_bilinear_pair(const PsTex& t, const uint8_t* data1, int le
     float fx = (float)w * u, fy = (float)h * v;
     float x0 = floorf(fx), y0 = floorf(fy);
     float ax = fx - x0, ay = fy - y0;
-    int ix = ps_cvt_i32(x0), iy = ps_cvt_i32(y0);
     int r0, r1, c0, c1;
-    ps_clamp_pair(t.wrap, h - 1, iy, r0, r1);
-    ps_clamp_pair(t.wrap, w - 1, ix, c0, c1);
+    ps_texel_pair(t.wrap, h - 1, y0, r0, r1);
+    ps_texel_pair(t.wrap, w - 1, x0, c0, c1);
     int scan = level == 0 ? t.scanline : w * t.elem_len;
     // a layer stays below 4 GiB (psgpu_texture_create): 32-bit texel offsets
     const uint32_t lo = (uint32_t)t.level_off[level];

@@ -2433,6 +2433,12 @@ __global__ void __launch_bounds__(256, 6) k_shade(const PsSpan* __restrict__ spa
     // shadowed 1280x720 31.5 -> 27.9 (a loop over the wave's draws, one copy of
     // the code: 168, 50, 265, 38; waves of several draws on a list for a second
     // kernel: 168 + 20, 45 + 11, 270, 29 + 10).
+    // What bounds the kernel is instruction issue, 90% of its time: some 1,280
+    // per wave, a third of them the span's start and the walk to the pixel,
+    // which neighbours share.  A lane per run of neighbours that leaves each
+    // pixel its accumulators in LDS issues a quarter less, but its barriers
+    // cost more (182 us against 176).  With ps_rsqrt and ps_texel_pair 160 us,
+    // 44, 251, 28.0.
     uint32_t c;
     bool hit;
     if (__ballot(di != __builtin_amdgcn_readfirstlane(di)) == 0) {
@@ -2550,6 +2556,13 @@ __global__ void k_selftest(int op, const float* a, const float* b, float* out, i
         break;
     }
     case 10: r = (float)ps_sse_pack_byte(a[i]); break;
+    case 11: r = ps_rsqrt(a[i]); break;
+    case 12: case 13: {         // texel pair of a whole coordinate, m the last texel, wrapped where the sign bit of m is set
+        int m = __float_as_int(b[i]), c0, c1;
+        ps_texel_pair(m < 0, m & 0x7fffffff, a[i], c0, c1);
+        r = __int_as_float(op == 12 ? c0 : c1);
+        break;
+    }
     }
     out[i] = r;
 }

@@ -51,8 +51,7 @@ PS_DEV uint32_t ps_light_def(const PsDraw& d, float* oc, const float* wp, const 
     float L[4], E[4], H[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) L[k] = d.lightPos[k] - wp[k];
-    float dist = sqrtf(ps_dot4(L, L));
-    float rd = 1.0f / dist;
+    float rd = ps_rsqrt(ps_dot4(L, L));
 #pragma unroll
     for (int k = 0; k < 4; k++) L[k] *= rd;
 #pragma unroll
@@ -301,8 +300,7 @@ PS_DEV bool ps_blinn_fp(const PsDraw& d, const float* in, float r, const float* 
     float L[3], E[3], H[3];
 #pragma unroll
     for (int k = 0; k < 3; k++) L[k] = d.lightPos[k] - wp[k];
-    float dist = sqrtf(ps_dot3(L, L));
-    float rd = 1.0f / dist;
+    float rd = ps_rsqrt(ps_dot3(L, L));
 #pragma unroll
     for (int k = 0; k < 3; k++) L[k] *= rd;
 #pragma unroll
@@ -388,7 +386,7 @@ template <> struct PsProc<PSGPU_PROC_CLOUD> {
         float L[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) L[k] = d.lightPos[k] - in[4 + k];
-        float rd = 1.0f / sqrtf(ps_dot4(L, L));
+        float rd = ps_rsqrt(ps_dot4(L, L));
 #pragma unroll
         for (int k = 0; k < 4; k++) L[k] *= rd;
         float lambert = 2.0f * ps_dot4(L, in);

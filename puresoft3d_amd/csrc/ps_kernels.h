@@ -11,8 +11,8 @@ void psk_few_fills(hipStream_t s, const PsFewFills& fills, int n, int64_t max_pi
 // the log's overflow flag, sizes and statistics to the host, and all zero again
 // (after an overflow only with reset)
 void psk_finish(hipStream_t s, PsCounters* c, uint32_t* sizes, PsFinish* out, bool reset);
-// row_part (optional, flushes of one programme): each block of psk_setup_block()
-// triangles writes its row total there
+// prog: the flush's programme, 0 if it has several; each block of
+// psk_setup_block() triangles writes its row total to row_part
 int psk_setup_block();
 void psk_setup(hipStream_t s, int prog, bool share, const PsDraw* draws, int nd, int64_t T, PsTri* tris, float* vary, int nvs,
                float* grads, uint32_t* nrows, uint32_t* row_part, PsCounters* cnt, const PsView* views);
@@ -22,9 +22,6 @@ int psk_scan_blocks(int64_t cap);
 // bstart (bcap entries) the triangle of every 64th row item; empties the list `wide`
 void psk_scan_parts(hipStream_t s, const uint32_t* in, int64_t n, uint32_t* out, const uint32_t* parts, int pgran,
                     uint32_t* total_out, uint32_t* bstart, int64_t bcap, uint32_t* wide);
-// the same from the counts alone (block totals into partial first)
-void psk_scan_rows(hipStream_t s, const uint32_t* in, int64_t n, uint32_t* out, uint32_t* partial, uint32_t* total_out,
-                   uint32_t* bstart, int64_t bcap, uint32_t* wide);
 // exclusive scan of the per-tile counts (pieces | runs << 32) into tstart
 // (n + 1 entries); the piece total into *total_out, its running maximum at
 // total_out[2]
@@ -50,10 +47,11 @@ void psk_raster(hipStream_t s, bool debug, const PsSpan* spans, const PsSeg* seg
 void psk_raster_imm(hipStream_t s, int prog, bool debug, const PsSpan* spans, const PsSeg* segs, const PsTri* tris,
                     const PsDraw* draws, const PsFrame& f, int waves_per_group, PsCounters* cnt, const float* vary, int nvs,
                     const float* ck);
-// clears: this launch also writes the views' fused colour clears (one launch of a flush does)
+// prog: the programme of the flush's colour-writing draws, 0 if they have
+// several; also writes the views' fused colour clears
 void psk_shade(hipStream_t s, int prog, const PsSpan* spans, const PsSeg* segs, const float* ck, const PsTri* tris,
                const float* vary, int nvs, const float* grads, const PsDraw* draws, const PsFrame& f,
-               const PsCounters* cnt, bool clears);
+               const PsCounters* cnt);
 // up to six levels of the mip chains of `layers` layers, from a source level of
 // w x h texels: off[0] its offset in the layer, off[1 .. levels] those to write;
 // rows are tight

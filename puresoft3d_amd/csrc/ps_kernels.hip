@@ -25,6 +25,8 @@
 //            to the pixel, runs the FP twin and writes BGRA8.
 //  The depth test is order dependent, so per pixel the fragments are applied
 //  strictly in submission order; no atomics touch depth or colour.
+#include <type_traits>
+
 #include "ps_kernels.h"
 #include "ps_procs.h"
 
@@ -396,17 +398,24 @@ __device__ __forceinline__ int ps_find_draw_wave(const PsDraw* __restrict__ draw
     return d;
 }
 
-// row_part (flushes of one programme): the block's row total, for the scan
-// of the row counts.  At least three waves per SIMD: a 1080p frame's 200k
+// row_part: the block's row total, for the scan of the row counts.  At least three waves per SIMD: a 1080p frame's 200k
 // triangles make only about three per SIMD, and the bound of four left the
 // Blinn-Phong instantiation at 128 VGPRs with a 12-byte spill.
+// PROG 0: flushes of several programmes, each wave running through those of its
+// triangles (the programmes that shade in the raster walk have their own
+// flushes).  A launch a programme went over all triangles each time: four
+// programmes at 1366x768, 38 + 4 us for the row totals -> 14.7, shading
+// likewise 49 -> 25, the frame 77 -> 59.  A flush of one programme keeps its
+// own instantiation, whose code and registers are that programme's alone.
+#define PS_SETUP_PROGS(X)                                                                            \
+    X(PSGPU_PROC_DEF01) X(PSGPU_PROC_DEF02) X(PSGPU_PROC_DEF03) X(PSGPU_PROC_DEF04)                  \
+    X(PSGPU_PROC_DEF05) X(PSGPU_PROC_LAMBERT) X(PSGPU_PROC_BLINN) X(PSGPU_PROC_SHADOWED)
 template <int PROG, bool SHARE>
 __global__ void __launch_bounds__(128, 3) k_setup(const PsDraw* __restrict__ draws, int nd, int64_t T, PsTri* __restrict__ tris,
                                                float* __restrict__ vary, int nvs, float* __restrict__ grads,
                                                uint32_t* __restrict__ nrows, uint32_t* __restrict__ row_part,
                                                PsCounters* cnt, const PsView* __restrict__ views)
 {
-    typedef PsProc<PROG> P;
     extern __shared__ float su[];   // per wave: the varyings of its 64 triangles, 3*nvs floats each
     __shared__ uint32_t wrows[2];
     int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -417,15 +426,17 @@ __global__ void __launch_bounds__(128, 3) k_setup(const PsDraw* __restrict__ dra
     const int lane = threadIdx.x & 63, n3 = 3 * nvs;
     float* wl = su + (size_t)(threadIdx.x & ~63) * n3;
     bool stage = false;
-    ps_with_draw(draws, di, [&](const PsDraw& d) {
-    if (live && d.prog == PROG) {
+    auto triangle = [&](auto k, const PsDraw& d) {
+    constexpr int K = decltype(k)::value;
+    typedef PsProc<K> P;
+    if (live && d.prog == K) {
         const int W = views[d.view].W, H = views[d.view].H;
         int64_t lt = t - d.tri_start;
         float pos[3][4];
         float u[3][P::NV > 0 ? P::NV : 1];
         float rw[3], z[3];
         bool pieces = false;
-        const bool skip = SHARE && ps_shares_varyings(PROG) && d.vary_skip;
+        const bool skip = SHARE && ps_shares_varyings(K) && d.vary_skip;
 #pragma unroll
         for (int v = 0; v < 3; v++) {
             if (skip) ps_vp_pos(d, lt * 3 + v, pos[v], u[v], ps_grad_iu<P>());
@@ -498,7 +509,7 @@ __global__ void __launch_bounds__(128, 3) k_setup(const PsDraw* __restrict__ dra
                 tr.split = split;
                 tr.code = code | ((uint32_t)di << 8);
                 tr.view = d.view;
-                tr.vflags = (uint32_t)(d.behavior & 3) | (d.writes_colour ? 4u : 0u) | (uint32_t)PROG << 4;
+                tr.vflags = (uint32_t)(d.behavior & 3) | (d.writes_colour ? 4u : 0u) | (uint32_t)K << 4;
                 tr.vary = (int)t + d.vary_delta;
                 tr.pad = 0;
                 n = (uint32_t)(last - first + 1);
@@ -533,13 +544,21 @@ __global__ void __launch_bounds__(128, 3) k_setup(const PsDraw* __restrict__ dra
                 for (int k = 0; k < P::NV; k++) wl[lane * n3 + v * nvs + k] = u[v][k];
         }
     }
+    };
+    ps_with_draw(draws, di, [&](const PsDraw& d) {
+        if constexpr (PROG != 0) {
+            triangle(std::integral_constant<int, PROG>(), d);
+        } else {
+#define SU_ONE(K) triangle(std::integral_constant<int, K>(), d);
+            PS_SETUP_PROGS(SU_ONE)
+#undef SU_ONE
+        }
     });
     // varyings of the wave's staged triangles: the wave's slots are one
     // contiguous block of 64 * 3*nvs floats, stored 16 bytes per lane and
-    // instruction.  A float is written only when its triangle staged in this
-    // launch (the slots of other programmes' triangles belong to their own
-    // launches); floats past NV of a staged vertex receive what the LDS
-    // holds, and nothing reads them.
+    // instruction.  A float is written only when its triangle staged; floats
+    // past NV of a staged vertex receive what the LDS holds, and nothing reads
+    // them.
     const uint64_t m = __ballot(stage);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -2340,44 +2359,15 @@ __global__ void __launch_bounds__(512) k_raster_imm(const PsSpan* __restrict__ s
 // -> (draw, varyings) and re-derive the span's start (x1, cf2) from the
 // triangle exactly as k_span did; only pixels of a piece with a varying
 // checkpoint read that piece and its span first.
+// a pixel of the programme, from its winner: the triangle, and of a piece with a
+// checkpoint (from_ck) its index wi, first pixel xa and factor cfa there
 template <int PROG>
-__global__ void __launch_bounds__(256, 6) k_shade(const PsSpan* __restrict__ spans, const PsSeg* __restrict__ segs,
-                                               const float* __restrict__ ck, const PsTri* __restrict__ tris,
+__device__ __forceinline__ void ps_shade_pixel(const PsView& V, int x, int y, int64_t crow, int tri, const PsTri& tr, bool from_ck,
+                                               uint32_t wi, int xa, float cfa, const float* __restrict__ ck, int ck_stride,
                                                const float* __restrict__ vary, int nvs, const float* __restrict__ grads,
-                                               const PsDraw* __restrict__ draws, PsFrame f, const PsCounters* cnt, int clears)
+                                               const PsDraw* __restrict__ draws)
 {
     typedef PsProc<PROG> P;
-    const bool poisoned = ps_poisoned(cnt);
-    const int64_t lb = ps_xcd_remap<4>(blockIdx.x, gridDim.x);
-    const PsView& V = f.views[ps_view_of_stile(f, lb)];
-    int64_t st = lb - V.stile_base;
-    // a view has fewer than 2^31 shading blocks
-    const uint32_t st32 = (uint32_t)st, nsx = (uint32_t)V.n_stiles_x;
-    int sy = (int)(st32 / nsx), sx = (int)(st32 - (uint32_t)sy * nsx);
-    int x = sx * 16 + (threadIdx.x & 15);
-    int y = sy * 16 + (threadIdx.x >> 4);
-    if (x >= V.W || y >= V.H) return;
-    const int64_t crow = V.colour_top_down ? (int64_t)(V.colour_h - 1 - y) : (int64_t)y;
-    int w = V.winner[ps_winner_at(V, x, y)];
-    if (poisoned) return;
-    if (w == -1) {   // no fragment colours the pixel: a fused clear of its row, if any, is all it gets
-        if (clears && crow < V.cclear_rows) V.colour[crow * V.colour_scan + x] = V.cclear_value;
-        return;
-    }
-    // a piece with a checkpoint: its first pixel xa carries the accumulators
-    // as the serial walk from x1 leaves them
-    const bool from_ck = (uint32_t)w & PS_SEG_CK;
-    const uint32_t wi = (uint32_t)w & ~PS_SEG_CK;
-    int tri = (int)wi, xa = 0;
-    float cfa = 0.0f;
-    if (from_ck) {
-        const PsSeg sg = segs[wi];
-        tri = spans[sg.si & PS_SEG_SPAN_MASK].tri;
-        xa = (int)(sg.xab & 0xffffu);
-        cfa = sg.cf2;
-    }
-    const PsTri tr = tris[tri];
-    if (ps_tri_prog(tr) != PROG) return;
     const int di = (int)(tr.code >> 8);
     PsEdge L, R;
     ps_row_edges(tr, y, L, R);
@@ -2394,7 +2384,7 @@ __global__ void __launch_bounds__(256, 6) k_shade(const PsSpan* __restrict__ spa
     // the serial walk on to the pixel
     int xs = left < 0 ? 0 : left;
     if (from_ck) {
-        const float* c = ck + (int64_t)wi * f.ck_stride;
+        const float* c = ck + (int64_t)wi * ck_stride;
 #pragma unroll
         for (int i = 0; i < P::NV; i++) vs[i] = c[i];
         xs = xa;
@@ -2450,6 +2440,60 @@ __global__ void __launch_bounds__(256, 6) k_shade(const PsSpan* __restrict__ spa
     }
     if (hit) V.colour[crow * V.colour_scan + x] = c;
     else if (crow < V.cclear_rows) V.colour[crow * V.colour_scan + x] = V.cclear_value;
+}
+
+// PROG 0: every programme, each wave running through those of its pixels (see
+// k_setup)
+#define PS_SHADE_PROGS(X)                                                                            \
+    X(PSGPU_PROC_DEF01) X(PSGPU_PROC_DEF02) X(PSGPU_PROC_DEF03) X(PSGPU_PROC_DEF04)                  \
+    X(PSGPU_PROC_LAMBERT) X(PSGPU_PROC_BLINN) X(PSGPU_PROC_SHADOWED)
+template <int PROG>
+__global__ void __launch_bounds__(256, 6) k_shade(const PsSpan* __restrict__ spans, const PsSeg* __restrict__ segs,
+                                               const float* __restrict__ ck, const PsTri* __restrict__ tris,
+                                               const float* __restrict__ vary, int nvs, const float* __restrict__ grads,
+                                               const PsDraw* __restrict__ draws, PsFrame f, const PsCounters* cnt)
+{
+    const bool poisoned = ps_poisoned(cnt);
+    const int64_t lb = ps_xcd_remap<4>(blockIdx.x, gridDim.x);
+    const PsView& V = f.views[ps_view_of_stile(f, lb)];
+    int64_t st = lb - V.stile_base;
+    // a view has fewer than 2^31 shading blocks
+    const uint32_t st32 = (uint32_t)st, nsx = (uint32_t)V.n_stiles_x;
+    int sy = (int)(st32 / nsx), sx = (int)(st32 - (uint32_t)sy * nsx);
+    int x = sx * 16 + (threadIdx.x & 15);
+    int y = sy * 16 + (threadIdx.x >> 4);
+    if (x >= V.W || y >= V.H) return;
+    const int64_t crow = V.colour_top_down ? (int64_t)(V.colour_h - 1 - y) : (int64_t)y;
+    int w = V.winner[ps_winner_at(V, x, y)];
+    if (poisoned) return;
+    if (w == -1) {   // no fragment colours the pixel: a fused clear of its row, if any, is all it gets
+        if (crow < V.cclear_rows) V.colour[crow * V.colour_scan + x] = V.cclear_value;
+        return;
+    }
+    // a piece with a checkpoint: its first pixel xa carries the accumulators
+    // as the serial walk from x1 leaves them
+    const bool from_ck = (uint32_t)w & PS_SEG_CK;
+    const uint32_t wi = (uint32_t)w & ~PS_SEG_CK;
+    int tri = (int)wi, xa = 0;
+    float cfa = 0.0f;
+    if (from_ck) {
+        const PsSeg sg = segs[wi];
+        tri = spans[sg.si & PS_SEG_SPAN_MASK].tri;
+        xa = (int)(sg.xab & 0xffffu);
+        cfa = sg.cf2;
+    }
+    const PsTri tr = tris[tri];
+    const int prog = ps_tri_prog(tr);
+#define SH_PIXEL(K) \
+    ps_shade_pixel<K>(V, x, y, crow, tri, tr, from_ck, wi, xa, cfa, ck, f.ck_stride, vary, nvs, grads, draws)
+    if constexpr (PROG != 0) {
+        if (prog == PROG) SH_PIXEL(PROG);
+    } else {
+#define SH_ONE(K) if (prog == K) SH_PIXEL(K);
+        PS_SHADE_PROGS(SH_ONE)
+#undef SH_ONE
+    }
+#undef SH_PIXEL
 }
 
 // ---------------------------------------------------------------------------
@@ -2610,15 +2654,13 @@ void psk_setup(hipStream_t s, int prog, bool share, const PsDraw* draws, int nd,
     size_t lds = (size_t)128 * 3 * nvs * sizeof(float);
 #define SU_CASE(K)                                                                                                  \
     case K:                                                                                                         \
-        if (share && ps_shares_varyings(K))                                                                         \
+        if (share && (K == 0 || ps_shares_varyings(K)))                                                                         \
             hipLaunchKernelGGL((k_setup<K, true>), g, b, lds, s, draws, nd, T, tris, vary, nvs, grads, nrows, row_part, cnt, views); \
         else                                                                                                        \
             hipLaunchKernelGGL((k_setup<K, false>), g, b, lds, s, draws, nd, T, tris, vary, nvs, grads, nrows, row_part, cnt, views); \
         break;
     switch (prog) {
-    SU_CASE(PSGPU_PROC_DEF01) SU_CASE(PSGPU_PROC_DEF02) SU_CASE(PSGPU_PROC_DEF03) SU_CASE(PSGPU_PROC_DEF04)
-    SU_CASE(PSGPU_PROC_DEF05) SU_CASE(PSGPU_PROC_LAMBERT) SU_CASE(PSGPU_PROC_BLINN) SU_CASE(PSGPU_PROC_SHADOWED)
-    SU_CASE(PSGPU_PROC_CLOUD) SU_CASE(PSGPU_PROC_CLOUD_SHADOW)
+    SU_CASE(0) PS_SETUP_PROGS(SU_CASE) SU_CASE(PSGPU_PROC_CLOUD) SU_CASE(PSGPU_PROC_CLOUD_SHADOW)
     }
 #undef SU_CASE
 }
@@ -2658,14 +2700,6 @@ void psk_span(hipStream_t s, const PsTri* tris, const uint32_t* row_off, const u
     const int tile_cols = 64 / tile_rows;
     hipLaunchKernelGGL(k_span, dim3(g), dim3(256), 0, s, tris, row_off, bstart, T, cap, spans, tcnt, views, n_views,
                        chunk_w, tile_rows, tile_cols, heavy, wide, cnt, flag);
-}
-
-void psk_scan_rows(hipStream_t s, const uint32_t* in, int64_t n, uint32_t* out, uint32_t* partial, uint32_t* total_out,
-                   uint32_t* bstart, int64_t bcap, uint32_t* wide)
-{
-    hipLaunchKernelGGL(k_scan_reduce<uint32_t>, dim3(psk_scan_blocks(n)), dim3(256), 0, s, in, (const uint32_t*)nullptr, n,
-                       partial, (const PsCounters*)nullptr);
-    psk_scan_parts(s, in, n, out, partial, SCAN_BLOCK, total_out, bstart, bcap, wide);
 }
 
 void psk_segments(hipStream_t s, const PsSpan* spans, const uint32_t* row_off, int64_t T, const PsFrame& f,
@@ -2733,15 +2767,12 @@ void psk_raster_imm(hipStream_t s, int prog, bool debug, const PsSpan* spans, co
 }
 
 void psk_shade(hipStream_t s, int prog, const PsSpan* spans, const PsSeg* segs, const float* ck, const PsTri* tris,
-               const float* vary, int nvs, const float* grads, const PsDraw* draws, const PsFrame& f, const PsCounters* cnt,
-               bool clears)
+               const float* vary, int nvs, const float* grads, const PsDraw* draws, const PsFrame& f, const PsCounters* cnt)
 {
     dim3 g((unsigned)f.n_stiles), b(256);
-#define SH_CASE(K) case K: hipLaunchKernelGGL(k_shade<K>, g, b, 0, s, spans, segs, ck, tris, vary, nvs, grads, draws, f, cnt, \
-                                              clears ? 1 : 0); break;
+#define SH_CASE(K) case K: hipLaunchKernelGGL(k_shade<K>, g, b, 0, s, spans, segs, ck, tris, vary, nvs, grads, draws, f, cnt); break;
     switch (prog) {
-    SH_CASE(PSGPU_PROC_DEF01) SH_CASE(PSGPU_PROC_DEF02) SH_CASE(PSGPU_PROC_DEF03) SH_CASE(PSGPU_PROC_DEF04)
-    SH_CASE(PSGPU_PROC_LAMBERT) SH_CASE(PSGPU_PROC_BLINN) SH_CASE(PSGPU_PROC_SHADOWED)
+    SH_CASE(0) PS_SHADE_PROGS(SH_CASE)
     default: break;
     }
 #undef SH_CASE

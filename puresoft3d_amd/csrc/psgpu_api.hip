@@ -539,11 +539,11 @@ int stage_blob(psgpu_ctx* c, const Blob& b, uint8_t** out)
     return PSGPU_OK;
 }
 
-// partial sums of the row scan: one per scan block, or one per setup block
+// partial sums of the row scan: one per setup block
 int64_t row_partials(int64_t T)
 {
     const int sb = psk_setup_block();
-    return std::max<int64_t>(psk_scan_blocks(T), (T + sb - 1) / sb) + 1;
+    return (T + sb - 1) / sb + 1;
 }
 
 // size the per-flush scratch for a flush of T triangles, nvs varying floats
@@ -614,29 +614,23 @@ int run_flush(psgpu_ctx* c, const Cmd& cmd, uint8_t* staged)
     int* flag = c->in_stream_capture || c->fixed_scratch ? c->h_flags + psgpu_ctx::kFlagCap : c->flush_flag;
     int nd = blob.nd;
     const PsView* dv = f.views;
-    // a flush of one programme has one setup launch, which also leaves the
-    // row totals of its blocks for the row scan
-    int n_progs = 0;
-    for (int k = 1; k < PS_N_PROGS; k++) n_progs += progs[k] ? 1 : 0;
-    uint32_t* row_part = n_progs == 1 ? c->fb.partial.p : nullptr;
+    // one launch for all programmes, which also leaves the row totals of its
+    // blocks for the row scan
     {
         ProfScope p(c, "setup");
+        int prog = 0, n = 0;
+        bool shares = false;
         for (int k = 1; k < PS_N_PROGS; k++)
-            if (progs[k])
-                psk_setup(s, k, blob.shares[k], dd, nd, T, c->fb.tris.p, c->fb.vary.p, nvs, c->fb.grad.p, c->fb.nrows.p,
-                          row_part, c->d_cnt, dv);
+            if (progs[k]) { prog = k; n++; shares |= blob.shares[k]; }
+        psk_setup(s, n == 1 ? prog : 0, shares, dd, nd, T, c->fb.tris.p, c->fb.vary.p, nvs, c->fb.grad.p, c->fb.nrows.p,
+                  c->fb.partial.p, c->d_cnt, dv);
     }
     {
         ProfScope p(c, "scan_rows");
         // row counts never depend on buffer capacities: always scanned, so the
         // largest row total of the log is known even after an overflow
-        const int sb = psk_setup_block();
-        if (row_part)
-            psk_scan_parts(s, c->fb.nrows.p, T, c->fb.rowoff.p, row_part, sb, c->d_sizes + 0, c->fb.bstart.p,
-                           c->fb.span_cap / 64 + 2, c->fb.wide.p);
-        else
-            psk_scan_rows(s, c->fb.nrows.p, T, c->fb.rowoff.p, c->fb.partial.p, c->d_sizes + 0, c->fb.bstart.p,
-                          c->fb.span_cap / 64 + 2, c->fb.wide.p);
+        psk_scan_parts(s, c->fb.nrows.p, T, c->fb.rowoff.p, c->fb.partial.p, psk_setup_block(), c->d_sizes + 0, c->fb.bstart.p,
+                       c->fb.span_cap / 64 + 2, c->fb.wide.p);
     }
     // k_span finds each row's triangle by a search in the row offsets,
     // started from the row scan's table of every 64th item's triangle and
@@ -681,13 +675,13 @@ int run_flush(psgpu_ctx* c, const Cmd& cmd, uint8_t* staged)
     }
     {
         ProfScope p(c, "shade");
-        bool clears = true;   // the first shading launch also writes the fused colour clears
+        // one launch, which also writes the fused colour clears
+        int prog = 0, n = 0;
         for (int k = 1; k < PS_N_PROGS; k++)
-            if (shade_progs[k]) {
-                psk_shade(s, k, c->fb.spans.p, c->fb.segs.p, c->fb.ck.p, c->fb.tris.p, c->fb.vary.p, nvs, c->fb.grad.p, dd, f,
-                          c->d_cnt, clears);
-                clears = false;
-            }
+            if (shade_progs[k]) { prog = k; n++; }
+        if (n > 0)
+            psk_shade(s, n == 1 ? prog : 0, c->fb.spans.p, c->fb.segs.p, c->fb.ck.p, c->fb.tris.p, c->fb.vary.p, nvs,
+                      c->fb.grad.p, dd, f, c->d_cnt);
     }
     HIPCHK(c, hipGetLastError());
     c->stats.flushes++;

@@ -56,3 +56,25 @@ def test_draws_of_a_programme(oracle, prog, n_draws):
 @pytest.mark.parametrize("prog", [N.PROC_DEF03, N.PROC_BLINN, N.PROC_SHADOWED])
 def test_draws_between_another_programmes(oracle, prog):
     assert_same(draws_scene(prog, 5, 60 + prog, 131, 18, other=N.PROC_DEF02), oracle)
+
+
+def programmes_scene(seed, width, height, order):
+    """small draws of the listed programmes, which share the waves that set
+    their triangles up and those that shade them"""
+    sc = scenegen.micro_scene(N.PROC_SHADOWED, seed, width, height, n=6)
+    sc.name = "programmes_s%d_%dx%d_%s" % (seed, width, height, "_".join(map(str, order)))
+    sky = scenegen.micro_scene(N.PROC_DEF04, seed + 1, width, height, n=6)
+    sc.uniforms.update({0: sky.uniforms[0], 1: sky.uniforms[1], 2: np.array([len(sc.textures)], np.int32)})
+    sc.textures += sky.textures
+    rng = np.random.default_rng(seed)
+    sc.draws = []
+    for k, prog in enumerate(order):
+        sc.meshes["p%d" % k] = scenegen._slots_for(prog, scenegen.random_clip_triangles(rng, 5 + 6 * (k % 4)), rng)
+        u = {7: S.vec4(0.48, 0.6, 0.64)} if prog == N.PROC_LAMBERT else {}
+        sc.draws.append(S.DrawSpec("p%d" % k, prog, uniforms=u))
+    return sc
+
+
+@pytest.mark.parametrize("order", [PROGS, PROGS[::-1] + PROGS * 2, [N.PROC_SHADOWED, N.PROC_DEF04], [N.PROC_LAMBERT, N.PROC_DEF03]])
+def test_programmes_of_one_flush(oracle, order):
+    assert_same(programmes_scene(80 + len(order), 131, 37, order), oracle)

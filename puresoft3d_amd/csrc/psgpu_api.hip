@@ -28,7 +28,11 @@
 // memory, held from the library's load until the process ends.  Host code
 // never uses this name as an address: hipGetSymbolAddress gives each
 // device's copy (static_scratch_init), and that address is what kernels get.
-static __device__ __align__(256) uint8_t scratch[PSGPU_STATIC_SCRATCH_BYTES];
+// The slack holds what only widens accesses or shortens kernels (padded winner
+// rows, the heavy-tile list, the list of wide waves), so that these take nothing
+// from the spans and pieces that fit into the stated size.
+static constexpr size_t kStaticSlack = (size_t)8 << 20;
+static __device__ __align__(256) uint8_t scratch[PSGPU_STATIC_SCRATCH_BYTES + kStaticSlack];
 
 namespace {
 
@@ -1197,7 +1201,7 @@ struct Arena {
 };
 
 // the quantities a flush's scratch depends on, as build_blob lays them out
-struct FlushShape { int64_t T = 0, n_pix = 0, n_tiles = 0; int nvs = 1; };
+struct FlushShape { int64_t T = 0, n_pix = 0, n_pad = 0, n_tiles = 0; int nvs = 1; };   // n_pad: of n_pix, the padding
 
 FlushShape flush_shape(psgpu_ctx* c, const Cmd& cmd)
 {
@@ -1207,6 +1211,7 @@ FlushShape flush_shape(psgpu_ctx* c, const Cmd& cmd)
         int n_chunks = (sg.tg.vpw + cw - 1) / cw;
         sh.n_tiles += (int64_t)((n_chunks + tc - 1) / tc) * ((sg.tg.vph + tr - 1) / tr);
         sh.n_pix += PS_WINNER_PITCH(sg.tg.vpw) * sg.tg.vph;
+        sh.n_pad += (PS_WINNER_PITCH(sg.tg.vpw) - sg.tg.vpw) * sg.tg.vph;
         for (const PsDraw& d : sg.draws) {
             sh.T += d.tri_count;
             sh.nvs = std::max(sh.nvs, d.nv);
@@ -2373,6 +2378,9 @@ int psgpu_sync_noalloc(psgpu_ctx* c)
         if (sh.T > 0 && !(blob_dev = arena.take_bytes(bytes)))
             return fail(c, PSGPU_ERR_NOMEM, "the draw records exceed the static scratch array");
     }
+    // 192 KiB: the heavy-tile list, and a word per 64 spans of the list of wide
+    // waves for the two million spans that the array holds at most
+    arena.cap += std::min(kStaticSlack, (size_t)sh.n_pad * 4 + (192 << 10));
     if (sh.T > 0 && !carve_flush(arena, sh, sb))
         return fail(c, PSGPU_ERR_NOMEM,
                     "a flush of %lld triangles over %lld pixels needs more than the %zu-byte static scratch array",

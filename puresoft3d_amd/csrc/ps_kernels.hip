@@ -2341,10 +2341,11 @@ __global__ void __launch_bounds__(512) k_raster_imm(const PsSpan* __restrict__ s
         }
         if (dirty) ps_store_run<KCW>((uint32_t*)drow + X0, ncol, dv);
     } else {
-        for (int k = 0; k < ncol; k++) {
-            const uint2 q = pix[k * 64 + lane];
-            dirty |= q.x != __float_as_uint(drow[X0 + k]);
-            if (COLOUR && q.y != crow[X0 + k]) crow[X0 + k] = q.y;
+        // (one texture may be both targets)
+        for (int k = 0; k < ncol; k++) dirty |= pix[k * 64 + lane].x != __float_as_uint(drow[X0 + k]);
+        for (int k = 0; COLOUR && k < ncol; k++) {
+            const uint32_t c = pix[k * 64 + lane].y;
+            if (c != crow[X0 + k]) crow[X0 + k] = c;
         }
         if (dirty)
             for (int k = 0; k < ncol; k++) drow[X0 + k] = __uint_as_float(pix[k * 64 + lane].x);

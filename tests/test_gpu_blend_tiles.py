@@ -65,3 +65,34 @@ def test_layer_without_pieces_keeps_the_ground(oracle):
     sc = crowded_layers(N.PROC_CLOUD, 40, 131, 35, 3, False)
     sc.meshes["l0"][0][:, 0] += 50.0
     assert_both(sc, oracle)
+
+
+@pytest.mark.parametrize("tiling", [None, (2, 16, 1), (16, 4, 5)])
+def test_one_texture_as_both_targets(tiling):
+    """a blended layer that tests depth and leaves it, into a texture that is
+    colour and depth target at once: the colours of two separate targets of
+    the same bits"""
+    announce("one texture as both targets %s" % (tiling,))
+    w, h = 52, 35
+    sc = crowded_layers(N.PROC_CLOUD, 60, w, h, 21, False)
+    sc.draws = [S.DrawSpec("l0", N.PROC_CLOUD, behavior=N.TEST_DEPTH | N.ALPHABLEND)]
+    bits = np.random.default_rng(4).uniform(-1, 1, (h, w)).astype(np.float32).view(np.uint8).reshape(h, w, 4)
+    ctx = N.Context(w, h)
+    try:
+        if tiling:
+            ctx.tiling(*tiling)
+        gs = S.GpuScene(ctx, sc)
+        both, colour, depth = (ctx.texture_create(w, h, 4, wrap=N.CLAMP, pixels=bits) for _ in range(3))
+        got = []
+        for c, d in ((both, both), (colour, depth)):
+            ctx.target(c)
+            ctx.depth_target(d)
+            ctx.viewport(w, h)
+            gs.frame(clear=False)
+            got.append(ctx.texture_download(c).ravel())
+        unchanged = ctx.texture_download(depth).ravel()
+    finally:
+        ctx.close()
+    assert (got[1] != bits.ravel()).any()
+    np.testing.assert_array_equal(unchanged, bits.ravel())
+    np.testing.assert_array_equal(got[0], got[1])

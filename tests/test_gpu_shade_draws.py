@@ -78,3 +78,33 @@ def programmes_scene(seed, width, height, order):
 @pytest.mark.parametrize("order", [PROGS, PROGS[::-1] + PROGS * 2, [N.PROC_SHADOWED, N.PROC_DEF04], [N.PROC_LAMBERT, N.PROC_DEF03]])
 def test_programmes_of_one_flush(oracle, order):
     assert_same(programmes_scene(80 + len(order), 131, 37, order), oracle)
+
+
+def test_programmes_of_several_views():
+    """views of one flush whose draws, of several programmes, share varyings:
+    the images of the views rendered one by one"""
+    w, h = 75, 37
+    sc = programmes_scene(91, w, h, [N.PROC_BLINN, N.PROC_DEF04, N.PROC_DEF02, N.PROC_LAMBERT, N.PROC_BLINN])
+    pv = [S.colmajor(np.diag([1.0 - 0.2 * k, 1.0, 1.0, 1.0])) for k in range(3)]
+    ctx = N.Context(w, h)
+    try:
+        gs = S.GpuScene(ctx, sc)
+        images = []
+        for together in (False, True):
+            views = [(ctx.texture_create(w, h, 4, wrap=N.CLAMP), ctx.texture_create(w, h, 4, wrap=N.CLAMP)) for _ in pv]
+            for (c, d), m in zip(views, pv):
+                ctx.target(c)
+                ctx.depth_target(d)
+                ctx.viewport(w, h)
+                sc.uniforms[3] = m
+                gs.frame(flush=not together)
+            flushes = ctx.stats()["flushes"]
+            ctx.flush()
+            ctx.sync()
+            assert not together or ctx.stats()["flushes"] == flushes + 1
+            images.append([ctx.texture_download(t).ravel() for v in views for t in v])
+    finally:
+        ctx.close()
+    assert any((a != images[0][0]).any() for a in images[0][2::2])   # the views differ
+    for a, b in zip(*images):
+        np.testing.assert_array_equal(a, b)

@@ -840,9 +840,22 @@ bool split_flush(psgpu_ctx* c, size_t idx)
 // after one that overflowed do nothing until they are replayed.
 int run_logged(psgpu_ctx* c, size_t i)
 {
+    if (i >= (size_t)psgpu_ctx::kFlagCap) return fail(c, PSGPU_ERR_STATE, "internal: more logged commands than flag words");
     c->h_flags[i] = 0;
     c->flush_flag = c->h_flags + i;
     return run_cmd(c, c->log[i]);
+}
+
+// log a command and run it.  A log without a flag word left is ended by a sync
+// first, whatever adds to it: a recorded list may hold any number of commands.
+int log_and_run(psgpu_ctx* c, Cmd&& cmd)
+{
+    if (c->log.size() >= (size_t)psgpu_ctx::kFlagCap - 1) {
+        int rc = do_sync(c);
+        if (rc) return rc;
+    }
+    c->log.push_back(std::move(cmd));
+    return run_logged(c, c->log.size() - 1);
 }
 
 // a command is either recorded (between capture begin/end) or logged and run
@@ -852,12 +865,7 @@ int submit(psgpu_ctx* c, Cmd&& cmd)
         c->capture_list.push_back(std::move(cmd));
         return PSGPU_OK;
     }
-    if ((int)c->log.size() >= psgpu_ctx::kFlagCap - 1) {
-        int rc = do_sync(c);
-        if (rc) return rc;
-    }
-    c->log.push_back(std::move(cmd));
-    return run_logged(c, c->log.size() - 1);
+    return log_and_run(c, std::move(cmd));
 }
 
 // Clears that a flush can apply itself: a clear of a view's whole depth
@@ -1112,11 +1120,8 @@ int graph_prepare(psgpu_ctx* c, Graph& g)
     int rc = do_sync(c);
     if (rc) return rc;
     const int64_t splits = c->stats.splits;
-    for (const Cmd& cmd : g.cmds) {
-        Cmd copy = cmd;
-        c->log.push_back(std::move(copy));
-        if ((rc = run_logged(c, c->log.size() - 1))) return rc;
-    }
+    for (const Cmd& cmd : g.cmds)
+        if ((rc = log_and_run(c, Cmd(cmd)))) return rc;
     if ((rc = do_sync(c))) return rc;
     if (c->stats.splits != splits) return graph_too_large(c);
     return graph_rebuild(c, g);
@@ -2266,11 +2271,8 @@ int psgpu_capture_end(psgpu_ctx* c, int* out_graph)
     g.cmds.swap(c->capture_list);
     // first execution runs eagerly: it sizes every scratch buffer
     const int64_t splits = c->stats.splits;
-    for (const Cmd& cmd : g.cmds) {
-        Cmd copy = cmd;
-        c->log.push_back(std::move(copy));
-        if ((rc = run_logged(c, c->log.size() - 1))) return rc;
-    }
+    for (const Cmd& cmd : g.cmds)
+        if ((rc = log_and_run(c, Cmd(cmd)))) return rc;
     if ((rc = do_sync(c))) return rc;
     if (c->stats.splits != splits) return graph_too_large(c);
     for (const Cmd& cmd : g.cmds) {

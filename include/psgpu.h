@@ -289,7 +289,8 @@ int psgpu_graph_destroy(psgpu_ctx* ctx, int graph);
  * queued clears and draws, as psgpu_sync would, with every per-flush buffer
  * (triangle records, varyings, spans, pieces, sort keys, the winner plane,
  * the draw records themselves) carved from a fixed array of
- * PSGPU_STATIC_SCRATCH_BYTES in the device's memory, and waits for them.  It
+ * PSGPU_STATIC_SCRATCH_BYTES in the device's memory (512 KiB of lists lie
+ * beside it), and waits for them.  It
  * calls no hipMalloc, hipFree or other allocating routine.  Each GPU the
  * library runs on holds one such array from the library's load until the
  * process ends; all contexts on a GPU share it, and calls are serialised by a

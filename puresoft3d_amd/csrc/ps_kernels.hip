@@ -96,9 +96,12 @@ __device__ __forceinline__ int ps_view_of_stile(const PsFrame& f, int64_t t)
     return ps_find_view(f.n_views, t, [&](int v) { return f.views[v].stile_base; });
 }
 
-// Row pitch of a view's winner plane: rows start 32 bytes aligned, so that a
-// raster lane stores its chunk in one instruction.
-__device__ __forceinline__ int64_t ps_winner_at(const PsView& V, int x, int y) { return (int64_t)y * PS_WINNER_PITCH(V.W) + x; }
+// Rows of a padded winner plane start 32 bytes aligned, so that a raster lane
+// stores its chunk in one instruction.
+__device__ __forceinline__ int64_t ps_winner_at(const PsFrame& f, const PsView& V, int x, int y)
+{
+    return (int64_t)y * PS_WINNER_PITCH(V.W, f.winner_pad) + x;
+}
 
 // Workgroups are dealt to the 8 XCDs round-robin (workgroup b runs on XCD
 // b % 8), and each XCD has its own L2.  This maps workgroups to logical
@@ -2033,7 +2036,7 @@ __global__ void __launch_bounds__(512, 5) k_raster(const PsSpan* __restrict__ sp
         }
     }
     const bool write_depth = __any(dirty);
-    uint32_t* wrow = (uint32_t*)V.winner + ps_winner_at(V, 0, y);
+    uint32_t* wrow = (uint32_t*)V.winner + ps_winner_at(f, V, 0, y);
     if constexpr (KCW > 0) {
         uint32_t d[KCW], w[KCW];
 #pragma unroll
@@ -2465,7 +2468,7 @@ __global__ void __launch_bounds__(256, 6) k_shade(const PsSpan* __restrict__ spa
     int y = sy * 16 + (threadIdx.x >> 4);
     if (x >= V.W || y >= V.H) return;
     const int64_t crow = V.colour_top_down ? (int64_t)(V.colour_h - 1 - y) : (int64_t)y;
-    int w = V.winner[ps_winner_at(V, x, y)];
+    int w = V.winner[ps_winner_at(f, V, x, y)];
     if (poisoned) return;
     if (w == -1) {   // no fragment colours the pixel: a fused clear of its row, if any, is all it gets
         if (crow < V.cclear_rows) V.colour[crow * V.colour_scan + x] = V.cclear_value;

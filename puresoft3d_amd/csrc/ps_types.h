@@ -100,8 +100,9 @@ struct PsSeg {
     uint32_t win;
 };
 
-// words per row of a view's winner plane (a multiple of 8)
-#define PS_WINNER_PITCH(w) (((int64_t)(w) + 7) & ~(int64_t)7)
+// words per row of a view's winner plane: a multiple of pad + 1 (PsFrame::winner_pad)
+#define PS_WINNER_PITCH(w, pad) (((int64_t)(w) + (pad)) & ~(int64_t)(pad))
+#define PS_WINNER_PAD 7
 
 // One view of a flush: a viewport and its colour/depth targets.  A flush
 // renders any number of views with the same kernels; tiles and shading
@@ -114,7 +115,7 @@ struct PsView {
     int64_t stile_base;             // first shading block of the view
     uint32_t* colour; int colour_scan; int colour_top_down; int colour_h;  // scan in uint32
     float* depth; int depth_scan;   // scan in floats
-    // H rows of PS_WINNER_PITCH(W): what shading needs of the last colour-writing pass: its triangle,
+    // H rows of PS_WINNER_PITCH(W, winner_pad): what shading needs of the last colour-writing pass: its triangle,
     // or PS_SEG_CK | its piece when the piece keeps a varying checkpoint;
     // -1 for none
     int* winner;
@@ -132,6 +133,7 @@ struct PsView {
 // Flush-wide parameters passed by value to kernels.
 struct PsFrame {
     int chunk_w, tile_rows, tile_cols;   // raster tiling
+    int winner_pad;                      // PS_WINNER_PAD, or 0 where the padding would take scratch from the flush
     int ck_stride;                       // floats per varying checkpoint (the flush's widest NV)
     int n_views;
     int64_t n_tiles, n_stiles;

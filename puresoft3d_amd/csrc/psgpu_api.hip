@@ -28,10 +28,11 @@
 // memory, held from the library's load until the process ends.  Host code
 // never uses this name as an address: hipGetSymbolAddress gives each
 // device's copy (static_scratch_init), and that address is what kernels get.
-// The slack holds what only widens accesses or shortens kernels (padded winner
-// rows, the heavy-tile list, the list of wide waves), so that these take nothing
-// from the spans and pieces that fit into the stated size.
-static constexpr size_t kStaticSlack = (size_t)8 << 20;
+// The slack holds the lists that only shorten kernels (heavy tiles, wide waves),
+// so that these take nothing from the spans and pieces that fit into the stated
+// size.  The winner planes there are not padded: the padding of many narrow
+// views is up to seven times the planes.
+static constexpr size_t kStaticSlack = (size_t)512 << 10;
 static __device__ __align__(256) uint8_t scratch[PSGPU_STATIC_SCRATCH_BYTES + kStaticSlack];
 
 namespace {
@@ -457,6 +458,7 @@ int build_blob(psgpu_ctx* c, const Cmd& cmd, Blob& b, PsFrame& f, int64_t& T, in
     f.chunk_w = c->tiling.chunk_width;
     f.tile_rows = c->tiling.tile_rows;
     f.tile_cols = 64 / f.tile_rows;
+    f.winner_pad = c->fixed_scratch ? 0 : PS_WINNER_PAD;
     int64_t tile_base = 0, stile_base = 0;
     for (size_t v = 0; v < cmd.views.size(); v++) {
         const Segment& sg = cmd.views[v];
@@ -481,7 +483,7 @@ int build_blob(psgpu_ctx* c, const Cmd& cmd, Blob& b, PsFrame& f, int64_t& T, in
         pv.cclear_rows = sg.cclear_rows;
         pv.cclear_value = sg.cclear_value;
         pv.winner = (int*)(intptr_t)n_pix;   // offset; rebased once the winner buffer is known
-        n_pix += PS_WINNER_PITCH(pv.W) * pv.H;
+        n_pix += PS_WINNER_PITCH(pv.W, f.winner_pad) * pv.H;
         views.push_back(pv);
         for (PsDraw d : sg.draws) {
             d.view = (int)v;
@@ -1206,7 +1208,7 @@ struct Arena {
 };
 
 // the quantities a flush's scratch depends on, as build_blob lays them out
-struct FlushShape { int64_t T = 0, n_pix = 0, n_pad = 0, n_tiles = 0; int nvs = 1; };   // n_pad: of n_pix, the padding
+struct FlushShape { int64_t T = 0, n_pix = 0, n_tiles = 0; int nvs = 1; };
 
 FlushShape flush_shape(psgpu_ctx* c, const Cmd& cmd)
 {
@@ -1215,8 +1217,7 @@ FlushShape flush_shape(psgpu_ctx* c, const Cmd& cmd)
     for (const Segment& sg : cmd.views) {
         int n_chunks = (sg.tg.vpw + cw - 1) / cw;
         sh.n_tiles += (int64_t)((n_chunks + tc - 1) / tc) * ((sg.tg.vph + tr - 1) / tr);
-        sh.n_pix += PS_WINNER_PITCH(sg.tg.vpw) * sg.tg.vph;
-        sh.n_pad += (PS_WINNER_PITCH(sg.tg.vpw) - sg.tg.vpw) * sg.tg.vph;
+        sh.n_pix += (int64_t)sg.tg.vpw * sg.tg.vph;
         for (const PsDraw& d : sg.draws) {
             sh.T += d.tri_count;
             sh.nvs = std::max(sh.nvs, d.nv);
@@ -1225,34 +1226,39 @@ FlushShape flush_shape(psgpu_ctx* c, const Cmd& cmd)
     return sh;
 }
 
-// carve every buffer of run_flush for a flush of this shape; the span and
-// piece capacities take what is left (pieces at 1.5 per span, as the
-// allocating path starts them)
-bool carve_flush(Arena& a, const FlushShape& sh, FlushBufs& b)
+// Carve every buffer of run_flush for a flush of this shape from the array a
+// and its slack; the span and piece capacities take what is left of a (pieces
+// at 1.5 per span, as the allocating path starts them).
+bool carve_flush(Arena& a, Arena& slack, const FlushShape& sh, FlushBufs& b)
 {
     const int64_t T = sh.T;
     if (!a.take(b.winner, sh.n_pix) || !a.take(b.tris, T) || !a.take(b.vary, (size_t)T * 3 * sh.nvs) ||
         !a.take(b.grad, (size_t)T * 8) || !a.take(b.nrows, T) || !a.take(b.rowoff, T + 1) ||
         !a.take(b.partial, row_partials(T)) || !a.take(b.tcnt, sh.n_tiles + 1) ||
         !a.take(b.tstart, sh.n_tiles + 1) || !a.take(b.tpartial, psk_scan_blocks(sh.n_tiles) + 1) ||
-        !a.take(b.heavy, psk_heavy_cap() + 1))
+        !slack.take(b.heavy, psk_heavy_cap() + 1))
         return false;
-    // bytes per span: record, entries of the row-start table and the list of wide waves, and 1.5 pieces of
+    // bytes per span: record, entry of the row-start table, and 1.5 pieces of
     // record, checkpoint and two run records
-    const double per_span = 32 + 8.0 / 64 + 1.5 * (sizeof(PsSeg) + 4.0 * sh.nvs + 16);
+    const double per_span = 32 + 4.0 / 64 + 1.5 * (sizeof(PsSeg) + 4.0 * sh.nvs + 16);
+    // the list of wide waves has a word per 64 spans: 153 KiB for the most
+    // spans that the array holds
+    static_assert(PSGPU_STATIC_SCRATCH_BYTES / (32 + (sizeof(PsSeg) + 20) * 3 / 2) / 64 * sizeof(uint32_t) + (64 << 10) <= kStaticSlack,
+                  "the lists fit into the slack");
     size_t left = a.cap - a.used;
     int64_t spans = (int64_t)((double)left / per_span);
     spans = std::min<int64_t>(spans, (int64_t)1 << 26);
-    for (; spans >= 1024; spans -= spans / 16 + 1) {
-        Arena t = a;
+    for (; spans >= 1024; spans--) {   // a few steps: the buffers' alignment
+        Arena t = a, u = slack;
         FlushBufs x = b;
         x.span_cap = spans;
         x.seg_cap = spans * 3 / 2;
-        if (t.take(x.bstart, x.span_cap / 64 + 2) && t.take(x.wide, x.span_cap / 64 + 3) &&
+        if (t.take(x.bstart, x.span_cap / 64 + 2) && u.take(x.wide, x.span_cap / 64 + 3) &&
             t.take(x.spans, x.span_cap) && t.take(x.segs, x.seg_cap) &&
             t.take(x.ck, (size_t)x.seg_cap * sh.nvs) && t.take(x.runs, (size_t)x.seg_cap * 2) &&
             t.take(x.runs2, (size_t)x.seg_cap * 2)) {
             a = t;
+            slack = u;
             b = x;
             return true;
         }
@@ -2380,10 +2386,8 @@ int psgpu_sync_noalloc(psgpu_ctx* c)
         if (sh.T > 0 && !(blob_dev = arena.take_bytes(bytes)))
             return fail(c, PSGPU_ERR_NOMEM, "the draw records exceed the static scratch array");
     }
-    // 192 KiB: the heavy-tile list, and a word per 64 spans of the list of wide
-    // waves for the two million spans that the array holds at most
-    arena.cap += std::min(kStaticSlack, (size_t)sh.n_pad * 4 + (192 << 10));
-    if (sh.T > 0 && !carve_flush(arena, sh, sb))
+    Arena slack{base + PSGPU_STATIC_SCRATCH_BYTES, kStaticSlack};
+    if (sh.T > 0 && !carve_flush(arena, slack, sh, sb))
         return fail(c, PSGPU_ERR_NOMEM,
                     "a flush of %lld triangles over %lld pixels needs more than the %zu-byte static scratch array",
                     (long long)sh.T, (long long)sh.n_pix, (size_t)PSGPU_STATIC_SCRATCH_BYTES);

@@ -31,31 +31,32 @@ struct Geo {
     float lam, s, spec, u, v;
 };
 
-__device__ __forceinline__ void norm3(float* a)
-{
-    float r = 1.0f / sqrtf((a[0] * a[0] + a[1] * a[1]) + a[2] * a[2]);
-    a[0] *= r; a[1] *= r; a[2] *= r;
-}
-
-__device__ __forceinline__ float dot3(const float* a, const float* b) { return (a[0] * b[0] + a[1] * b[1]) + a[2] * b[2]; }
-
+// lam and s from 64-bit sums and roots, rounded once, for both passes: a pixel
+// whose highlight the image has is one whose highlight the gradients have.
+// In FP32 the normalisations round unit vectors' lengths to one side, the
+// exponent multiplies that, and the bias it leaves in the image (some 1e-7)
+// was the largest part of the parameter gradients' error, which sum
+// differences to a target over the whole image (1237x891: 1.0e-6 to 1.7e-6,
+// now 0.1e-6 to 1.2e-6, the rounding of their own atomics); and where the
+// half vector grazes the surface, the sign of s was that of the rounding.  The
+// passes are bound by reading the geometry and by their atomics, and take as
+// long as with FP32 sums (1237x891: 12 and 34 us, 512^2: 5 and 26).
 __device__ __forceinline__ Geo geometry(const DiffArgs& A, const float* __restrict__ gbuf, int64_t p, float e)
 {
     Geo g;
     const float4* gp = (const float4*)(gbuf + p * 12);
-    float4 g0 = gp[0], g1 = gp[1], g2 = gp[2];
+    const float4 g0 = gp[0], g1 = gp[1], g2 = gp[2];
     g.covered = g0.w != 0.0f;
     if (!g.covered) return g;
-    float n[3] = {g0.x, g0.y, g0.z};
-    norm3(n);
-    float L[3], E[3], Hh[3];
-    L[0] = A.light[0] - g1.x; L[1] = A.light[1] - g1.y; L[2] = A.light[2] - g1.z;
-    E[0] = A.camera[0] - g1.x; E[1] = A.camera[1] - g1.y; E[2] = A.camera[2] - g1.z;
-    norm3(L);
-    norm3(E);
-    Hh[0] = L[0] + E[0]; Hh[1] = L[1] + E[1]; Hh[2] = L[2] + E[2];
-    norm3(Hh);
-    float lam = dot3(n, L), s = dot3(n, Hh);
+    const double n[3] = {g0.x, g0.y, g0.z}, at[3] = {g1.x, g1.y, g1.z};
+    double L[3], E[3], H[3];
+    auto dot = [](const double* u, const double* v) { return (u[0] * v[0] + u[1] * v[1]) + u[2] * v[2]; };
+#pragma unroll
+    for (int k = 0; k < 3; k++) { L[k] = (double)A.light[k] - at[k]; E[k] = (double)A.camera[k] - at[k]; }
+    const double rn = rsqrt(dot(n, n)), rl = rsqrt(dot(L, L)), re = rsqrt(dot(E, E));
+#pragma unroll
+    for (int k = 0; k < 3; k++) H[k] = L[k] * rl + E[k] * re;
+    const float lam = (float)(dot(n, L) * rl * rn), s = (float)(dot(n, H) * rsqrt(dot(H, H)) * rn);
     g.lam = lam > 0.0f ? lam : 0.0f;
     g.s = s > 0.0f ? s : 0.0f;
     g.spec = g.s > 0.0f ? A.ks * powf(g.s, e) : 0.0f;
@@ -101,37 +102,6 @@ __device__ __forceinline__ void footprint(const DiffArgs& A, float u, float v, i
     footprint_texels(A, ix, iy, ax, ay, idx, w);
 }
 
-// lam and s of the forward pass from 64-bit sums and roots, rounded once.  In
-// FP32 the normalisations round unit vectors' lengths to one side, the
-// exponent multiplies that, and the bias it leaves in the image (some 1e-7)
-// was the largest part of the parameter gradients' error, which sum
-// differences to a target over the whole image (1237x891: 1.0e-6 to 1.7e-6,
-// now 0.1e-6 to 1.2e-6, the rounding of their own atomics).  The kernel is
-// bound by reading the geometry and takes as long as before (13 us).
-__device__ __forceinline__ Geo geometry_exact(const DiffArgs& A, const float* __restrict__ gbuf, int64_t p, float e)
-{
-    Geo g;
-    const float4* gp = (const float4*)(gbuf + p * 12);
-    const float4 g0 = gp[0], g1 = gp[1], g2 = gp[2];
-    g.covered = g0.w != 0.0f;
-    if (!g.covered) return g;
-    const double n[3] = {g0.x, g0.y, g0.z}, at[3] = {g1.x, g1.y, g1.z};
-    double L[3], E[3], H[3];
-    auto dot = [](const double* u, const double* v) { return (u[0] * v[0] + u[1] * v[1]) + u[2] * v[2]; };
-#pragma unroll
-    for (int k = 0; k < 3; k++) { L[k] = (double)A.light[k] - at[k]; E[k] = (double)A.camera[k] - at[k]; }
-    const double rn = rsqrt(dot(n, n)), rl = rsqrt(dot(L, L)), re = rsqrt(dot(E, E));
-#pragma unroll
-    for (int k = 0; k < 3; k++) H[k] = L[k] * rl + E[k] * re;
-    const float lam = (float)(dot(n, L) * rl * rn), s = (float)(dot(n, H) * rsqrt(dot(H, H)) * rn);
-    g.lam = lam > 0.0f ? lam : 0.0f;
-    g.s = s > 0.0f ? s : 0.0f;
-    g.spec = g.s > 0.0f ? A.ks * powf(g.s, e) : 0.0f;
-    g.u = g2.x;
-    g.v = g2.y;
-    return g;
-}
-
 __global__ void __launch_bounds__(256) k_diff_forward(DiffArgs A, const float* __restrict__ gbuf,
                                                       const float* __restrict__ tex, const float* __restrict__ params,
                                                       float* __restrict__ out)
@@ -139,7 +109,7 @@ __global__ void __launch_bounds__(256) k_diff_forward(DiffArgs A, const float* _
     int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (p >= (int64_t)A.W * A.H) return;
     float a = params[0], e = params[1];
-    Geo g = geometry_exact(A, gbuf, p, e);
+    Geo g = geometry(A, gbuf, p, e);
     float c[3] = {0.0f, 0.0f, 0.0f};
     if (g.covered) {
         int64_t idx[4];

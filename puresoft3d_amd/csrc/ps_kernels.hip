@@ -585,17 +585,15 @@ __global__ void __launch_bounds__(128, 3) k_setup(const PsDraw* __restrict__ dra
     ps_wave_add(cnt, PS_ST_CULLED, culled, true);
     ps_wave_add(cnt, PS_ST_ZREJ, zrej, true);
     ps_wave_add(cnt, PS_ST_DROPPED, dropped, true);
-    if (row_part) {
-        const uint32_t w = __builtin_amdgcn_readlane(ps_wave_incl_scan(myrows), 63);
-        if (lane == 0) wrows[threadIdx.x >> 6] = w;
-        __syncthreads();
-        if (threadIdx.x == 0) row_part[blockIdx.x] = wrows[0] + wrows[1];
-    }
+    const uint32_t w = __builtin_amdgcn_readlane(ps_wave_incl_scan(myrows), 63);
+    if (lane == 0) wrows[threadIdx.x >> 6] = w;
+    __syncthreads();
+    if (threadIdx.x == 0) row_part[blockIdx.x] = wrows[0] + wrows[1];
 }
 
 // ---------------------------------------------------------------------------
-// exclusive scan (uint32, or uint64 holding two 32-bit counts side by side)
-// with a device-side length; out[n] = total
+// exclusive scans of the tiles' counts (two 32-bit counts side by side) and of
+// the triangles' row counts; out[n] = total
 // ---------------------------------------------------------------------------
 #define SCAN_ITEMS 16
 #define SCAN_BLOCK (256 * SCAN_ITEMS)
@@ -609,12 +607,12 @@ __host__ __device__ __forceinline__ int64_t ps_heavy_cap(int64_t n) { return n /
 
 // Pieces that make a tile heavy: three times the flush's mean per tile (at
 // least 96).  The flush's pieces are k_span's 64-bit count in the pending
-// statistics: ps_pend_pieces loads one stripe per lane (0 without counters),
+// statistics: ps_pend_pieces loads one stripe per lane,
 // ps_wave_sum64 adds the wave's stripes.
 __device__ __forceinline__ unsigned long long ps_pend_pieces(const PsCounters* c)
 {
     static_assert(PS_STRIPES == 64, "one stripe per lane");
-    return c ? c->pend[threadIdx.x & 63][PS_ST_SEGS] : 0ull;
+    return c->pend[threadIdx.x & 63][PS_ST_SEGS];
 }
 
 __device__ __forceinline__ unsigned long long ps_wave_sum64(unsigned long long x)
@@ -638,42 +636,34 @@ __device__ __forceinline__ uint32_t ps_heavy_min(unsigned long long pieces, int6
     return (uint32_t)min(max(h, 96ull), 0xffffffffull);
 }
 
-// inclusive wave scan of uint32, or of the two 32-bit halves of a uint64
-// separately (the packed counts never carry from the low half)
-__device__ __forceinline__ uint32_t ps_wave_incl_scan_t(uint32_t v) { return ps_wave_incl_scan(v); }
-__device__ __forceinline__ unsigned long long ps_wave_incl_scan_t(unsigned long long v)
+// inclusive wave scan of the two 32-bit halves separately (the packed counts
+// never carry from the low half)
+__device__ __forceinline__ unsigned long long ps_wave_incl_scan2(unsigned long long v)
 {
     return (unsigned long long)ps_wave_incl_scan((uint32_t)v) |
            ((unsigned long long)ps_wave_incl_scan((uint32_t)(v >> 32)) << 32);
 }
 
-__device__ __forceinline__ uint32_t ps_wave_bcast63(uint32_t v) { return __builtin_amdgcn_readlane(v, 63); }
-__device__ __forceinline__ uint32_t ps_wave_bcast0(uint32_t v) { return __builtin_amdgcn_readlane(v, 0); }
-__device__ __forceinline__ unsigned long long ps_wave_bcast0(unsigned long long v)
+__device__ __forceinline__ unsigned long long ps_readlane64(unsigned long long v, int lane)
 {
-    return (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((uint32_t)v, 0) |
-           ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((uint32_t)(v >> 32), 0) << 32);
-}
-__device__ __forceinline__ unsigned long long ps_wave_bcast63(unsigned long long v)
-{
-    return (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((uint32_t)v, 63) |
-           ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((uint32_t)(v >> 32), 63) << 32);
+    return (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((uint32_t)v, lane) |
+           ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((uint32_t)(v >> 32), lane) << 32);
 }
 
-// exclusive scan of one value per thread over a block of NW waves
-template <typename T, int NW>
-__device__ __forceinline__ T ps_block_excl_scan(T v, T* lds, T& total)
+// exclusive scan of one value per thread over a block of four waves
+__device__ __forceinline__ unsigned long long ps_block_excl_scan(unsigned long long v, unsigned long long* lds,
+                                                                 unsigned long long& total)
 {
-    int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    T x = ps_wave_incl_scan_t(v);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const unsigned long long x = ps_wave_incl_scan2(v);
     if (lane == 63) lds[wave] = x;
     __syncthreads();
-    T wbase = 0;
+    unsigned long long wbase = 0;
     total = 0;
 #pragma unroll
-    for (int w = 0; w < NW; w++) {
-        T l = lds[w];
-        wbase += (w < wave) ? l : (T)0;
+    for (int w = 0; w < 4; w++) {
+        const unsigned long long l = lds[w];
+        wbase += (w < wave) ? l : 0ull;
         total += l;
     }
     __syncthreads();
@@ -681,25 +671,22 @@ __device__ __forceinline__ T ps_block_excl_scan(T v, T* lds, T& total)
 }
 
 // Wave-striped ownership: the wave owns items [wbase, wbase + 64 * SCAN_ITEMS),
-// in groups of 64 * PER (PER = the items in 16 bytes); in group g the lane
-// owns the PER consecutive items wbase + g * 64 * PER + lane * PER + j, so
-// each group is one coalesced 16-byte load or store per lane.
-template <typename T>
-__device__ __forceinline__ void ps_load_items(const T* in, int64_t wbase, int64_t n, T* v)
+// in groups of 128; in group g the lane owns the two consecutive items
+// wbase + g * 128 + lane * 2 + j, so each group is one coalesced 16-byte load
+// or store per lane.
+__device__ __forceinline__ void ps_load_items(const unsigned long long* in, int64_t wbase, int64_t n, unsigned long long* v)
 {
-    constexpr int PER = 16 / sizeof(T);
     const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int g = 0; g < SCAN_ITEMS / PER; g++) {
-        const int64_t i = wbase + (int64_t)g * 64 * PER + lane * PER;
-        if (i + PER <= n) {
-            const uint4 u = *(const uint4*)(in + i);
-            const T* t = (const T*)&u;
-#pragma unroll
-            for (int j = 0; j < PER; j++) v[g * PER + j] = t[j];
+    for (int g = 0; g < SCAN_ITEMS / 2; g++) {
+        const int64_t i = wbase + (int64_t)g * 128 + lane * 2;
+        if (i + 2 <= n) {
+            const ulonglong2 u = *(const ulonglong2*)(in + i);
+            v[g * 2] = u.x;
+            v[g * 2 + 1] = u.y;
         } else {
-#pragma unroll
-            for (int j = 0; j < PER; j++) v[g * PER + j] = i + j < n ? in[i + j] : (T)0;
+            v[g * 2] = i < n ? in[i] : 0ull;
+            v[g * 2 + 1] = 0ull;
         }
     }
 }
@@ -708,15 +695,14 @@ __device__ __forceinline__ void ps_load_items(const T* in, int64_t wbase, int64_
 // least heavy_min pieces.
 __device__ __forceinline__ uint32_t ps_heavy_count(int64_t wbase, int64_t n, const unsigned long long* v, uint32_t heavy_min)
 {
-    constexpr int PER = 2;
     const int lane = threadIdx.x & 63;
     uint32_t nh = 0;
 #pragma unroll
-    for (int g = 0; g < SCAN_ITEMS / PER; g++)
+    for (int g = 0; g < SCAN_ITEMS / 2; g++)
 #pragma unroll
-        for (int j = 0; j < PER; j++) {
-            const int64_t i = wbase + (int64_t)g * 64 * PER + lane * PER + j;
-            nh += (i < n && (uint32_t)v[g * PER + j] >= heavy_min) ? 1u : 0u;
+        for (int j = 0; j < 2; j++) {
+            const int64_t i = wbase + (int64_t)g * 128 + lane * 2 + j;
+            nh += (i < n && (uint32_t)v[g * 2 + j] >= heavy_min) ? 1u : 0u;
         }
     return nh;
 }
@@ -734,151 +720,115 @@ __device__ __forceinline__ uint32_t ps_heavy_reserve(uint32_t nh, uint32_t* heav
     return __builtin_amdgcn_readlane(base, 0) + incl - nh;
 }
 
-// The wave's exclusive prefix of its items (from `run` on) into out.  Tile
-// scans (T = uint64, heavy given) also list the tiles of at least heavy_min
-// pieces in heavy[1 ..], the lane's from slot hslot on (up to hcap are
-// listed), and mark the listed ones with bit 63 of their start.
-template <typename T>
-__device__ __forceinline__ void ps_store_scan(T* out, int64_t wbase, int64_t n, const T* v, T run,
-                                              uint32_t heavy_min = 0xffffffffu, uint32_t* heavy = nullptr,
-                                              uint32_t hslot = 0xffffffffu, uint32_t hcap = 0)
+// The wave's exclusive prefix of its items (from `run` on) into out.  With a
+// heavy list (hslot given) it also lists the tiles of at least heavy_min pieces
+// in heavy[1 ..], the lane's from slot hslot on (up to hcap are listed), and
+// marks the listed ones with bit 63 of their start.
+__device__ __forceinline__ void ps_store_scan(unsigned long long* out, int64_t wbase, int64_t n, const unsigned long long* v,
+                                              unsigned long long run, uint32_t heavy_min, uint32_t* heavy, uint32_t hslot,
+                                              uint32_t hcap)
 {
-    constexpr int PER = 16 / sizeof(T);
     const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int g = 0; g < SCAN_ITEMS / PER; g++) {
-        T sum = 0;
+    for (int g = 0; g < SCAN_ITEMS / 2; g++) {
+        const unsigned long long sum = v[g * 2] + v[g * 2 + 1];
+        const unsigned long long x = ps_wave_incl_scan2(sum);
+        const int64_t i = wbase + (int64_t)g * 128 + lane * 2;
+        unsigned long long o[2] = {run + x - sum, run + x - v[g * 2 + 1]};
 #pragma unroll
-        for (int j = 0; j < PER; j++) sum += v[g * PER + j];
-        const T x = ps_wave_incl_scan_t(sum);
-        T r = run + x - sum;
-        const int64_t i = wbase + (int64_t)g * 64 * PER + lane * PER;
-        T o[PER];
-#pragma unroll
-        for (int j = 0; j < PER; j++) {
-            o[j] = r;
-            if constexpr (sizeof(T) == 8) {
-                if (hslot != 0xffffffffu && i + j < n && (uint32_t)v[g * PER + j] >= heavy_min) {
-                    if (hslot < hcap) {
-                        heavy[1 + hslot] = (uint32_t)(i + j);
-                        o[j] |= 1ull << 63;
-                    }
-                    hslot++;
+        for (int j = 0; j < 2; j++)
+            if (hslot != 0xffffffffu && i + j < n && (uint32_t)v[g * 2 + j] >= heavy_min) {
+                if (hslot < hcap) {
+                    heavy[1 + hslot] = (uint32_t)(i + j);
+                    o[j] |= 1ull << 63;
                 }
+                hslot++;
             }
-            r += v[g * PER + j];
-        }
-        if (i + PER <= n) {
-            uint4 u;
-            T* t = (T*)&u;
-#pragma unroll
-            for (int j = 0; j < PER; j++) t[j] = o[j];
-            *(uint4*)(out + i) = u;
-        } else {
-            for (int j = 0; j < PER; j++)
-                if (i + j < n) out[i + j] = o[j];
-        }
-        run += ps_wave_bcast63(x);
+        if (i + 2 <= n) *(ulonglong2*)(out + i) = make_ulonglong2(o[0], o[1]);
+        else if (i < n) out[i] = o[0];
+        run += ps_readlane64(x, 63);
     }
 }
 
-// The tile scan (T = uint64) adds 32-bit piece counts: when the flush's
-// pieces, which k_span also counts in 64 bits into the pending statistics,
-// do not fit, it reports the largest total and flags an overflow, so that
-// the flush is split.  Called by the 64 lanes of one wave.
-template <typename T>
-__device__ __forceinline__ void ps_scan_total(T tot, int64_t n, int64_t cap, T* out, uint32_t* total_out,
-                                              PsCounters* c, int* flag, unsigned long long pieces = 0)
+// The tile scan adds 32-bit piece counts: when the flush's pieces, which
+// k_span also counts in 64 bits into the pending statistics, do not fit, it
+// reports the largest total and flags an overflow, so that the flush is
+// split.  Called by the 64 lanes of one wave.
+__device__ __forceinline__ void ps_scan_total(unsigned long long tot, int64_t n, unsigned long long* out, uint32_t* total_out,
+                                              PsCounters* c, int* flag, unsigned long long pieces)
 {
-    const int lane = threadIdx.x & 63;
-    if (lane == 0 && n <= cap) {
-        out[n] = tot;
-        if (total_out) {
-            *total_out = (uint32_t)tot;
-            atomicMax(total_out + 2, (uint32_t)tot);
-        }
-    }
-    if constexpr (sizeof(T) == 8) {
-        if (lane == 0 && pieces != (uint32_t)tot) {
-            if (total_out) atomicMax(total_out + 2, 0xffffffffu);
-            ps_overflow(c, 1, flag);
-        }
+    if ((threadIdx.x & 63) != 0) return;
+    out[n] = tot;
+    *total_out = (uint32_t)tot;
+    atomicMax(total_out + 2, (uint32_t)tot);
+    if (pieces != (uint32_t)tot) {
+        atomicMax(total_out + 2, 0xffffffffu);
+        ps_overflow(c, 1, flag);
     }
 }
 
-template <typename T>
-__global__ void __launch_bounds__(256) k_scan_reduce(const T* __restrict__ in, const uint32_t* n_ptr, int64_t n_host,
-                                                     T* __restrict__ partial, const PsCounters* c)
+__global__ void __launch_bounds__(256) k_scan_reduce(const unsigned long long* __restrict__ in, int64_t n,
+                                                     unsigned long long* __restrict__ partial, const PsCounters* c)
 {
-    __shared__ T lds[4];
-    int64_t n = n_ptr ? (int64_t)*n_ptr : n_host;
-    int64_t wbase = blockIdx.x * (int64_t)SCAN_BLOCK + (int64_t)(threadIdx.x >> 6) * (64 * SCAN_ITEMS);
-    T s = 0;
-    if (!(c && ps_poisoned(c)) && wbase < n) {
-        T v[SCAN_ITEMS];
+    __shared__ unsigned long long lds[4];
+    const int64_t wbase = blockIdx.x * (int64_t)SCAN_BLOCK + (int64_t)(threadIdx.x >> 6) * (64 * SCAN_ITEMS);
+    unsigned long long s = 0;
+    if (!ps_poisoned(c) && wbase < n) {
+        unsigned long long v[SCAN_ITEMS];
         ps_load_items(in, wbase, n, v);
 #pragma unroll
         for (int i = 0; i < SCAN_ITEMS; i++) s += v[i];
     }
-    T tot;
-    ps_block_excl_scan<T, 4>(s, lds, tot);
+    unsigned long long tot;
+    ps_block_excl_scan(s, lds, tot);
     if (threadIdx.x == 0) partial[blockIdx.x] = tot;
 }
 
 // sum of partial[0, end) over a 256-thread block
-template <typename T>
-__device__ __forceinline__ T ps_block_sum_prefix(const T* partial, int end, T* lds)
+__device__ __forceinline__ unsigned long long ps_block_sum_prefix(const unsigned long long* partial, int end,
+                                                                  unsigned long long* lds)
 {
-    T s = 0;
+    unsigned long long s = 0;
 #pragma unroll 8
     for (int i = threadIdx.x; i < end; i += 256) s += partial[i];
-    T tot;
-    ps_block_excl_scan<T, 4>(s, lds, tot);
+    unsigned long long tot;
+    ps_block_excl_scan(s, lds, tot);
     return tot;
 }
 
-// block b: prefix of the partial sums before it (partial i sums items
-// [i * pgran, (i + 1) * pgran), pgran dividing SCAN_BLOCK), then the block's
-// own scan.  Block 0 also writes the total.  With a host-side length the
-// overflow flag is tested only before the first store: the loads stay in
-// bounds either way, so its round trip overlaps theirs.
-template <typename T>
-__global__ void __launch_bounds__(256) k_scan_final(const T* __restrict__ in, const uint32_t* n_ptr, int64_t n_host,
-                                                    const T* __restrict__ partial, int nb, int pgran, T* __restrict__ out,
-                                                    uint32_t* total_out, int64_t cap, PsCounters* c,
+// block b: prefix of the partial sums before it (one per block of items),
+// then the block's own scan.  Block 0 also writes the total.  The overflow flag
+// is tested only before the first store: the loads stay in bounds either way,
+// so its round trip overlaps theirs.
+__global__ void __launch_bounds__(256) k_scan_final(const unsigned long long* __restrict__ in, int64_t n,
+                                                    const unsigned long long* __restrict__ partial, int nb,
+                                                    unsigned long long* __restrict__ out, uint32_t* total_out, PsCounters* c,
                                                     uint32_t* heavy, int* flag)
 {
-    __shared__ T lds[4];
-    const bool poisoned = c && ps_poisoned(c);
-    if (n_ptr && poisoned) return;
-    const unsigned long long pend = sizeof(T) == 8 ? ps_pend_pieces(c) : 0ull;
-    const int64_t n = n_ptr ? (int64_t)*n_ptr : n_host;
+    __shared__ unsigned long long lds[4];
+    const bool poisoned = ps_poisoned(c);
+    const unsigned long long pend = ps_pend_pieces(c);
     const int64_t wbase = blockIdx.x * (int64_t)SCAN_BLOCK + (int64_t)(threadIdx.x >> 6) * (64 * SCAN_ITEMS);
-    const bool mine = blockIdx.x * (int64_t)SCAN_BLOCK < n;
-    T v[SCAN_ITEMS];
-    if (mine) ps_load_items(in, wbase, n, v);
-    T total = 0, before = 0;
+    unsigned long long v[SCAN_ITEMS];
+    ps_load_items(in, wbase, n, v);
+    unsigned long long total = 0, before = 0;
     if (blockIdx.x == 0) total = ps_block_sum_prefix(partial, nb, lds);
-    else if (mine) before = ps_block_sum_prefix(partial, blockIdx.x * (SCAN_BLOCK / pgran), lds);
+    else before = ps_block_sum_prefix(partial, blockIdx.x, lds);
     if (poisoned) return;
     const unsigned long long pieces = ps_wave_sum64(pend);
-    if (blockIdx.x == 0 && threadIdx.x < 64) ps_scan_total(total, n, cap, out, total_out, c, flag, pieces);
-    if (!mine) return;
-    T s = 0;
+    if (blockIdx.x == 0 && threadIdx.x < 64) ps_scan_total(total, n, out, total_out, c, flag, pieces);
+    unsigned long long s = 0;
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; i++) s += v[i];
-    T tot;
+    unsigned long long tot;
     // the waves before this one: the block scan of the lane sums, taken at lane 0
-    const T wpre = ps_block_excl_scan<T, 4>(s, lds, tot);
+    const unsigned long long wpre = ps_block_excl_scan(s, lds, tot);
     uint32_t hm = 0xffffffffu, hslot = 0xffffffffu;
-    const uint32_t hcap = (uint32_t)ps_heavy_cap(n);
-    if constexpr (sizeof(T) == 8) {
-        if (heavy) {
-            hm = ps_heavy_min(ps_pend_approx(pend), n);
-            hslot = ps_heavy_reserve(ps_heavy_count(wbase, n, v, hm), heavy);
-        }
+    if (heavy) {
+        hm = ps_heavy_min(ps_pend_approx(pend), n);
+        hslot = ps_heavy_reserve(ps_heavy_count(wbase, n, v, hm), heavy);
     }
-    ps_store_scan(out, wbase, n, v, before + ps_wave_bcast0(wpre), hm, heavy, hslot, hcap);
+    ps_store_scan(out, wbase, n, v, before + ps_readlane64(wpre, 0), hm, heavy, hslot, (uint32_t)ps_heavy_cap(n));
 }
 
 // One pass for tile counts up to SCAN_DIRECT_MAX.  Blocks of 16 waves; each
@@ -937,9 +887,9 @@ __global__ void __launch_bounds__(1024) k_scan_direct(const unsigned long long* 
     const uint32_t ha = (uint32_t)va >= hm ? 1u : 0u, hb = (uint32_t)vb >= hm ? 1u : 0u;
     // the wave's inclusive scans of its own tiles and heavy marks, and its
     // totals before the block
-    const T own = ps_wave_incl_scan_t(va + vb);
+    const T own = ps_wave_incl_scan2(va + vb);
     const uint32_t hown = ps_wave_incl_scan(ha + hb);
-    const T pre_w = ps_wave_incl_scan_t(pre);
+    const T pre_w = ps_wave_incl_scan2(pre);
     const uint32_t hpre_w = ps_wave_incl_scan(hpre);
     if (lane == 63) xw[wave] = PsDirectWave{pre_w, own, hpre_w, hown};
     __syncthreads();
@@ -970,7 +920,7 @@ __global__ void __launch_bounds__(1024) k_scan_direct(const unsigned long long* 
         out[i] = oa;
     }
     if (blockIdx.x == gridDim.x - 1 && wave == 0) {
-        ps_scan_total(before + btot, n, n, out, total_out, c, flag, ps_wave_sum64(pend));
+        ps_scan_total(before + btot, n, out, total_out, c, flag, ps_wave_sum64(pend));
         if (heavy && lane == 0) heavy[0] = hbefore + hbtot;
     }
 }
@@ -1025,13 +975,11 @@ __global__ void __launch_bounds__(1024) k_scan_parts(const uint32_t* __restrict_
 #pragma unroll
     for (int j = 0; j < 4; j++) { o[j] = r; r += v[j]; }
     // the triangle of every 64th row item: item 64b lies in item i + j's rows
-    if (bstart) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if (i + j >= n) break;
-            const int64_t b1 = min(((int64_t)o[j] + v[j] + 63) >> 6, bcap);
-            for (int64_t b = ((int64_t)o[j] + 63) >> 6; b < b1; b++) bstart[b] = (uint32_t)(i + j);
-        }
+    for (int j = 0; j < 4; j++) {
+        if (i + j >= n) break;
+        const int64_t b1 = min(((int64_t)o[j] + v[j] + 63) >> 6, bcap);
+        for (int64_t b = ((int64_t)o[j] + 63) >> 6; b < b1; b++) bstart[b] = (uint32_t)(i + j);
     }
     if (i + 4 <= n) {
         *(uint4*)(out + i) = make_uint4(o[0], o[1], o[2], o[3]);
@@ -1040,7 +988,11 @@ __global__ void __launch_bounds__(1024) k_scan_parts(const uint32_t* __restrict_
         for (int j = 0; j < 4; j++)
             if (i + j < n) out[i + j] = o[j];
     }
-    if (blockIdx.x == gridDim.x - 1 && wave == 0) ps_scan_total(before + btot, n, n, out, total_out, (PsCounters*)nullptr, nullptr);
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) {
+        out[n] = before + btot;
+        *total_out = before + btot;
+        atomicMax(total_out + 2, before + btot);
+    }
 }
 
 // Triangle of row item i: the t with row_off[t] <= i < row_off[t + 1]
@@ -2690,9 +2642,8 @@ void psk_scan_tiles(hipStream_t s, const unsigned long long* tcnt, int64_t n, un
         return;
     }
     int nb = psk_scan_blocks(n);
-    hipLaunchKernelGGL(k_scan_reduce<unsigned long long>, dim3(nb), dim3(256), 0, s, tcnt, nullptr, n, partial, c);
-    hipLaunchKernelGGL(k_scan_final<unsigned long long>, dim3(nb), dim3(256), 0, s, tcnt, nullptr, n, partial, nb,
-                       SCAN_BLOCK, tstart, total_out, n, c, heavy, flag);
+    hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(256), 0, s, tcnt, n, partial, c);
+    hipLaunchKernelGGL(k_scan_final, dim3(nb), dim3(256), 0, s, tcnt, n, partial, nb, tstart, total_out, c, heavy, flag);
 }
 
 

@@ -2291,7 +2291,7 @@ int psgpu_capture_end(psgpu_ctx* c, int* out_graph)
             bool p1[PS_N_PROGS] = {false}, p2[PS_N_PROGS] = {false};
             if ((rc = build_blob(c, cmd, b, f, T, nvs, p1, p2, npx))) return rc;
             g.flushes++;
-        } else if (cmd.type == CMD_CLEARS) {
+        } else if (cmd.type == CMD_CLEARS && cmd.fills.size() > PS_FEW_FILLS) {   // fewer are kernel arguments
             b.bytes.assign(cmd.fills.size() * sizeof(PsFill), 0);
             memcpy(b.bytes.data(), cmd.fills.data(), b.bytes.size());
         }
@@ -2371,7 +2371,7 @@ int psgpu_sync_noalloc(psgpu_ctx* c)
     std::lock_guard<std::mutex> guard(g_static_lock);
     Arena arena{base, PSGPU_STATIC_SCRATCH_BYTES};
     uint8_t* fill_dev = nullptr;
-    if (!clears.fills.empty() && !(fill_dev = arena.take_bytes(clears.fills.size() * sizeof(PsFill))))
+    if (clears.fills.size() > PS_FEW_FILLS && !(fill_dev = arena.take_bytes(clears.fills.size() * sizeof(PsFill))))
         return fail(c, PSGPU_ERR_NOMEM, "%zu clears exceed the static scratch array", clears.fills.size());
     FlushShape sh = flush_shape(c, flush);
     FlushBufs sb;
@@ -2402,9 +2402,9 @@ int psgpu_sync_noalloc(psgpu_ctx* c)
     if (fill_dev) {
         hipError_t e = hipMemcpyAsync(fill_dev, clears.fills.data(), clears.fills.size() * sizeof(PsFill),
                                       hipMemcpyHostToDevice, c->stream);
-        rc = e != hipSuccess ? fail(c, PSGPU_ERR_DEVICE, "hipMemcpyAsync: %s", hipGetErrorString(e))
-                             : run_clears(c, clears, fill_dev);
+        if (e != hipSuccess) rc = fail(c, PSGPU_ERR_DEVICE, "hipMemcpyAsync: %s", hipGetErrorString(e));
     }
+    if (!rc) rc = run_clears(c, clears, fill_dev);
     // the tile counts start at zero (the array may have held anything)
     if (!rc && blob_dev) {
         hipError_t e = hipMemsetAsync(c->fb.tcnt.p, 0, c->fb.tcnt.cap * sizeof(unsigned long long), c->stream);

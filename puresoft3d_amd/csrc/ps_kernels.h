@@ -19,26 +19,29 @@ void psk_setup(hipStream_t s, int prog, bool share, const PsDraw* draws, int nd,
 int psk_scan_blocks(int64_t cap);
 // exclusive scan of the row counts from given partial sums of pgran items
 // each (pgran divides 4096); out[n] and *total_out receive the total, and
-// bstart (bcap entries) the triangle of every 64th row item; empties the list `wide`
+// bstart (bcap entries) the triangle of every 64th row item; empties the lists `wide`
 void psk_scan_parts(hipStream_t s, const uint32_t* in, int64_t n, uint32_t* out, const uint32_t* parts, int pgran,
-                    uint32_t* total_out, uint32_t* bstart, int64_t bcap, uint32_t* wide);
+                    uint32_t* total_out, uint32_t* bstart, int64_t bcap, unsigned long long* wide);
 // exclusive scan of the per-tile counts (pieces | runs << 32) into tstart
 // (n + 1 entries); the piece total into *total_out, its running maximum at
 // total_out[2]
-// flag: the host's word for the command (pinned), set where the kernel finds an overflow
+// flag: the host's word for the command (pinned), set where the kernel finds an overflow;
+// more than seg_cap pieces are one
 // heavy (optional, 1 + psk_heavy_cap() words): the heavy-tile list of PsFrame.heavy
 int psk_heavy_cap();
 void psk_scan_tiles(hipStream_t s, const unsigned long long* tcnt, int64_t n, unsigned long long* tstart,
-                    unsigned long long* partial, uint32_t* total_out, PsCounters* c, uint32_t* heavy, int* flag);
+                    unsigned long long* partial, uint32_t* total_out, unsigned long long* wide, int64_t seg_cap, PsCounters* c,
+                    uint32_t* heavy, int* flag);
 // spans of every row item; tcnt[t] += the pieces in tile t | their runs << 32; wide: the
-// waves of 64 items that hold a wide span ([0] = how many)
+// lists of the waves of 64 items that hold a wide span (PS_WIDE_LISTS), whose pieces tcnt
+// does not count
 void psk_span(hipStream_t s, const PsTri* tris, const uint32_t* row_off, const uint32_t* bstart, int64_t T,
               PsSpan* spans, unsigned long long* tcnt, const PsView* views, int n_views, int chunk_w, int tile_rows,
-              int64_t cap, uint32_t* heavy, uint32_t* wide, PsCounters* cnt, int* flag);
+              int64_t cap, uint32_t* heavy, unsigned long long* wide, PsCounters* cnt, int* flag);
 // the pieces, into runs of the tile lists f.tstart / f.runs; counts tcnt back down to zero.
 void psk_segments(hipStream_t s, const PsSpan* spans, const uint32_t* row_off, int64_t T, const PsFrame& f,
                   const PsTri* tris, const PsDraw* draws, const float* vary, int nvs, unsigned long long* tcnt, PsSeg* segs,
-                  float* ck, int64_t span_cap, int64_t seg_cap, const uint32_t* wide, PsCounters* cnt, int* flag);
+                  float* ck, int64_t span_cap, int64_t seg_cap, const unsigned long long* wide, PsCounters* cnt, int* flag);
 size_t psk_raster_lds(int chunk_w, int waves);
 void psk_raster(hipStream_t s, bool debug, const PsSpan* spans, const PsSeg* segs, const PsTri* tris, const PsDraw* draws,
                 const PsFrame& f, int waves_per_group, PsCounters* cnt);

@@ -186,6 +186,27 @@ __device__ __forceinline__ uint32_t ps_wave_incl_scan(uint32_t v)
     return v;
 }
 
+// keeps the compiler from moving LDS accesses across: the LDS operations of a
+// wave are performed in order
+__device__ __forceinline__ void ps_lds_turn()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// inclusive scan over each group of G (16 or 32) lanes
+template <int G>
+__device__ __forceinline__ uint32_t ps_group_incl_scan(uint32_t v)
+{
+    v += PS_DPP(v, 0x111, 0xf, true);
+    v += PS_DPP(v, 0x112, 0xf, true);
+    v += PS_DPP(v, 0x114, 0xf, true);
+    v += PS_DPP(v, 0x118, 0xf, true);
+    if constexpr (G == 32) v += PS_DPP(v, 0x142, 0xa, false);
+    return v;
+}
+
 // a wave's statistic (lane values whose wave total fits 32 bits, every lane
 // active): into the committed counters (pending = false) or the flush's
 // pending ones; one atomic per wave, on a per-block stripe
@@ -606,7 +627,7 @@ __global__ void __launch_bounds__(128, 3) k_setup(const PsDraw* __restrict__ dra
 __host__ __device__ __forceinline__ int64_t ps_heavy_cap(int64_t n) { return n / 3 + 1 < PS_HEAVY_MAX ? n / 3 + 1 : PS_HEAVY_MAX; }
 
 // Pieces that make a tile heavy: three times the flush's mean per tile (at
-// least 96).  The flush's pieces are k_span's 64-bit count in the pending
+// least 96), not counting those of waves that hold a wide span (k_span).  The flush's pieces are k_span's 64-bit count in the pending
 // statistics: ps_pend_pieces loads one stripe per lane,
 // ps_wave_sum64 adds the wave's stripes.
 __device__ __forceinline__ unsigned long long ps_pend_pieces(const PsCounters* c)
@@ -731,10 +752,10 @@ __device__ __forceinline__ void ps_store_scan(unsigned long long* out, int64_t w
     const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int g = 0; g < SCAN_ITEMS / 2; g++) {
-        const unsigned long long sum = v[g * 2] + v[g * 2 + 1];
+        const unsigned long long v1 = v[g * 2 + 1], sum = v[g * 2] + v1;
         const unsigned long long x = ps_wave_incl_scan2(sum);
         const int64_t i = wbase + (int64_t)g * 128 + lane * 2;
-        unsigned long long o[2] = {run + x - sum, run + x - v[g * 2 + 1]};
+        unsigned long long o[2] = {run + x - sum, run + x - v1};
 #pragma unroll
         for (int j = 0; j < 2; j++)
             if (hslot != 0xffffffffu && i + j < n && (uint32_t)v[g * 2 + j] >= heavy_min) {
@@ -750,21 +771,35 @@ __device__ __forceinline__ void ps_store_scan(unsigned long long* out, int64_t w
     }
 }
 
-// The tile scan adds 32-bit piece counts: when the flush's pieces, which
-// k_span also counts in 64 bits into the pending statistics, do not fit, it
-// reports the largest total and flags an overflow, so that the flush is
-// split.  Called by the 64 lanes of one wave.
-__device__ __forceinline__ void ps_scan_total(unsigned long long tot, int64_t n, unsigned long long* out, uint32_t* total_out,
-                                              PsCounters* c, int* flag, unsigned long long pieces)
+// the head of list `lane` of the wide waves
+__device__ __forceinline__ unsigned long long ps_wide_head(const unsigned long long* wide)
 {
-    if ((threadIdx.x & 63) != 0) return;
+    static_assert(PS_WIDE_LISTS == 64, "one list per lane");
+    return wide[PS_WIDE_STEP * (threadIdx.x & 63)];
+}
+
+// The tile scan adds 32-bit piece counts: when the flush's pieces, which k_span
+// also counts in 64 bits into the pending statistics, do not fit, it reports
+// the largest total and flags an overflow, so that the flush is split; so it
+// does when they are more than seg_cap.  Called by the 64 lanes of one wave;
+// head: the lane's of the wide lists.
+__device__ __forceinline__ void ps_scan_total(unsigned long long tot, int64_t n, unsigned long long* out, uint32_t* total_out,
+                                              unsigned long long head, unsigned long long* wide, int64_t seg_cap, PsCounters* c,
+                                              int* flag, unsigned long long pieces)
+{
+    const int lane = threadIdx.x & 63;
+    const uint32_t waves = (uint32_t)(head & PS_WIDE_COUNT), mine = (uint32_t)(head >> 20);
+    const uint32_t w = ps_wave_incl_scan(waves), p = ps_wave_incl_scan(mine);
+    wide[PS_WIDE_BEFORE + lane] = (unsigned long long)(w - waves) | (unsigned long long)(p - mine) << 32;
+    if (lane == 63) wide[PS_WIDE_BEFORE + 64] = (unsigned long long)w | (unsigned long long)p << 32;
+    if (lane != 63) return;
     out[n] = tot;
-    *total_out = (uint32_t)tot;
-    atomicMax(total_out + 2, (uint32_t)tot);
-    if (pieces != (uint32_t)tot) {
-        atomicMax(total_out + 2, 0xffffffffu);
-        ps_overflow(c, 1, flag);
-    }
+    // (a sum that wrapped has more than 2^32 pieces)
+    const bool fits = pieces == (unsigned long long)(uint32_t)tot + p && pieces <= 0xffffffffull;
+    const uint32_t total = fits ? (uint32_t)pieces : 0xffffffffu;
+    *total_out = total;
+    atomicMax(total_out + 2, total);
+    if (!fits || (int64_t)pieces > seg_cap) ps_overflow(c, 1, flag);
 }
 
 __global__ void __launch_bounds__(256) k_scan_reduce(const unsigned long long* __restrict__ in, int64_t n,
@@ -802,12 +837,15 @@ __device__ __forceinline__ unsigned long long ps_block_sum_prefix(const unsigned
 // so its round trip overlaps theirs.
 __global__ void __launch_bounds__(256) k_scan_final(const unsigned long long* __restrict__ in, int64_t n,
                                                     const unsigned long long* __restrict__ partial, int nb,
-                                                    unsigned long long* __restrict__ out, uint32_t* total_out, PsCounters* c,
-                                                    uint32_t* heavy, int* flag)
+                                                    unsigned long long* __restrict__ out, uint32_t* total_out,
+                                                    unsigned long long* wide, int64_t seg_cap, PsCounters* c, uint32_t* heavy,
+                                                    int* flag)
 {
     __shared__ unsigned long long lds[4];
     const bool poisoned = ps_poisoned(c);
     const unsigned long long pend = ps_pend_pieces(c);
+    const bool totals = blockIdx.x == 0 && threadIdx.x < 64;   // the wave that writes them
+    const unsigned long long head = totals ? ps_wide_head(wide) : 0ull;
     const int64_t wbase = blockIdx.x * (int64_t)SCAN_BLOCK + (int64_t)(threadIdx.x >> 6) * (64 * SCAN_ITEMS);
     unsigned long long v[SCAN_ITEMS];
     ps_load_items(in, wbase, n, v);
@@ -816,7 +854,7 @@ __global__ void __launch_bounds__(256) k_scan_final(const unsigned long long* __
     else before = ps_block_sum_prefix(partial, blockIdx.x, lds);
     if (poisoned) return;
     const unsigned long long pieces = ps_wave_sum64(pend);
-    if (blockIdx.x == 0 && threadIdx.x < 64) ps_scan_total(total, n, out, total_out, c, flag, pieces);
+    if (totals) ps_scan_total(total, n, out, total_out, head, wide, seg_cap, c, flag, pieces);
     unsigned long long s = 0;
 #pragma unroll
     for (int i = 0; i < SCAN_ITEMS; i++) s += v[i];
@@ -847,7 +885,8 @@ struct PsDirectWave {
 };
 __global__ void __launch_bounds__(1024) k_scan_direct(const unsigned long long* __restrict__ in, int64_t n,
                                                       unsigned long long* __restrict__ out, uint32_t* total_out,
-                                                      PsCounters* c, uint32_t* heavy, int* flag)
+                                                      unsigned long long* wide, int64_t seg_cap, PsCounters* c,
+                                                      uint32_t* heavy, int* flag)
 {
     typedef unsigned long long T;
     __shared__ PsDirectWave xw[16];
@@ -869,6 +908,8 @@ __global__ void __launch_bounds__(1024) k_scan_direct(const unsigned long long* 
     };
     if (nk > 0) chunk_load(0);
     const unsigned long long pend = ps_pend_pieces(c);   // after the loads: one wait covers them all
+    const bool totals = blockIdx.x == gridDim.x - 1 && wave == 0;   // the wave that writes them
+    const unsigned long long head = totals ? ps_wide_head(wide) : 0ull;
     const uint32_t hm = heavy ? ps_heavy_min(ps_pend_approx(pend), n) : 0xffffffffu;
     T pre = 0;
     uint32_t hpre = 0;
@@ -919,8 +960,8 @@ __global__ void __launch_bounds__(1024) k_scan_direct(const unsigned long long* 
     } else if (i < n) {
         out[i] = oa;
     }
-    if (blockIdx.x == gridDim.x - 1 && wave == 0) {
-        ps_scan_total(before + btot, n, out, total_out, c, flag, ps_wave_sum64(pend));
+    if (totals) {
+        ps_scan_total(before + btot, n, out, total_out, head, wide, seg_cap, c, flag, ps_wave_sum64(pend));
         if (heavy && lane == 0) heavy[0] = hbefore + hbtot;
     }
 }
@@ -937,10 +978,10 @@ struct PsRowWave {
 __global__ void __launch_bounds__(1024) k_scan_parts(const uint32_t* __restrict__ in, int64_t n,
                                                      const uint32_t* __restrict__ partial, int pgran,
                                                      uint32_t* __restrict__ out, uint32_t* total_out,
-                                                     uint32_t* __restrict__ bstart, int64_t bcap, uint32_t* wide)
+                                                     uint32_t* __restrict__ bstart, int64_t bcap, unsigned long long* wide)
 {
     __shared__ PsRowWave xw[16];
-    if (blockIdx.x == 0 && threadIdx.x == 0) wide[0] = 0;   // k_span's list of waves with wide spans
+    if (blockIdx.x == 0 && threadIdx.x < PS_WIDE_LISTS) wide[PS_WIDE_STEP * threadIdx.x] = 0;   // for k_span
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t i = blockIdx.x * (int64_t)SCAN_BLOCK + 4 * (int64_t)threadIdx.x;   // items i .. i + 3
     uint32_t v[4];
@@ -1057,30 +1098,31 @@ __device__ __forceinline__ int ps_row_tri(const uint32_t* __restrict__ row_off, 
 __device__ __forceinline__ bool ps_span_has_ck(const PsSpan& sp) { return sp.x2 - sp.x1 + 1 >= PS_CK_MIN; }
 
 #define SPAN_BINS 512
-// A wave of span items whose longest span has at least this many pixels gives
-// each of its spans runs of its own, which k_segments then places span by span
-// with a lane per accumulator instead of a span per lane.
+// The spans of a wave of span items whose longest has at least this many pixels
+// are placed by k_segments span by span, with a lane per accumulator instead of
+// a span per lane.
 // This is also where spans start to keep varying checkpoints, so only those
 // waves carry varyings (24 to 96 measure alike; below 40 a small sphere's
 // frame, whose spans are mostly that long, loses 3 us).
 #define PS_WIDE_MIN PS_CK_MIN
+#define PS_TC_RUN (1ull << 32)
 // called by every lane of the wave; n: the lane's span's pixels, if it has one
-__device__ __forceinline__ bool ps_wave_own_runs(bool has, uint32_t n) { return __any(has && n >= PS_WIDE_MIN); }
+__device__ __forceinline__ bool ps_wave_wide(bool has, uint32_t n) { return __any(has && n >= PS_WIDE_MIN); }
 
-// Also counts, per tile, the span pieces in it and their runs: tcnt[t] +=
-// pieces | runs << 32.  A run holds a wave's (of 64 span items) pieces there,
-// or, in the waves that hold a wide span, one span's; those waves go on the
-// list `wide` ([0] = how many).  Eight
-// waves per SIMD (64 VGPRs, no spill): at seven the 256-view batch's span
+// Also counts, per tile, the pieces in it and the waves (of 64 span items) that
+// have some there, each of which writes them as one run: tcnt[t] += pieces |
+// waves << 32.  Waves that hold a wide span count their runs only
+// and go on the lists `wide`; their pieces lie after those of all other waves.
+// Eight waves per SIMD (64 VGPRs, no spill): at seven the 256-view batch's span
 // pass took 1.55 ms instead of 1.21.
 __global__ void __launch_bounds__(256, 8) k_span(const PsTri* __restrict__ tris,
                                               const uint32_t* __restrict__ row_off, const uint32_t* __restrict__ bstart,
                                               int64_t T, int64_t cap,
                                               PsSpan* __restrict__ spans, unsigned long long* __restrict__ tcnt,
                                               const PsView* __restrict__ views, int n_views, int chunk_w, int tile_rows,
-                                              int tile_cols, uint32_t* heavy, uint32_t* wide, PsCounters* cnt, int* flag)
+                                              int tile_cols, uint32_t* heavy, unsigned long long* wide, PsCounters* cnt, int* flag)
 {
-    // per wave: pieces | runs << 16 of the tiles [kmin, kmin + SPAN_BINS) its spans touch
+    // per wave: piece counts of the tiles [kmin, kmin + SPAN_BINS) its spans touch
     __shared__ uint32_t bins_all[4][SPAN_BINS];
     uint32_t* bins = bins_all[threadIdx.x >> 6];
     const int lane = threadIdx.x & (PS_WAVE - 1);
@@ -1139,17 +1181,28 @@ __global__ void __launch_bounds__(256, 8) k_span(const PsTri* __restrict__ tris,
             }
             spans[i] = sp;
         }
+        const uint32_t npieces = has ? (uint32_t)(st.cx1 - st.cx0 + 1) : 0u;
+        all_spans += nspan;
+        all_pieces += npieces;
+        all_frags += nfrag;
+        const bool in_wide = ps_wave_wide(has, nfrag);
+        if (in_wide) {
+            const uint32_t n = __builtin_amdgcn_readlane(ps_wave_incl_scan(npieces), 63);
+            if (lane == 0) {
+                const uint32_t w = (uint32_t)(i0 >> 6), l = w % PS_WIDE_LISTS;
+                const unsigned long long old = atomicAdd(wide + PS_WIDE_STEP * l, (unsigned long long)n << 20 | 1ull);
+                wide[PS_WIDE_REC + PS_WIDE_PER(cap) * l + (int64_t)(old & PS_WIDE_COUNT)] = w | (old >> 20) << 32;
+            }
+        }
         // per tile of the wave's spans: its pieces there and one run.  When
         // the wave's tiles lie within SPAN_BINS of each other (about nine
         // tiles of one or two tile rows, typically), the lanes add their
         // pieces into LDS bins and one atomic per touched bin follows;
         // otherwise the wave visits its tiles in rounds (lane j adds the
-        // j-th tile's counts, so a batch of tiles is one atomic).
-        const uint32_t npieces = has ? (uint32_t)(st.cx1 - st.cx0 + 1) : 0u;
+        // j-th tile's counts, so a batch of tiles is one atomic), or, if it
+        // holds a wide span, the first span in a tile counts the run.
         const uint32_t kmin = ps_wave_min(has ? st.g0 : 0xffffffffu);
         const uint32_t kmax = ps_wave_max(has ? st.g1 : 0u);
-        const bool own = ps_wave_own_runs(has, nfrag);
-        if (own && lane == 0) wide[1 + atomicAdd(wide, 1u)] = (uint32_t)(i0 >> 6);
         if (kmin != 0xffffffffu && kmax - kmin < (uint32_t)SPAN_BINS) {
             const uint32_t nbin = kmax - kmin + 1;
             for (uint32_t b = lane; b < nbin; b += PS_WAVE) bins[b] = 0;
@@ -1160,38 +1213,58 @@ __global__ void __launch_bounds__(256, 8) k_span(const PsTri* __restrict__ tris,
                 for (uint32_t k = st.g0; k <= st.g1; k++) {
                     int lo, hi;
                     ps_span_tile_chunks(st, tile_cols, k, lo, hi);
-                    atomicAdd(&bins[k - kmin], (uint32_t)(hi - lo + 1) + (own ? 1u << 16 : 0u));
+                    atomicAdd(&bins[k - kmin], (uint32_t)(hi - lo + 1));
                 }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             for (uint32_t b = lane; b < nbin; b += PS_WAVE) {
                 const uint32_t c = bins[b];
-                if (c) atomicAdd(&tcnt[kmin + b], (unsigned long long)(c & 0xffffu) | (unsigned long long)(own ? c >> 16 : 1u) << 32);
+                if (c) atomicAdd(&tcnt[kmin + b], in_wide ? PS_TC_RUN : (unsigned long long)c | PS_TC_RUN);
             }
             // the next iteration clears the bins only after every lane read them
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        } else if (own) {
-            if (has)
-                for (uint32_t k = st.g0; k <= st.g1; k++) {
-                    int lo, hi;
-                    ps_span_tile_chunks(st, tile_cols, k, lo, hi);
-                    atomicAdd(&tcnt[k], (unsigned long long)(hi - lo + 1) | (1ull << 32));
+        } else if (in_wide) {
+            // 32 of a span's tiles at a time, without those that the spans
+            // before it in the same tile row cover.  (In rounds a wave across
+            // a 1080p screen makes 540: 68 us for two triangles, now 13.)
+            int ln = lane;
+            asm volatile("" : "+v"(ln));   // nothing of this is kept in registers outside
+            uint64_t before = 0;
+            for (uint64_t todo = __ballot(has); todo;) {
+                const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)(st.g0 - (uint32_t)st.tx0), __builtin_ctzll(todo));
+                const uint64_t m = __ballot(has && st.g0 - (uint32_t)st.tx0 == r);
+                if ((m >> ln) & 1ull) before = m & ((1ull << ln) - 1ull);
+                todo &= ~m;
+            }
+            const int most = (int)ps_wave_max((uint32_t)__popcll(before));
+            const int nt = has ? (int)(st.g1 - st.g0) + 1 : 0, tiles = (int)ps_wave_max((uint32_t)nt);
+            const uint32_t cols = (uint32_t)st.tx0 | (uint32_t)(st.tx0 + nt - 1) << 16;   // below 2^16 each
+            for (int q0 = 0; q0 < tiles; q0 += 32) {
+                uint32_t bits = nt - q0 >= 32 ? ~0u : nt > q0 ? (1u << (nt - q0)) - 1u : 0u;
+                uint64_t m = before;
+                for (int k = 0; k < most; k++) {   // the same for every lane: all of them are read
+                    const uint32_t c = (uint32_t)__shfl((int)cols, m ? __builtin_ctzll(m) : lane, PS_WAVE);
+                    const int lo = (int)(c & 0xffffu) - st.tx0 - q0, hi = (int)(c >> 16) - st.tx0 - q0;
+                    if (m && lo < 32 && hi >= 0) bits &= ~((~0u << max(lo, 0)) & (~0u >> (31 - min(hi, 31))));
+                    m &= m - 1ull;
                 }
+                while (bits) {
+                    atomicAdd(&tcnt[st.g0 + (uint32_t)(q0 + __builtin_ctz(bits))], PS_TC_RUN);
+                    bits &= bits - 1u;
+                }
+            }
         } else {
             uint32_t cur = has ? st.g0 : 0xffffffffu;
             for (;;) {
                 uint32_t bk, bn;
                 const int nb = ps_wave_tile_batch(st, tile_cols, cur, bk, bn);
-                if (lane < nb) atomicAdd(&tcnt[bk], (unsigned long long)bn | (1ull << 32));
+                if (lane < nb) atomicAdd(&tcnt[bk], (unsigned long long)bn | PS_TC_RUN);
                 if (nb < PS_WAVE) break;
             }
         }
-        all_spans += nspan;
-        all_pieces += npieces;
-        all_frags += nfrag;
     }
     ps_wave_add(cnt, PS_ST_SPANS, all_spans, true);
     ps_wave_add(cnt, PS_ST_SEGS, all_pieces, true);
@@ -1214,25 +1287,36 @@ __global__ void __launch_bounds__(256, 8) k_span(const PsTri* __restrict__ tris,
 // of the batch's tiles into their slots; a span's tiles are consecutive in
 // the visit order, so each walk goes on from tile to tile.
 #define SG_BATCH 16
-// Reserves the run of n pieces of tile k (counting its counter down from
-// k_span's count) and writes its record; returns its first piece.  The counts
-// k_span left must cover the run (they always do: both kernels visit the same
-// tiles); 0xffffffff, and the flag set, if they do not: never write outside.
-__device__ __forceinline__ uint32_t ps_reserve_run(const PsFrame& f, unsigned long long* tcnt, uint32_t k, uint32_t n,
-                                                   uint32_t mark, uint32_t key, int64_t cap, PsCounters* cnt, int* flag)
+// The record of a run of n pieces from `first` on, the one that a tile with
+// `left` runs still to take and runs up to `end` takes; false if it has none
+// left or the pieces lie outside.
+__device__ __forceinline__ bool ps_put_run(const PsFrame& f, uint32_t left, unsigned long long end, uint32_t first, uint32_t n,
+                                           uint32_t wave_id, int64_t cap)
 {
-    const unsigned long long take = (unsigned long long)n | (1ull << 32);
-    const unsigned long long left = atomicAdd(&tcnt[k], (unsigned long long)0 - take);
+    if (left == 0u || (uint64_t)first + n > (uint64_t)cap) return false;
+    *(uint2*)(f.runs + 2 * (size_t)((uint32_t)(end >> 32) - left)) = make_uint2(first, wave_id << 12 | (n - 1u));
+    return true;
+}
+
+// Takes a run of n pieces of tile k off the tile's counter and writes its
+// record.  The tile's pieces that k_span counted are those of its runs in the
+// order they are taken; returns the run's first.  The counts must cover the run
+// (they always do: both kernels visit the same tiles); 0xffffffff, and the
+// flag set, if they do not: never write outside.
+__device__ __forceinline__ uint32_t ps_take_run(const PsFrame& f, unsigned long long* tcnt, uint32_t k, uint32_t n,
+                                                uint32_t wave_id, int64_t cap, PsCounters* cnt, int* flag)
+{
+    const unsigned long long left = atomicAdd(&tcnt[k], 0ull - (n | PS_TC_RUN));
     const unsigned long long end = PS_TS(f.tstart[k + 1]);
-    const uint32_t fp = (uint32_t)end - (uint32_t)left;
+    const uint32_t first = (uint32_t)end - (uint32_t)left;
     const uint32_t slot = (uint32_t)(end >> 32) - (uint32_t)(left >> 32);
-    if ((uint32_t)left < n || (uint32_t)(left >> 32) == 0u || (uint64_t)fp + n > (uint64_t)cap) {
+    if ((uint32_t)left < n || (uint32_t)(left >> 32) == 0u || (uint64_t)first + n > (uint64_t)cap) {
         ps_overflow(cnt, 2, flag);
         return 0xffffffffu;
     }
-    f.runs[2 * (size_t)slot] = fp | mark;
-    f.runs[2 * (size_t)slot + 1] = key | (n - 1u);
-    return fp;
+    f.runs[2 * (size_t)slot] = first;  // two stores: as one, 123 us where this takes 119 (32 views)
+    f.runs[2 * (size_t)slot + 1] = wave_id << 12 | (n - 1u);
+    return first;
 }
 
 // Spans of the listed waves (those that hold a wide span): G (16 or 32) lanes
@@ -1242,50 +1326,71 @@ __device__ __forceinline__ uint32_t ps_reserve_run(const PsFrame& f, unsigned lo
 // 22 accumulators a pixel while the lanes whose spans lie in other tile rows
 // waited: 24 objects and a full-view quad at 1366x768 took 2,830 us, now 38
 // (1920x1080 terrain with spans of over 1,000 pixels, 8-pixel tiles: 93 -> 33);
-// what is left is the chain of a span's loads, reservations and adds.
+// what is left is the chain of a span's loads and adds.
 // Lane j of the group holds word j of the span's piece records (PsSeg: 2 is
 // cf2, 3 the depth numerator) and, from 8 on, varying j - 8, so a piece is one
-// store.  The group first places the span's pieces, one run per tile: its
-// lanes reserve as many tiles at once.
+// store.
+// A wave's pieces of a tile are one run here too, although its spans are
+// placed by waves that know nothing of each other: a listed wave's pieces are
+// one block (its first piece is on the list), ordered by tile row, tile and
+// span, so that the place of each follows from the chunks that the wave's 64
+// spans cover, one per lane.  The first span in a tile writes the run's record.
+// (A run for each span, placed among the tile's own pieces, made eight of one,
+// and sorting them was most of the raster kernel: 48 triangle pairs across
+// 1920x1080 1,514 us there, now 279; frames of 4,000 triangles of 60 to 240
+// pixels 1,150 -> 647, of 200,000 small ones with each fifth 60 pixels wide
+// 3,470 -> 1,580.)
 template <int G>
 __device__ __forceinline__ void ps_wide_spans(const PsSpan* __restrict__ spans, int64_t R, const PsFrame& f,
                                               const PsTri* __restrict__ tris, const PsDraw* __restrict__ draws,
-                                              const float* __restrict__ vary, int nvs, const uint32_t* __restrict__ wide,
-                                              unsigned long long* __restrict__ tcnt, PsSeg* __restrict__ segs,
-                                              float* __restrict__ ck, int64_t cap, PsCounters* cnt, int* flag)
+                                              const float* __restrict__ vary, int nvs, const unsigned long long* __restrict__ wide,
+                                              int64_t wide_per, uint32_t listed, uint32_t narrow, int64_t tb1,
+                                              int ntx1, unsigned long long* __restrict__ tcnt, PsSeg* __restrict__ segs,
+                                              float* __restrict__ ck, int64_t cap, uint32_t* lds, PsCounters* cnt, int* flag)
 {
     constexpr int SPW = 64 / G;
+    static_assert(SPW * (G + 1) <= 4 * PS_WAVE && 6 * PS_WAVE <= SG_BATCH * PS_WAVE, "the wave's LDS");
     const int lane = threadIdx.x & (PS_WAVE - 1), j = lane & (G - 1), grp = lane & ~(G - 1);
-    const int CW = f.chunk_w, TC = f.tile_cols;
-    const uint32_t units = wide[0] * G, stride = gridDim.x * (blockDim.x / PS_WAVE);
-    for (uint32_t u = blockIdx.x * (blockDim.x / PS_WAVE) + threadIdx.x / PS_WAVE; u < units; u += stride) {
-        const uint32_t wave_id = wide[1 + u / G], in_wave = (u % G) * SPW + (uint32_t)grp / G;
-        const int64_t i = (int64_t)wave_id * PS_WAVE + in_wave;
-        PsSpan sp;
+    const int CW = f.chunk_w, TC = f.tile_cols, cw_shift = __builtin_ctz((unsigned)CW), tc_shift = __builtin_ctz((unsigned)TC);
+    // what is before list `lane` waits in LDS, out of the registers
+    uint2* before_list = (uint2*)(lds + PS_WAVE * 4);
+    before_list[lane] = *(const uint2*)(wide + PS_WIDE_BEFORE + lane);
+    const uint32_t units = listed * G;
+    // the first unit goes to the first wave that has fewer items than the one
+    // before it (or none), when the rest of the kernel deals them out
+    const uint32_t stride = gridDim.x * (blockDim.x / PS_WAVE), less = (uint32_t)((R + PS_WAVE - 1) / PS_WAVE) % stride;
+    const uint32_t id = blockIdx.x * (blockDim.x / PS_WAVE) + threadIdx.x / PS_WAVE;
+    for (uint32_t u = id >= less ? id - less : id + stride - less; u < units; u += stride) {
+        ps_lds_turn();
+        const uint2 bl = before_list[lane];
+        const int l = __popcll(__ballot(bl.x <= u / G)) - 1;   // the last list that begins at or before it
+        const unsigned long long rec = wide[PS_WIDE_REC + wide_per * l + (u / G - (uint32_t)__builtin_amdgcn_readlane((int)bl.x, l))];
+        const uint32_t wave_id = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)rec);
+        const uint32_t block0 = narrow + (uint32_t)__builtin_amdgcn_readlane((int)bl.y, l) +
+                                (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(rec >> 32));
+        const int sub = (int)(u % G) * SPW, in_wave = sub + grp / G;
+        const int64_t i0 = (int64_t)wave_id * PS_WAVE;
+        PsSpan sp;   // the group's span
         sp.tri = -1;
-        if (i < R) sp = spans[i];
+        if (i0 + in_wave < R) sp = spans[i0 + in_wave];
         const bool has = sp.tri >= 0;
         if (!__any(has)) continue;
-        PsSpanTiles st = {};
-        int nv = 0, nt = 0;
+        int nv = 0;
         bool need_ck = false;
         uint32_t word = 0;          // what the lane stores of each piece, where it does not change
         float v = 0.0f, step = 0.0f;
         if (has) {
             const int y = sp.y & 0xffffff;
-            const PsTri tr = tris[sp.tri];
-            const PsView& V = f.views[tr.view];
-            st = ps_span_tiles(V.tile_base, V.n_tiles_x, f.tile_rows, TC, CW, y, sp.x1, sp.x2);
-            nt = (int)(st.g1 - st.g0) + 1;
-            need_ck = st.cx1 > st.cx0 && ((sp.y >> 28) & 1) && ps_span_has_ck(sp);
+            need_ck = (sp.x2 >> cw_shift) > (sp.x1 >> cw_shift) && ((sp.y >> 28) & 1) && ps_span_has_ck(sp);
             const uint32_t flags = ((uint32_t)(sp.y >> 24) & 3u) << 26 | ((uint32_t)(sp.y >> 28) & 1u) << 28;
-            if (j == 0) word = (uint32_t)i | flags;
+            if (j == 0) word = (uint32_t)(i0 + in_wave) | flags;
             if (j == 2) { v = sp.cf2; step = sp.cf2_step; }
             if (j == 3) { v = sp.pz; step = sp.pz_step; }
             if (j == 4) word = __float_as_uint(sp.cf2_step);
             if (j == 5) word = __float_as_uint(sp.pz_step);
             if (j == 6) word = (uint32_t)y;
             if (need_ck) {
+                const PsTri tr = tris[sp.tri];
                 const PsDraw& d = draws[tr.code >> 8];
                 nv = d.nv;
                 PsEdge L, Rr;
@@ -1300,31 +1405,108 @@ __device__ __forceinline__ void ps_wide_spans(const PsSpan* __restrict__ spans, 
                 }
             }
         }
+        // the listed wave's spans, one per lane: first tile of the tile row
+        // (0xffffffff: no span) and chunks, cx0 | cx1 + 1 << 16
+        uint32_t row = 0xffffffffu, chunks = 0;
+        {
+            int ln = lane;
+            asm volatile("" : "+v"(ln));   // or its address is kept in registers all along
+            PsSpan one;
+            one.tri = -1;
+            if (i0 + ln < R) one = spans[i0 + ln];
+            int64_t vtb = tb1;
+            int vntx = ntx1;
+            if (f.n_views != 1) {
+                // triangles come view by view: one view if the first and the
+                // last have the same
+                const uint64_t m = __ballot(one.tri >= 0);
+                const int va = tris[__builtin_amdgcn_readlane(one.tri, __builtin_ctzll(m))].view;
+                const int vb = tris[__builtin_amdgcn_readlane(one.tri, 63 - __builtin_clzll(m))].view;
+                const PsView& V = f.views[va == vb || one.tri < 0 ? va : tris[one.tri].view];
+                vtb = V.tile_base;
+                vntx = V.n_tiles_x;
+            }
+            if (one.tri >= 0) {
+                const PsSpanTiles st = ps_span_tiles(vtb, vntx, f.tile_rows, TC, CW, one.y & 0xffffff, one.x1, one.x2);
+                row = st.g0 - (uint32_t)st.tx0;
+                chunks = (uint32_t)st.cx0 | (uint32_t)(st.cx1 + 1) << 16;
+            }
+        }
+        const uint32_t np = (chunks >> 16) - (chunks & 0xffffu);
+        // of the group's span: its tile row, and the first piece there
+        uint32_t seg0 = 0, row0 = 0;
+#pragma unroll
+        for (int k = 0; k < SPW; k++) {
+            const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)row, sub + k);
+            const uint32_t before = (uint32_t)__builtin_amdgcn_readlane((int)ps_wave_incl_scan(row < r ? np : 0u), 63);
+            if (grp == k * G) {
+                seg0 = block0 + before;
+                row0 = r;
+            }
+        }
+        PsSpanTiles st = {};
+        int nt = 0;
+        if (has) {
+            st = ps_span_tiles(row0, 0, f.tile_rows, TC, CW, 0, sp.x1, sp.x2);
+            nt = (int)(st.g1 - st.g0) + 1;
+        }
         const bool acc = j == 2 || j == 3 || j >= 8;
         // the lane's words of consecutive pieces lie `next` words apart; a
         // whole chunk further, the pixel range and the checkpointed piece's
         // own index move by `move`
-        const int64_t next = j < 8 ? (int64_t)(sizeof(PsSeg) / 4) : f.ck_stride;
+        const int next = j < 8 ? (int)(sizeof(PsSeg) / 4) : f.ck_stride;
         const uint32_t move = j == 1 ? (uint32_t)CW * 0x10001u : (j == 7 && need_ck) ? 1u : 0u;
         const int maxnt = (int)ps_wave_max((uint32_t)nt);
         for (int q0 = 0; q0 < maxnt; q0 += G) {
-            uint32_t first = 0xffffffffu;
-            if (q0 + j < nt) {
-                const uint32_t k = st.g0 + (uint32_t)(q0 + j);
-                int lo, hi;
-                ps_span_tile_chunks(st, TC, k, lo, hi);
-                first = ps_reserve_run(f, tcnt, k, (uint32_t)(hi - lo + 1), PS_RUN_OWN, wave_id << 12 | in_wave << 6, cap, cnt, flag);
+            // Lane j: in the span's tile q0 + j, the pieces that the listed
+            // wave's spans have there, those of the spans before this one, and
+            // the first of them all.  A span's pieces per tile, from one column
+            // to the next, change at its first and last tile only, so the spans
+            // (one per lane) add four changes each for every group's tile row,
+            // all spans' in the lower half of a word and the earlier ones' in
+            // the upper (at most 4,096 pieces each), and sums along the columns
+            // give the rest.  (Span by span it was 130 cycles for each of up to
+            // 63 others.)
+            for (int i = lane; i < SPW * (G + 1); i += PS_WAVE) lds[i] = 0;
+            ps_lds_turn();
+            uint32_t first = seg0;
+#pragma unroll 1
+            for (int k = 0; k < SPW; k++) {
+                const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)row, sub + k);
+                const int w0 = __builtin_amdgcn_readlane(st.tx0, k * G) + q0;
+                const bool in_row = row == r && np != 0;
+                const int lo = (int)(chunks & 0xffffu), hi = (int)(chunks >> 16), t0 = lo >> tc_shift, t1 = (hi - 1) >> tc_shift;
+                // those before the first of these tiles
+                const uint32_t left = (uint32_t)__builtin_amdgcn_readlane(
+                    (int)ps_wave_incl_scan(in_row ? (uint32_t)(min(max(w0 * TC, lo), hi) - lo) : 0u), 63);
+                if (grp == k * G) first += left;
+                if (!in_row) continue;
+                const int nl = (t0 + 1) * TC - lo, nr = hi - t1 * TC;
+                const uint32_t both = lane < sub + k ? 0x10001u : 1u;
+                const int at[4] = {t0, t0 + 1, t1, t1 + 1}, change[4] = {nl, TC - nl, nr - TC, -nr};
+                uint32_t* row_k = lds + k * (G + 1);
+#pragma unroll
+                for (int i = 0; i < 4; i++)   // [G]: beyond these tiles
+                    atomicAdd(row_k + min(max(at[i] - w0, 0), G), (uint32_t)change[i] * both);
             }
+            ps_lds_turn();
+            const uint32_t sums = ps_group_incl_scan<G>(lds[grp / G * (G + 1) + j]), here = sums & 0xffffu, earlier = sums >> 16;
+            first += ps_group_incl_scan<G>(here) - here;
+            ps_lds_turn();
+            // the first span in a tile takes the run; its record is written after
+            // the pieces, which need not wait for the counter
+            const bool takes = q0 + j < nt && earlier == 0;
+            uint32_t left = 0;
+            if (takes) left = (uint32_t)(atomicAdd(&tcnt[st.g0 + (uint32_t)(q0 + j)], 0ull - PS_TC_RUN) >> 32);
+            first += earlier;
             for (int q = q0; q < min(q0 + G, maxnt); q++) {
                 const uint32_t s = (uint32_t)__shfl((int)first, grp + (q - q0), PS_WAVE);
                 if (q >= nt) continue;
                 int lo, hi;
                 ps_span_tile_chunks(st, TC, st.g0 + (uint32_t)q, lo, hi);
-                const bool lost = s == 0xffffffffu;   // not placed: step over the tile
-                uint32_t* at = j < 8 ? (uint32_t*)(segs + (lost ? 0u : s)) + j
-                                     : (uint32_t*)ck + (int64_t)(lost ? 0u : s) * f.ck_stride + (j - 8);
+                uint32_t* at = j < 8 ? (uint32_t*)(segs + s) + j : (uint32_t*)ck + (int64_t)s * f.ck_stride + (j - 8);
                 const bool begins = lo == st.cx0;
-                bool on = !lost && (j < 8 || (j - 8 < nv && !begins));   // the span's first piece keeps no checkpoint
+                bool on = j < 8 || (j - 8 < nv && !begins);   // the span's first piece keeps no checkpoint
                 if (j == 1) word = (uint32_t)max(sp.x1, lo * CW) | (uint32_t)min(sp.x2, lo * CW + CW - 1) << 16;
                 if (j == 7) word = need_ck && !begins ? (s | PS_SEG_CK) : (uint32_t)sp.tri;
                 int n = hi - lo + 1;
@@ -1333,16 +1515,14 @@ __device__ __forceinline__ void ps_wide_spans(const PsSpan* __restrict__ spans, 
                     const int x = (st.cx0 + 1) * CW;
                     for (int k = sp.x1; k < x; k++) v += step;
                     at += next;
-                    on = !lost && (j < 8 || j - 8 < nv);
+                    on = j < 8 || j - 8 < nv;
                     if (j == 1) word = (uint32_t)x | (uint32_t)(x + CW - 1) << 16;
                     if (j == 7 && need_ck) word = (s + 1u) | PS_SEG_CK;
                     n--;
                 }
                 const bool ends = n > 0 && hi == st.cx1;
                 if (ends) n--;
-                if (lost) {
-                    for (int k = n * CW; k > 0; k--) v += step;
-                } else if (on) {   // the other lanes carry nothing
+                if (on) {   // the other lanes carry nothing
                     auto whole = [&](int adds) {
                         *at = acc ? __float_as_uint(v) : word;
                         at += next;
@@ -1368,6 +1548,8 @@ __device__ __forceinline__ void ps_wide_spans(const PsSpan* __restrict__ spans, 
                     if (on) *at = acc ? __float_as_uint(v) : word;
                 }
             }
+            if (takes && !ps_put_run(f, left, PS_TS(f.tstart[st.g0 + (uint32_t)(q0 + j) + 1]), first, here, wave_id, cap))
+                ps_overflow(cnt, 2, flag);
         }
     }
 }
@@ -1376,27 +1558,26 @@ __device__ __forceinline__ void ps_wide_spans(const PsSpan* __restrict__ spans, 
 // two accumulators: with the varyings beside them the kernel took 96 VGPRs
 // (five waves per SIMD) for 14 floats and 149 for 20.
 template <int G>
-__global__ void __launch_bounds__(256) k_segments(const PsSpan* __restrict__ spans, const uint32_t* __restrict__ row_off,
+__global__ void __launch_bounds__(256, 6) k_segments(const PsSpan* __restrict__ spans, const uint32_t* __restrict__ row_off,
                                                   int64_t T, PsFrame f, const PsTri* __restrict__ tris,
                                                   const PsDraw* __restrict__ draws, const float* __restrict__ vary, int nvs,
                                                   unsigned long long* __restrict__ tcnt, PsSeg* __restrict__ segs,
-                                                  float* __restrict__ ck, int64_t cap, const uint32_t* __restrict__ wide,
+                                                  float* __restrict__ ck, int64_t cap, const unsigned long long* __restrict__ wide, int64_t wide_per,
                                                   PsCounters* cnt, int* flag)
 {
     __shared__ uint32_t rel_all[4][SG_BATCH][PS_WAVE];   // per wave: [iteration][lane] offset in the run
     const bool poisoned = ps_poisoned(cnt);
     const int64_t R = row_off[T];
-    const int64_t S = (uint32_t)f.tstart[f.n_tiles];
-    if (poisoned) return;
-    if (S > cap) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) ps_overflow(cnt, 1, flag);
-        return;
-    }
-    ps_wide_spans<G>(spans, R, f, tris, draws, vary, nvs, wide, tcnt, segs, ck, cap, cnt, flag);
-    const int CW = f.chunk_w, TC = f.tile_cols;
+    const uint32_t narrow = (uint32_t)f.tstart[f.n_tiles];   // pieces of the waves that are not listed
+    const uint32_t listed = (uint32_t)wide[PS_WIDE_BEFORE + PS_WIDE_LISTS];
     int64_t tb1 = 0;   // the only view of a one-view flush, read once
     int ntx1 = 0;
     if (f.n_views == 1) { tb1 = f.views[0].tile_base; ntx1 = f.views[0].n_tiles_x; }
+    if (poisoned) return;   // also if there are more pieces than cap
+    if (listed)
+        ps_wide_spans<G>(spans, R, f, tris, draws, vary, nvs, wide, wide_per, listed, narrow, tb1, ntx1, tcnt, segs, ck, cap,
+                         &rel_all[threadIdx.x >> 6][0][0], cnt, flag);
+    const int CW = f.chunk_w, TC = f.tile_cols;
     const int lane = threadIdx.x & (PS_WAVE - 1);
     uint32_t (*rel)[PS_WAVE] = rel_all[threadIdx.x >> 6];
     for (int64_t base = blockIdx.x * (int64_t)blockDim.x; base < R; base += (int64_t)gridDim.x * blockDim.x) {
@@ -1406,7 +1587,7 @@ __global__ void __launch_bounds__(256) k_segments(const PsSpan* __restrict__ spa
         sp.tri = -1;
         if (i < R) sp = spans[i];
         const bool has = sp.tri >= 0;
-        if (ps_wave_own_runs(has, (uint32_t)(sp.x2 - sp.x1 + 1))) continue;   // placed above
+        if (ps_wave_wide(has, (uint32_t)(sp.x2 - sp.x1 + 1))) continue;   // placed above
         PsSpanTiles st = {};
         int y = 0;
         uint32_t flags = 0;
@@ -1452,7 +1633,7 @@ __global__ void __launch_bounds__(256) k_segments(const PsSpan* __restrict__ spa
             }
             if (nb == 0) break;
             uint32_t first = 0xffffffffu;
-            if (lane < nb) first = ps_reserve_run(f, tcnt, bk, bn, 0u, wave_id << 12, cap, cnt, flag);
+            if (lane < nb) first = ps_take_run(f, tcnt, bk, bn, wave_id, cap, cnt, flag);
             // every lane walks its pieces of the batch's tiles
             const int maxtb = __builtin_amdgcn_readfirstlane(ps_wave_max((uint32_t)ntb));
             for (int q = 0; q < maxtb; q++) {
@@ -1488,12 +1669,6 @@ __global__ void __launch_bounds__(256) k_segments(const PsSpan* __restrict__ spa
 // ---------------------------------------------------------------------------
 // tile lists: the runs of a tile in submission order
 // ---------------------------------------------------------------------------
-// pieces of a run (PsFrame.runs: first piece and mark, key)
-__device__ __forceinline__ uint32_t ps_run_count(uint32_t first, uint32_t key)
-{
-    return (key & ((first & PS_RUN_OWN) ? 0x3fu : 0xfffu)) + 1u;
-}
-
 // For each lane's keys key[0 .. Q): how many of the n keys they are compared
 // with lie below.  Those are held one per lane in `other` (lanes from n on are
 // not looked at); each is read from its lane by a constant index, so a key
@@ -1533,8 +1708,8 @@ __device__ __forceinline__ void ps_sort_lanes(uint32_t& key, uint32_t& val, uint
 // Window of up to 64 runs from run w0 on, one per lane: rbase = the run's
 // first piece, rv = the list position of that piece (0xffffffff past the last
 // run), vhi = the list position where the window ends.  A tile of at most 64
-// runs is sorted here; longer lists come ordered by ps_order_runs, with each
-// run's key replaced by its list position.
+// runs is sorted here; longer lists of n_list pieces come ordered by
+// ps_order_runs, with each run's key replaced by its list position.
 __device__ __forceinline__ void ps_run_window(const uint32_t* rl, uint32_t nr, uint32_t w0, uint32_t n_list,
                                               uint32_t& rbase, uint32_t& rv, uint32_t& vhi)
 {
@@ -1544,30 +1719,29 @@ __device__ __forceinline__ void ps_run_window(const uint32_t* rl, uint32_t nr, u
         uint32_t key = j < nr ? rl[2 * j + 1] : 0xffffffffu;
         rbase = j < nr ? rl[2 * j] : 0u;
         ps_sort_lanes(key, rbase, nw);
-        const uint32_t c = j < nr ? ps_run_count(rbase, key) : 0u;
-        rbase &= ~PS_RUN_OWN;
+        const uint32_t c = j < nr ? (key & 0xfffu) + 1u : 0u;
         const uint32_t incl = ps_wave_incl_scan(c);
         rv = j < nr ? incl - c : 0xffffffffu;
-        vhi = n_list;
+        vhi = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
     } else {
         rbase = j < nr ? rl[2 * j] : 0u;
         rv = j < nr ? rl[2 * j + 1] : 0xffffffffu;
-        vhi = w0 + 64 < nr ? rl[2 * (w0 + 64) + 1] : n_list;
+        vhi = w0 + nw < nr ? rl[2 * (w0 + nw) + 1] : n_list;
     }
 }
 
-// A tile with more than PS_LDS_RUNS runs: one wave sorts them by their keys from bit 6 up, which tell any two
-// runs of a tile apart (LSD radix, 7-bit digits above the smallest, ping-ponging
+// A tile with more than PS_LDS_RUNS runs: one wave sorts them by wave (LSD
+// radix, 7-bit digits of the wave index above the smallest, ping-ponging
 // between the tile's parts a and b of the two run arrays), then replaces each
 // run's key by the list position of its first piece.  cnt128: 128 words of
-// the wave's LDS.  Returns the array that holds the result.
-__device__ uint32_t* ps_order_runs(uint32_t* a, uint32_t* b, uint32_t nr, uint32_t* cnt128)
+// the wave's LDS.  Returns the array that holds the result; n_list: the pieces.
+__device__ uint32_t* ps_order_runs(uint32_t* a, uint32_t* b, uint32_t nr, uint32_t* cnt128, uint32_t& n_list)
 {
     const int lane = threadIdx.x & 63;
     const uint64_t lt = ps_lt_mask();
     uint32_t mn = 0xffffffffu, mx = 0;
     for (uint32_t j = lane; j < nr; j += 64) {
-        const uint32_t w = a[2 * j + 1] >> 6;
+        const uint32_t w = a[2 * j + 1] >> 12;
         mn = min(mn, w);
         mx = max(mx, w);
     }
@@ -1579,7 +1753,7 @@ __device__ uint32_t* ps_order_runs(uint32_t* a, uint32_t* b, uint32_t nr, uint32
         cnt128[lane + 64] = 0;
         __builtin_amdgcn_wave_barrier();
         for (uint32_t j = lane; j < nr; j += 64)
-            atomicAdd(&cnt128[(((a[2 * j + 1] >> 6) - mn) >> shift) & 127u], 1u);
+            atomicAdd(&cnt128[(((a[2 * j + 1] >> 12) - mn) >> shift) & 127u], 1u);
         __builtin_amdgcn_wave_barrier();
         {
             const uint32_t c0 = cnt128[2 * lane], c1 = cnt128[2 * lane + 1];
@@ -1593,7 +1767,7 @@ __device__ uint32_t* ps_order_runs(uint32_t* a, uint32_t* b, uint32_t nr, uint32
             const uint32_t j = j0 + lane;
             const bool valid = j < nr;
             const uint32_t e0 = valid ? a[2 * j] : 0u, e1 = valid ? a[2 * j + 1] : 0u;
-            const uint32_t dig = valid ? (((e1 >> 6) - mn) >> shift) & 127u : 0u;
+            const uint32_t dig = valid ? (((e1 >> 12) - mn) >> shift) & 127u : 0u;
             uint64_t same = __ballot(valid);
 #pragma unroll
             for (int bit = 0; bit < 7; bit++) {
@@ -1616,16 +1790,13 @@ __device__ uint32_t* ps_order_runs(uint32_t* a, uint32_t* b, uint32_t nr, uint32
     uint32_t carry = 0;
     for (uint32_t j0 = 0; j0 < nr; j0 += 64) {
         const uint32_t j = j0 + lane;
-        const uint32_t first = j < nr ? a[2 * j] : 0u;
-        const uint32_t c = j < nr ? ps_run_count(first, a[2 * j + 1]) : 0u;
+        const uint32_t c = j < nr ? (a[2 * j + 1] & 0xfffu) + 1u : 0u;
         const uint32_t incl = ps_wave_incl_scan(c);
-        if (j < nr) {
-            a[2 * j] = first & ~PS_RUN_OWN;
-            a[2 * j + 1] = carry + incl - c;
-        }
+        if (j < nr) a[2 * j + 1] = carry + incl - c;
         carry += __builtin_amdgcn_readlane(incl, 63);
     }
     __threadfence();
+    n_list = carry;
     return a;
 }
 
@@ -1639,21 +1810,12 @@ __device__ uint32_t* ps_order_runs(uint32_t* a, uint32_t* b, uint32_t nr, uint32
 #define PS_LDS_RUNS 256
 #define RA_PIX_WORDS(cw) (PS_LDS_RUNS * 2 + 64 + 64 * 2 + (cw) * 64 * 2)
 
-// keeps the compiler from moving LDS accesses across: the LDS operations of a
-// wave are performed in order
-__device__ __forceinline__ void ps_lds_turn()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The runs of a tile of 65 to PS_LDS_RUNS runs, sorted by wave and with each
 // key replaced by the list position of the run's first piece, into the wave's
 // LDS: every key is counted against all of them (1 us for 128 runs), where
 // sorting them in global memory takes several dependent passes over it
 // (11 to 38 us, the longest part of the tiles that end the kernel).
-__device__ __forceinline__ void ps_sort_runs_lds(const uint32_t* rl, uint32_t nr, uint2* out)
+__device__ __forceinline__ void ps_sort_runs_lds(const uint32_t* rl, uint32_t nr, uint2* out, uint32_t& n_list)
 {
     constexpr int Q = PS_LDS_RUNS / 64;
     const uint32_t lane = threadIdx.x & 63;
@@ -1671,7 +1833,7 @@ __device__ __forceinline__ void ps_sort_runs_lds(const uint32_t* rl, uint32_t nr
         if (nr > 64u * q) ps_count_below<Q>(key, key[q], min(nr - 64u * q, 64u), rank);
 #pragma unroll
     for (int q = 0; q < Q; q++)
-        if (q * 64 + lane < nr) out[rank[q]] = make_uint2(val[q] & ~PS_RUN_OWN, ps_run_count(val[q], key[q]));
+        if (q * 64 + lane < nr) out[rank[q]] = make_uint2(val[q], (key[q] & 0xfffu) + 1u);
     ps_lds_turn();
     uint32_t carry = 0;
     for (uint32_t j0 = 0; j0 < nr; j0 += 64) {
@@ -1681,6 +1843,7 @@ __device__ __forceinline__ void ps_sort_runs_lds(const uint32_t* rl, uint32_t nr
         if (j < nr) out[j].y = carry + incl - r.y;
         carry += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
     }
+    n_list = carry;
     ps_lds_turn();
 }
 
@@ -1813,12 +1976,12 @@ __global__ void __launch_bounds__(512, 5) k_raster(const PsSpan* __restrict__ sp
     const bool dclear = V.dclear != 0;
     // the tile's runs in submission order, up to 64 at a time (one per lane)
     const unsigned long long ta = PS_TS(f.tstart[tile]), tb = PS_TS(f.tstart[tile + 1]);
-    const uint32_t n_list = (uint32_t)tb - (uint32_t)ta;
     const uint32_t r0 = (uint32_t)(ta >> 32), nr = (uint32_t)(tb >> 32) - r0;
     const uint32_t* rl = f.runs + 2 * (size_t)r0;
     const bool in_lds = nr > 64 && nr <= PS_LDS_RUNS;
-    if (in_lds) ps_sort_runs_lds(rl, nr, lruns);
-    else if (nr > 64) rl = ps_order_runs(f.runs + 2 * (size_t)r0, f.runs2 + 2 * (size_t)r0, nr, (uint32_t*)lruns);
+    uint32_t n_list = 0;   // the tile's pieces, where the runs are sorted here
+    if (in_lds) ps_sort_runs_lds(rl, nr, lruns, n_list);
+    else if (nr > 64) rl = ps_order_runs(f.runs + 2 * (size_t)r0, f.runs2 + 2 * (size_t)r0, nr, (uint32_t*)lruns, n_list);
     if constexpr (KCW > 0) {
         uint32_t d[KCW];
         if (dclear) {
@@ -2065,13 +2228,13 @@ __global__ void __launch_bounds__(512) k_raster_imm(const PsSpan* __restrict__ s
     const bool dclear = V.dclear != 0;
     // the tile's runs in submission order, up to 64 at a time (one per lane)
     const unsigned long long ta = PS_TS(f.tstart[tile]), tb = PS_TS(f.tstart[tile + 1]);
-    const uint32_t n_list = (uint32_t)tb - (uint32_t)ta;
     const uint32_t r0 = (uint32_t)(ta >> 32), nr = (uint32_t)(tb >> 32) - r0;
     if (nr == 0 && !dclear) return;
     const uint32_t* rl = f.runs + 2 * (size_t)r0;
     const bool in_lds = nr > 64 && nr <= PS_LDS_RUNS;
-    if (in_lds) ps_sort_runs_lds(rl, nr, lruns);
-    else if (nr > 64) rl = ps_order_runs(f.runs + 2 * (size_t)r0, f.runs2 + 2 * (size_t)r0, nr, (uint32_t*)lruns);
+    uint32_t n_list = 0;   // the tile's pieces, where the runs are sorted here
+    if (in_lds) ps_sort_runs_lds(rl, nr, lruns, n_list);
+    else if (nr > 64) rl = ps_order_runs(f.runs + 2 * (size_t)r0, f.runs2 + 2 * (size_t)r0, nr, (uint32_t*)lruns, n_list);
     // the chunk as the flush finds it, to write back what it changes
     uint32_t d0[KCW > 0 ? KCW : 1], c0[KCW > 0 ? KCW : 1];
     if constexpr (KCW > 0) {
@@ -2625,7 +2788,7 @@ int psk_scan_blocks(int64_t cap) { return gsz(cap, SCAN_BLOCK); }
 
 
 void psk_scan_parts(hipStream_t s, const uint32_t* in, int64_t n, uint32_t* out, const uint32_t* parts, int pgran,
-                    uint32_t* total_out, uint32_t* bstart, int64_t bcap, uint32_t* wide)
+                    uint32_t* total_out, uint32_t* bstart, int64_t bcap, unsigned long long* wide)
 {
     hipLaunchKernelGGL(k_scan_parts, dim3(psk_scan_blocks(n)), dim3(1024), 0, s, in, n, parts, pgran, out, total_out,
                        bstart, bcap, wide);
@@ -2634,22 +2797,23 @@ void psk_scan_parts(hipStream_t s, const uint32_t* in, int64_t n, uint32_t* out,
 int psk_heavy_cap() { return PS_HEAVY_MAX; }
 
 void psk_scan_tiles(hipStream_t s, const unsigned long long* tcnt, int64_t n, unsigned long long* tstart,
-                    unsigned long long* partial, uint32_t* total_out, PsCounters* c, uint32_t* heavy, int* flag)
+                    unsigned long long* partial, uint32_t* total_out, unsigned long long* wide, int64_t seg_cap, PsCounters* c,
+                    uint32_t* heavy, int* flag)
 {
     if (n <= SCAN_DIRECT_MAX) {
         hipLaunchKernelGGL(k_scan_direct, dim3(gsz(n, DIRECT_BLOCK)), dim3(1024), 0, s, tcnt, n, tstart,
-                           total_out, c, heavy, flag);
+                           total_out, wide, seg_cap, c, heavy, flag);
         return;
     }
     int nb = psk_scan_blocks(n);
     hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(256), 0, s, tcnt, n, partial, c);
-    hipLaunchKernelGGL(k_scan_final, dim3(nb), dim3(256), 0, s, tcnt, n, partial, nb, tstart, total_out, c, heavy, flag);
+    hipLaunchKernelGGL(k_scan_final, dim3(nb), dim3(256), 0, s, tcnt, n, partial, nb, tstart, total_out, wide, seg_cap, c, heavy, flag);
 }
 
 
 void psk_span(hipStream_t s, const PsTri* tris, const uint32_t* row_off, const uint32_t* bstart, int64_t T,
               PsSpan* spans, unsigned long long* tcnt, const PsView* views, int n_views, int chunk_w, int tile_rows,
-              int64_t cap, uint32_t* heavy, uint32_t* wide, PsCounters* cnt, int* flag)
+              int64_t cap, uint32_t* heavy, unsigned long long* wide, PsCounters* cnt, int* flag)
 {
     int g = gsz(cap, 256); if (g > 2048) g = 2048;
     const int tile_cols = 64 / tile_rows;
@@ -2659,12 +2823,12 @@ void psk_span(hipStream_t s, const PsTri* tris, const uint32_t* row_off, const u
 
 void psk_segments(hipStream_t s, const PsSpan* spans, const uint32_t* row_off, int64_t T, const PsFrame& f,
                   const PsTri* tris, const PsDraw* draws, const float* vary, int nvs, unsigned long long* tcnt, PsSeg* segs,
-                  float* ck, int64_t span_cap, int64_t seg_cap, const uint32_t* wide, PsCounters* cnt, int* flag)
+                  float* ck, int64_t span_cap, int64_t seg_cap, const unsigned long long* wide, PsCounters* cnt, int* flag)
 {
     int g = gsz(span_cap, 256); if (g > 2048) g = 2048;
 #define SG_LAUNCH(G)                                                                                                  \
     hipLaunchKernelGGL(k_segments<G>, dim3(g), dim3(256), 0, s, spans, row_off, T, f, tris, draws, vary, nvs, tcnt,   \
-                       segs, ck, seg_cap, wide, cnt, flag)
+                       segs, ck, seg_cap, wide, PS_WIDE_PER(span_cap), cnt, flag)
     static_assert(PS_MAX_NV <= 24, "a lane per varying float beside the 8 of the record");
     if (nvs <= 8) SG_LAUNCH(16);
     else SG_LAUNCH(32);

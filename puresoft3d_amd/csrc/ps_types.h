@@ -128,7 +128,20 @@ struct PsView {
     int cclear_rows; uint32_t cclear_value;
 };
 
-#define PS_RUN_OWN 0x80000000u
+// The waves of 64 span items that hold a wide span: PS_WIDE_LISTS lists (all
+// waves of a flush on one address took 12 ns each), wave w on list w % 64.
+// Word PS_WIDE_STEP * l, on a cache line of its own, is the head of list l: how
+// many (bits 0-19) and their pieces (from bit 20 on).  From PS_WIDE_BEFORE on,
+// written by the tile scan, the waves | pieces << 32 on the lists before l, and
+// the total.  From PS_WIDE_REC on `per` words for each list: a wave's index |
+// the first of its pieces among the list's << 32.
+#define PS_WIDE_LISTS 64
+#define PS_WIDE_STEP 16
+#define PS_WIDE_COUNT 0xfffffull
+#define PS_WIDE_BEFORE (PS_WIDE_LISTS * PS_WIDE_STEP)
+#define PS_WIDE_REC (PS_WIDE_BEFORE + PS_WIDE_LISTS + 16)
+#define PS_WIDE_PER(span_cap) (((int64_t)(span_cap) + 64 * PS_WIDE_LISTS - 1) / (64 * PS_WIDE_LISTS))
+#define PS_WIDE_WORDS(span_cap) (PS_WIDE_REC + PS_WIDE_LISTS * PS_WIDE_PER(span_cap))
 
 // Flush-wide parameters passed by value to kernels.
 struct PsFrame {
@@ -139,13 +152,11 @@ struct PsFrame {
     int64_t n_tiles, n_stiles;
     const PsView* views;
     // tile lists.  Each wave of 64 span items writes its pieces of a tile as
-    // one run of consecutive pieces, in span order; a wave that holds a wide
-    // span writes one run per span instead.  tstart[t] holds the first piece
-    // (low 32 bits) and the first run (bits 32-62) of tile t (n_tiles + 1
-    // entries); run r is runs[2r] = its first piece, with PS_RUN_OWN set in a
-    // run of one span, and runs[2r+1] = its key: wave << 12 | pieces - 1, or
-    // wave << 12 | span in the wave << 6 | pieces - 1.  Ordered by key, the
-    // runs of a tile are in submission order.
+    // one run of consecutive pieces, in span order.  tstart[t] holds the first
+    // piece (low 32 bits) and the first run (bits 32-62) of tile t (n_tiles + 1
+    // entries); run r is runs[2r] = its first piece, runs[2r+1] = wave << 12 |
+    // pieces - 1.  The pieces of the waves that hold a wide span lie after
+    // those that tstart counts, a block for each of these waves.
     // runs2 is scratch of the same size for ordering long run lists.
     const unsigned long long* tstart;
     uint32_t* runs;

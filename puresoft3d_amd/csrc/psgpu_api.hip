@@ -148,7 +148,7 @@ struct FlushBufs {
     DevBuf<float> grad;   // per triangle: screen gradients for the mip level (8 floats)
     DevBuf<uint32_t> nrows, rowoff, partial;
     DevBuf<uint32_t> bstart;   // triangle of every 64th row item, written by the row scan
-    DevBuf<uint32_t> wide;     // count and list of the span waves that hold a wide span
+    DevBuf<unsigned long long> wide;   // lists of the span waves that hold a wide span
     DevBuf<PsSpan> spans;
     // tile lists: per-tile piece and run counts (zero between flushes: the
     // piece kernel counts them back down), their scan, the scan's block sums,
@@ -569,7 +569,7 @@ int size_flush_scratch(psgpu_ctx* c, int64_t T, int nvs, int64_t n_tiles)
         return fail(c, PSGPU_ERR_NOMEM, "more than %lld spans or %lld pieces in one flush", (long long)c->max_spans,
                     (long long)c->max_segs);
     if ((rc = ensure(c, b.partial, row_partials(T))) ||
-        (rc = ensure(c, b.bstart, b.span_cap / 64 + 2)) || (rc = ensure(c, b.wide, b.span_cap / 64 + 3)) || (rc = ensure(c, b.spans, b.span_cap)) ||
+        (rc = ensure(c, b.bstart, b.span_cap / 64 + 2)) || (rc = ensure(c, b.wide, PS_WIDE_WORDS(b.span_cap))) || (rc = ensure(c, b.spans, b.span_cap)) ||
         (rc = ensure(c, b.segs, b.seg_cap)) || (rc = ensure(c, b.ck, (size_t)b.seg_cap * nvs)) ||
         (rc = ensure(c, b.runs, (size_t)b.seg_cap * 2)) || (rc = ensure(c, b.runs2, (size_t)b.seg_cap * 2)) ||
         (rc = ensure(c, b.tstart, n_tiles + 1)) || (rc = ensure(c, b.tpartial, psk_scan_blocks(n_tiles) + 1)) ||
@@ -656,7 +656,8 @@ int run_flush(psgpu_ctx* c, const Cmd& cmd, uint8_t* staged)
     }
     {
         ProfScope p(c, "scan_tiles");
-        psk_scan_tiles(s, c->fb.tcnt.p, f.n_tiles, c->fb.tstart.p, c->fb.tpartial.p, c->d_sizes + 1, c->d_cnt, heavy, flag);
+        psk_scan_tiles(s, c->fb.tcnt.p, f.n_tiles, c->fb.tstart.p, c->fb.tpartial.p, c->d_sizes + 1, c->fb.wide.p, c->fb.seg_cap,
+                       c->d_cnt, heavy, flag);
     }
     f.tstart = c->fb.tstart.p;
     f.runs = c->fb.runs.p;
@@ -1241,9 +1242,8 @@ bool carve_flush(Arena& a, Arena& slack, const FlushShape& sh, FlushBufs& b)
     // bytes per span: record, entry of the row-start table, and 1.5 pieces of
     // record, checkpoint and two run records
     const double per_span = 32 + 4.0 / 64 + 1.5 * (sizeof(PsSeg) + 4.0 * sh.nvs + 16);
-    // the list of wide waves has a word per 64 spans: 153 KiB for the most
-    // spans that the array holds
-    static_assert(PSGPU_STATIC_SCRATCH_BYTES / (32 + (sizeof(PsSeg) + 20) * 3 / 2) / 64 * sizeof(uint32_t) + (64 << 10) <= kStaticSlack,
+    // the lists of wide waves: 310 KiB for the most spans that the array holds
+    static_assert(PS_WIDE_WORDS(PSGPU_STATIC_SCRATCH_BYTES / (32 + (sizeof(PsSeg) + 20) * 3 / 2)) * 8 + (64 << 10) <= kStaticSlack,
                   "the lists fit into the slack");
     size_t left = a.cap - a.used;
     int64_t spans = (int64_t)((double)left / per_span);
@@ -1253,7 +1253,7 @@ bool carve_flush(Arena& a, Arena& slack, const FlushShape& sh, FlushBufs& b)
         FlushBufs x = b;
         x.span_cap = spans;
         x.seg_cap = spans * 3 / 2;
-        if (t.take(x.bstart, x.span_cap / 64 + 2) && u.take(x.wide, x.span_cap / 64 + 3) &&
+        if (t.take(x.bstart, x.span_cap / 64 + 2) && u.take(x.wide, PS_WIDE_WORDS(x.span_cap)) &&
             t.take(x.spans, x.span_cap) && t.take(x.segs, x.seg_cap) &&
             t.take(x.ck, (size_t)x.seg_cap * sh.nvs) && t.take(x.runs, (size_t)x.seg_cap * 2) &&
             t.take(x.runs2, (size_t)x.seg_cap * 2)) {

@@ -8,8 +8,9 @@ parameters (albedo scale, specular exponent):
 
     c = albedo_scale * bilinear(tex, u, v) * max(n.L, 0) + ks * max(n.H, 0)^spec_exp
 
-with a hand-written adjoint (psgpu_diff_backward): texel gradients are
-scattered with atomics, parameter gradients are reduced per wavefront.
+with a hand-written adjoint (psgpu_diff_backward): texel gradients
+are added up over pixels that share texels before they go out with atomics,
+parameter gradients are summed in 64 bits over a block's pixels.
 
 torch must be imported before libpsgpu is first loaded, so that both use the
 one HIP runtime torch brings (this module imports torch first).

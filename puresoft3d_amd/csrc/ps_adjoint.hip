@@ -149,6 +149,14 @@ __global__ void __launch_bounds__(256) k_diff_forward(DiffArgs A, const float* _
 // is the chain of reductions and barriers of a tile and its LDS atomics.
 const int kTileW = 32, kTileH = 32, kDiffThreads = 512, kDiffWaves = kDiffThreads / 64;
 const int kLdsTexels = 3400;   // 40 KiB
+// Images of up to so many pixels (see k_diff_backward_small), and of up to so
+// many a texel and beside them: of few texels all waves share some.
+// In tiles and there, us: 8x8 texels, 40^2 pixels 9.8 and 8.2, 64^2 9.8 and
+// 11.3; 16x16, 80^2 10.7 and 9.6, 128^2 11.0 and 13.5; 32x32, 181x140 12.4 and
+// 11.9.  The same texture magnified until 181x140 pixels lie in four texels
+// takes 11.4 and 13.1, and more beyond; 200^2 pixels with a texel each 25 and 13.
+const int64_t kSmallPixels = 32768, kSmallPerTexel = 24, kSmallBeside = 1024;
+const int kSmallTile = 16, kSmallThreads = kSmallTile * kSmallTile;
 
 // Whether the texture stays in LDS: with the first column and row again at the
 // end, so that footprints need not wrap there either.
@@ -195,19 +203,28 @@ __device__ __forceinline__ TexRect tex_rect(const int* e)
     return r;
 }
 
-// One step of adding up a quad's contributions: lanes whose key equals their
-// partner's (the lane DPP control CTRL names) take both, and the upper of the
-// two drops out (key -1).  Called by every lane.
-template <int CTRL>
+// the value that lane ^ X has
+template <int X>
+__device__ __forceinline__ int lane_xor(int v)
+{
+    if (X == 1) return __builtin_amdgcn_mov_dpp(v, 0xb1, 0xf, 0xf, false);   // quad_perm [1,0,3,2]
+    if (X == 2) return __builtin_amdgcn_mov_dpp(v, 0x4e, 0xf, 0xf, false);   // quad_perm [2,3,0,1]
+    return __shfl_xor(v, X, 64);
+}
+
+// One step of adding up the lanes' contributions: lanes whose key equals that
+// of lane ^ X take both, and the upper of the two drops out (key -1).  Called
+// by every lane.
+template <int X>
 __device__ __forceinline__ void merge_lanes(int& key, float* c, bool upper)
 {
     // read before any branch: a lane switched off by one would read as 0
-    const int other = __builtin_amdgcn_mov_dpp(key, CTRL, 0xf, 0xf, false);
+    const int other = lane_xor<X>(key);
     const bool same = (other == key) & (key >= 0);
     if (!__any(same)) return;
 #pragma unroll
     for (int k = 0; k < 12; k++) {
-        const float o = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(c[k]), CTRL, 0xf, 0xf, false));
+        const float o = __int_as_float(lane_xor<X>(__float_as_int(c[k])));
         c[k] = same ? c[k] + o : c[k];
     }
     if (same && upper) key = -1;
@@ -308,8 +325,8 @@ __global__ void __launch_bounds__(kDiffThreads) k_diff_backward(DiffArgs A, cons
             }
 #pragma unroll
             for (int q = 0; q < 2; q++) {
-                merge_lanes<0xb1>(key[q], c[q], t & 1);
-                merge_lanes<0x4e>(key[q], c[q], t & 2);
+                merge_lanes<1>(key[q], c[q], t & 1);
+                merge_lanes<2>(key[q], c[q], t & 2);
             }
 #pragma unroll
             for (int q = 0; q < 2; q++) {
@@ -382,6 +399,104 @@ __global__ void __launch_bounds__(kDiffThreads) k_diff_backward(DiffArgs A, cons
     }
 }
 
+// The same for an image of few pixels, which would leave most CUs without a
+// tile (64x64 pixels: four tiles), each tile a chain of extents, LDS sums and a
+// pass over its rectangle.  Here a thread has one pixel and adds its gradients
+// to the texture itself, after those of pixels with the same texels were added
+// up: in the wave's 8 x 8 pixels by halves (the lanes are in Morton order, and
+// a step without equals costs one comparison), then the first lanes of the
+// block's waves.  Bound by the latency of the loads and of 12 scattered atomics
+// a lane; where the texture is magnified so far that waves share texels, by
+// the atomics on those.
+// 64x64 pixels and a 250x130 texture 18.6 us in tiles, 5.6 here (without
+// adding up 5.3, but 123 where all of the image lies in four texels: 8 here,
+// 10 in tiles); 40x40 and 1024^2 17.8 and 7.1, 181x140 18.2 and 9.7.
+__global__ void __launch_bounds__(kSmallThreads) k_diff_backward_small(DiffArgs A, const float* __restrict__ gbuf,
+                                                             const float* __restrict__ tex, const float* __restrict__ params,
+                                                             const float* __restrict__ gout, float* __restrict__ gtex,
+                                                             float* __restrict__ gparams, int blocks_x)
+{
+    __shared__ double sums[2][kSmallThreads / 64];
+    __shared__ int first[kSmallThreads / 64];      // key and contributions of each wave's first lane
+    __shared__ float firsts[kSmallThreads / 64][12];
+    const int t = threadIdx.x;
+    const int by = (int)blockIdx.x / blocks_x, bx = (int)blockIdx.x - by * blocks_x;
+    // the lane's bits are those of x and y in turn: lanes 4, 16 and 64 of a
+    // kind are squares of pixels
+    const int x = bx * kSmallTile + (t >> 6 & 1) * 8 + ((t & 1) | (t >> 1 & 2) | (t >> 2 & 4));
+    const int y = by * kSmallTile + (t >> 7) * 8 + ((t >> 1 & 1) | (t >> 2 & 2) | (t >> 3 & 4));
+    double ga = 0.0, ge = 0.0;
+    int key = -1;
+    int64_t idx[4] = {0, 0, 0, 0};
+    float c[12];
+#pragma unroll
+    for (int k = 0; k < 12; k++) c[k] = 0.0f;
+    if (x < A.W && y < A.H) {
+        const int64_t p = (int64_t)y * A.W + x;
+        const float a = params[0], e = params[1];
+        const Geo g = geometry(A, gbuf, p, e);
+        if (g.covered) {
+            float w[4];
+            footprint(A, g.u, g.v, idx, w);
+            key = (int)idx[0];
+            const float go[3] = {gout[p * 3], gout[p * 3 + 1], gout[p * 3 + 2]};
+            const float al = a * g.lam;
+#pragma unroll
+            for (int ch = 0; ch < 3; ch++) {
+                const float s = ((w[0] * tex[idx[0] * 3 + ch] + w[1] * tex[idx[1] * 3 + ch]) + w[2] * tex[idx[2] * 3 + ch]) +
+                                w[3] * tex[idx[3] * 3 + ch];
+                ga += (double)(go[ch] * s * g.lam);
+                const float gc = go[ch] * al;
+#pragma unroll
+                for (int k = 0; k < 4; k++) c[k * 3 + ch] = gc != 0.0f && w[k] != 0.0f ? gc * w[k] : 0.0f;
+            }
+            if (g.s > 0.0f) ge = (double)(((go[0] + go[1]) + go[2]) * g.spec * logf(g.s));
+        }
+    }
+    merge_lanes<1>(key, c, t & 1);
+    merge_lanes<2>(key, c, t & 2);
+    merge_lanes<4>(key, c, t & 4);
+    merge_lanes<8>(key, c, t & 8);
+    merge_lanes<16>(key, c, t & 16);
+    merge_lanes<32>(key, c, t & 32);
+    if ((t & 63) == 0) {
+        first[t >> 6] = key;
+#pragma unroll
+        for (int k = 0; k < 12; k++) firsts[t >> 6][k] = c[k];
+    } else if (key >= 0) {
+#pragma unroll
+        for (int k = 0; k < 12; k++)
+            if (c[k] != 0.0f) unsafeAtomicAdd(gtex + idx[k / 3] * 3 + k % 3, c[k]);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        ga += __shfl_xor(ga, o, 64);
+        ge += __shfl_xor(ge, o, 64);
+    }
+    if ((t & 63) == 0) { sums[0][t >> 6] = ga; sums[1][t >> 6] = ge; }
+    __syncthreads();
+    if (t < 12) {
+        float v = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kSmallThreads / 64; w++) {
+            const int k = first[w];
+            if (k < 0) continue;
+            v += firsts[w][t];
+            if (w + 1 < kSmallThreads / 64 && first[w + 1] == k) continue;
+            int ix = k % A.tw, iy = k / A.tw;
+            if ((t / 3 & 1) && ++ix == A.tw) ix = 0;
+            if (t >= 6 && ++iy == A.th) iy = 0;
+            if (v != 0.0f) unsafeAtomicAdd(gtex + ((int64_t)iy * A.tw + ix) * 3 + t % 3, v);
+            v = 0.0f;
+        }
+    } else if (t >= 64 && t < 66) {
+        double s = 0.0;
+#pragma unroll
+        for (int w = 0; w < kSmallThreads / 64; w++) s += sums[t - 64][w];
+        unsafeAtomicAdd(gparams + t - 64, (float)s);
+    }
+}
+
 int make_args(const psgpu_diff_desc* d, DiffArgs& A)
 {
     if (!d || d->width < 1 || d->height < 1 || d->tex_w < 1 || d->tex_h < 1) return PSGPU_ERR_INVALID;
@@ -414,6 +529,13 @@ extern "C" int psgpu_diff_backward(psgpu_ctx* ctx, const psgpu_diff_desc* desc, 
     if (!ctx || !gbuf || !tex || !params || !grad_out || !grad_tex || !grad_params || make_args(desc, A))
         return PSGPU_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
+    const int64_t pixels = (int64_t)A.W * A.H, texels = (int64_t)A.tw * A.th;
+    if (pixels <= kSmallPixels && texels <= INT_MAX && pixels <= kSmallBeside + kSmallPerTexel * texels) {
+        const int blocks_x = (A.W + kSmallTile - 1) / kSmallTile, blocks_y = (A.H + kSmallTile - 1) / kSmallTile;
+        hipLaunchKernelGGL(k_diff_backward_small, dim3((unsigned)(blocks_x * blocks_y)), dim3(kSmallThreads), 0, s, A, gbuf, tex, params,
+                           grad_out, grad_tex, grad_params, blocks_x);
+        return hipGetLastError() == hipSuccess ? PSGPU_OK : PSGPU_ERR_DEVICE;
+    }
     const int tiles_x = (int)(((int64_t)A.W + kTileW - 1) / kTileW);
     const int64_t n_tiles = tiles_x * (((int64_t)A.H + kTileH - 1) / kTileH);
     // two blocks a CU; one where every block adds to the whole of a small texture

@@ -1923,7 +1923,11 @@ __device__ __forceinline__ void ps_store_run(uint32_t* p, int n, const uint32_t*
 // 1024^2 (3.7M) 158 -> 77, 515x389 (86k, as long as its longest tile) 37 ->
 // 21; 1920x1080 in 16x8 tiles (1.1M) 33 -> 22.
 // KCW: the chunk width when it is 1, 2, 4 or 8 (a batch's pixels are then
-// unrolled and share their rounds), else 0.
+// unrolled and share their rounds), else 0: of a chunk of 16 pixels or more a
+// piece covers so few that rounds over all of them mostly pass lanes by, and
+// each lane walks the batch's pieces of its own chunk instead.  1920x1080
+// terrain in 16x8 tiles 209 -> 184 us, 64x4 726 -> 339; a lane's pieces from
+// lists split in LDS took 201 and 417.
 template <bool DEBUG, int KCW>
 __global__ void __launch_bounds__(512, 5) k_raster(const PsSpan* __restrict__ spans, const PsSeg* __restrict__ segs,
                          const PsTri* __restrict__ tris, const PsDraw* __restrict__ draws, PsFrame f, int64_t n_tiles,
@@ -2056,12 +2060,14 @@ __global__ void __launch_bounds__(512, 5) k_raster(const PsSpan* __restrict__ sp
                 h ^= h >> 16; h *= 0x85ebca6bu; h ^= h >> 13; h *= 0xc2b2ae35u; h ^= h >> 16;
                 th = h;
             }
-            // lanes of the same chunk
-            uint64_t same = ~0ull;
+            // lanes of the same chunk; with wide chunks, those of the chunk
+            // that is the lane's
+            const int of = KCW ? key : lane;
+            uint64_t same = KCW ? ~0ull : __ballot(valid);
 #pragma unroll
             for (int bit = 0; bit < 6; bit++) {
                 const uint64_t m = __ballot((key >> bit) & 1);
-                same &= ((key >> bit) & 1) ? m : ~m;
+                same &= ((of >> bit) & 1) ? m : ~m;
             }
             const bool all_test = __all(test || !valid);
             // candidates before this lane at the same pixel
@@ -2134,19 +2140,60 @@ __global__ void __launch_bounds__(512, 5) k_raster(const PsSpan* __restrict__ sp
                     ps_lds_turn();
                 }
             } else {
-                for (int k = 0; k < CW; k++) {
-                    const bool in = k >= a && k <= b;
-                    if (!__any(in)) continue;
-                    const float z = depth_at(in);
-                    if (DEBUG && in) drawn(k);
-                    const bool cand = in && -1.0f < z;
-                    const int rank = rank_of(cand);
-                    for (int r = 0; __any(cand && rank >= r); r++) {
-                        fragment(cand && rank == r, k, z, pix[k * 64 + key]);
-                        if (DEBUG) __threadfence();
-                        ps_lds_turn();
+                // each lane walks the pieces of its own chunk, one after the
+                // other, four pixels at a time
+                const int ends = a | b << 8 | (int)(ra.x >> 26) << 16;
+                int k = 1, last = 0, how = 0, code = 0, hash = 0, id = 0;
+                float f2 = 0.0f, zn = 0.0f, f2s = 0.0f, zns = 0.0f;
+                auto from = [](int j, int v) { return __builtin_amdgcn_ds_bpermute(j * 4, v); };
+                auto fromf = [&](int j, float v) { return __int_as_float(from(j, __float_as_int(v))); };
+                while (__any((same != 0) | (k <= last))) {
+                    const bool take = (k > last) & (same != 0);
+                    if (__any(take)) {
+                        const int j = __builtin_ctzll(same | 1ull << 63);
+                        const int e = from(j, ends), wj = from(j, (int)wcode);
+                        const float g0 = fromf(j, cf2), g1 = fromf(j, pz), g2 = fromf(j, cst), g3 = fromf(j, pst);
+                        const int hj = DEBUG ? from(j, (int)th) : 0, ij = DEBUG ? from(j, tid) : 0;
+                        if (take) {
+                            k = e & 0xff; last = e >> 8 & 0xff; how = e >> 16;
+                            code = wj; f2 = g0; zn = g1; f2s = g2; zns = g3; hash = hj; id = ij;
+                            same &= same - 1;
+                        }
                     }
+                    uint2 cur[4];
+                    float z[4];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) cur[j] = pix[min(k + j, CW - 1) * 64 + lane];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {   // interpolateNextStep (interp.cpp:82-92)
+                        const float r = 1.0f / f2;
+                        z[j] = zn * r;
+                        f2 += f2s;
+                        zn += zns;
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {   // fragthrd.cpp:216-237
+                        const float dd = how & PSGPU_TEST_DEPTH ? __uint_as_float(cur[j].x) : 1.0f;
+                        const bool in = k + j <= last, pass = in & (-1.0f < z[j]) & (z[j] - dd < -0.0001f);
+                        if (how & PSGPU_UPDATE_DEPTH) cur[j].x = __float_as_uint(z[j]);
+                        if (how & 4) cur[j].y = (uint32_t)code;
+                        if (pass) pix[(k + j) * 64 + lane] = cur[j];
+                        passes += pass ? 1u : 0u;
+                        dirty |= pass & ((how & PSGPU_UPDATE_DEPTH) != 0);
+                        if (DEBUG && in) {
+                            const int64_t at = (int64_t)y * VW + X0 + k + j;
+                            f.dbg_rcount[at] += 1;
+                            f.dbg_rhash[at] ^= (uint32_t)hash;
+                            if (pass) {
+                                f.dbg_pcount[at] += 1;
+                                f.dbg_phash[at] ^= (uint32_t)hash;
+                                f.dbg_last[at] = id;
+                            }
+                        }
+                    }
+                    k += 4;
                 }
+                ps_lds_turn();
             }
         }
     }
@@ -2189,7 +2236,11 @@ __global__ void __launch_bounds__(512, 5) k_raster(const PsSpan* __restrict__ sp
 // (each lane its chunk's pieces, one after the other, and a piece's pixels one
 // after the other) and after, a layer over a 960x540 scene: blended 57 -> 30
 // us, discarding 35 -> 17.  Unrolled over the chunk (KCW) the texture reads of
-// its pixels overlap: 34 -> 30 and 21 -> 17; other widths walk it.
+// its pixels overlap: 34 -> 30 and 21 -> 17; other widths go through its
+// pixels in turn (KCW 0), but of 64 pixels each lane walks the pieces of its own
+// chunk, as in k_raster: 64x64 tiles 643 -> 502 us (32x32 1,134 -> 1,264, 16x16
+// 592 -> 688 the frame, since a batch's pieces lie in few chunks and lanes
+// without one shade along).
 template <int PROG, bool DEBUG, int KCW>
 __global__ void __launch_bounds__(512) k_raster_imm(const PsSpan* __restrict__ spans, const PsSeg* __restrict__ segs,
                          const PsTri* __restrict__ tris, const PsDraw* __restrict__ draws, PsFrame f, int64_t n_tiles,
@@ -2201,6 +2252,7 @@ __global__ void __launch_bounds__(512) k_raster_imm(const PsSpan* __restrict__ s
     extern __shared__ uint32_t lds[];
     if (ps_poisoned(cnt)) return;
     ps_commit_pending(cnt);
+    constexpr bool UNROLL = KCW > 0 && KCW <= 4, OWN = KCW > 4;
     const int CW = KCW ? KCW : f.chunk_w;
     int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int waves = blockDim.x >> 6;
@@ -2236,8 +2288,8 @@ __global__ void __launch_bounds__(512) k_raster_imm(const PsSpan* __restrict__ s
     if (in_lds) ps_sort_runs_lds(rl, nr, lruns, n_list);
     else if (nr > 64) rl = ps_order_runs(f.runs + 2 * (size_t)r0, f.runs2 + 2 * (size_t)r0, nr, (uint32_t*)lruns, n_list);
     // the chunk as the flush finds it, to write back what it changes
-    uint32_t d0[KCW > 0 ? KCW : 1], c0[KCW > 0 ? KCW : 1];
-    if constexpr (KCW > 0) {
+    uint32_t d0[UNROLL ? KCW : 1], c0[UNROLL ? KCW : 1];
+    if constexpr (UNROLL) {
         ps_load_run<KCW>((const uint32_t*)drow + X0, ncol, d0);
 #pragma unroll
         for (int k = 0; k < KCW; k++) c0[k] = 0;
@@ -2332,12 +2384,14 @@ __global__ void __launch_bounds__(512) k_raster_imm(const PsSpan* __restrict__ s
                 h ^= h >> 16; h *= 0x85ebca6bu; h ^= h >> 13; h *= 0xc2b2ae35u; h ^= h >> 16;
                 th = h;
             }
-            // lanes of the same chunk
-            uint64_t same = ~0ull;
+            // lanes of the same chunk; with wide chunks, those of the chunk
+            // that is the lane's
+            const int of = OWN ? lane : key;
+            uint64_t same = OWN ? __ballot(valid) : ~0ull;
 #pragma unroll
             for (int bit = 0; bit < 6; bit++) {
                 const uint64_t bm = __ballot((key >> bit) & 1);
-                same &= ((key >> bit) & 1) ? bm : ~bm;
+                same &= ((of >> bit) & 1) ? bm : ~bm;
             }
             const bool all_test = __all(test || !valid);
             // candidates before this lane at the same pixel
@@ -2392,7 +2446,7 @@ __global__ void __launch_bounds__(512) k_raster_imm(const PsSpan* __restrict__ s
                     f.dbg_last[at] = tid;
                 }
             };
-            if constexpr (KCW > 0) {
+            if constexpr (UNROLL) {
                 float z[KCW], r[KCW];
                 uint2 cur[KCW];
                 bool cand[KCW], some = false;
@@ -2426,6 +2480,59 @@ __global__ void __launch_bounds__(512) k_raster_imm(const PsSpan* __restrict__ s
 #pragma unroll
                     for (int k = 0; k < KCW; k++) cur[k] = pix[k * 64 + key];
                 }
+            } else if constexpr (OWN) {
+                // each lane walks the pieces of its own chunk, one after the other
+                const int ends = a | b << 8 | (int)(ra.x >> 26) << 16;
+                int k = 1, last = 0, how = 0, dj = 0;
+                float f2 = 0.0f, zn = 0.0f, f2s = 0.0f, zns = 0.0f;
+                float ws[NV > 0 ? NV : 1], wt[NV > 0 ? NV : 1];
+#pragma unroll
+                for (int i = 0; i < NV; i++) ws[i] = wt[i] = 0.0f;
+                auto from = [](int j, int v) { return __builtin_amdgcn_ds_bpermute(j * 4, v); };
+                auto fromf = [&](int j, float v) { return __int_as_float(from(j, __float_as_int(v))); };
+                while (__any((same != 0) | (k <= last))) {
+                    const bool take = (k > last) & (same != 0);
+                    if (__any(take)) {
+                        const int j = __builtin_ctzll(same | 1ull << 63);
+                        const int e = from(j, ends), g = from(j, di);
+                        const float g0 = fromf(j, cf2), g1 = fromf(j, pz), g2 = fromf(j, cst), g3 = fromf(j, pst);
+                        if (take) {
+                            k = e & 0xff; last = e >> 8 & 0xff; how = e >> 16;
+                            dj = g; f2 = g0; zn = g1; f2s = g2; zns = g3;
+                            same &= same - 1;
+                        }
+#pragma unroll
+                        for (int i = 0; i < NV; i++) {
+                            const float s0 = fromf(j, vs[i]), s1 = fromf(j, vt[i]);
+                            ws[i] = take ? s0 : ws[i];
+                            wt[i] = take ? s1 : wt[i];
+                        }
+                    }
+                    uint2* at = pix + min(k, CW - 1) * 64 + lane;
+                    uint2 cur = *at;
+                    const float r = 1.0f / f2, z = zn * r, dd = how & PSGPU_TEST_DEPTH ? __uint_as_float(cur.x) : 1.0f;
+                    const bool pass = (k <= last) & (-1.0f < z) & (z - dd < -0.0001f);
+                    if (__any(pass)) {
+                        const PsDraw& dr = draws[dj];
+                        float v[NV > 0 ? NV : 1];
+#pragma unroll
+                        for (int i = 0; i < NV; i++) v[i] = ws[i] * r;
+                        uint32_t col = 0;
+                        const int fr = P::fpi(dr, v, col);
+                        const bool depth = pass & ((how & PSGPU_UPDATE_DEPTH) != 0) & (fr != 2);
+                        const bool paint = COLOUR & pass & ((how & 4) != 0) & (fr == 1);
+                        if (depth) cur.x = __float_as_uint(z);
+                        if (paint) cur.y = (dr.behavior & PSGPU_ALPHABLEND) ? ps_blend4(cur.y, col) : col;
+                        if (depth | paint) *at = cur;
+                    }
+                    passes += pass ? 1u : 0u;
+                    f2 += f2s;
+                    zn += zns;
+#pragma unroll
+                    for (int i = 0; i < NV; i++) ws[i] += wt[i];
+                    k++;
+                }
+                ps_lds_turn();
             } else {
                 for (int k = 0; k < CW; k++) {
                     const bool in = k >= a && k <= b;
@@ -2448,7 +2555,7 @@ __global__ void __launch_bounds__(512) k_raster_imm(const PsSpan* __restrict__ s
     }
     // the colours that changed, then the depths of chunks in which one did
     bool dirty = dclear;
-    if constexpr (KCW > 0) {
+    if constexpr (UNROLL) {
         uint32_t dv[KCW];
 #pragma unroll
         for (int k = 0; k < KCW; k++) {
@@ -2875,6 +2982,7 @@ void psk_raster_imm(hipStream_t s, int prog, bool debug, const PsSpan* spans, co
     case P:                                                                                                          \
         if (debug) RI_LAUNCH(P, true, 0);                                                                            \
         else if (f.chunk_w == 4) RI_LAUNCH(P, false, 4);                                                             \
+        else if (f.chunk_w == 64) RI_LAUNCH(P, false, 64);                                                           \
         else RI_LAUNCH(P, false, 0);                                                                                 \
         break;
     switch (prog) {

@@ -14,9 +14,10 @@ LDS_LIMIT = 65536
 
 
 def lds_bytes(chunk_width, waves):
-    """LDS of the raster kernel: per wave, depth and winner columns plus 128
-    staged pieces of 7 words and 128 words of counts (ps_kernels.hip RA_WORDS)"""
-    return waves * (chunk_width * 64 * 2 + 128 * 7 + 128) * 4
+    """LDS that a tiling is taken or refused by: per wave, depth and winner of
+    the tile's pixels plus 1,024 words, which the raster kernels' run lists stay
+    below (ps_kernels.hip psk_raster_lds)"""
+    return waves * (chunk_width * 64 * 2 + 1024) * 4
 
 
 def candidates(min_side=8, max_side=64, waves=(1, 2, 4, 8)):

@@ -50,7 +50,9 @@ PS_DEV void ps_m4v4(float* r, const float* m, const float* v)
 // reciprocal as the two operations do (Markstein, IBM J. Res. Dev. 34, 1990),
 // but for an s whose bits are all ones: 1 / s lies next to the midpoint of two
 // floats.  That is the root of the last two floats below a power of four.
-// Every float has been compared.
+// All 2,139,095,041 floats from 0 to infinity were compared with the host's root
+// and division once, none different; the tests compare two binades, the ends and
+// a million others.
 PS_DEV float ps_rsqrt(float x)
 {
     if (x >= 0x1p-100f && x <= 0x1p+100f && (__float_as_uint(x) & 0x7ffffeu) != 0x7ffffeu) {

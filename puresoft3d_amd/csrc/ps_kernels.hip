@@ -2731,8 +2731,8 @@ __global__ void __launch_bounds__(256, 6) k_shade(const PsSpan* __restrict__ spa
 // one texel is its own pair.  The levels stay in LDS between the steps, so the
 // chain reads its source once and a texture of up to 4,096 texels a side takes
 // two launches, for all its layers at once; one launch per level and layer
-// spent its time between launches (six layers of 1024^2: 60 launches, 233 us;
-// now 2 of 5 us, 41 with the waits around them).
+// spent its time between launches (six layers of 1024^2: 60 launches, 217 to
+// 222 us; now 2 of 5 to 8 us, 22 with the wait at their end).
 __device__ __forceinline__ uint32_t ps_mean4(uint32_t a, uint32_t b, uint32_t c, uint32_t d)
 {
     const uint32_t m = 0x00ff00ffu, r = 0x00020002u;   // two 16-bit sums a word

@@ -1200,7 +1200,7 @@ __global__ void __launch_bounds__(256, 8) k_span(const PsTri* __restrict__ tris,
         // pieces into LDS bins and one atomic per touched bin follows;
         // otherwise the wave visits its tiles in rounds (lane j adds the
         // j-th tile's counts, so a batch of tiles is one atomic), or, if it
-        // holds a wide span, the first span in a tile counts the run.
+        // holds a wide span, counts one run for each tile that some span covers.
         const uint32_t kmin = ps_wave_min(has ? st.g0 : 0xffffffffu);
         const uint32_t kmax = ps_wave_max(has ? st.g1 : 0u);
         if (kmin != 0xffffffffu && kmax - kmin < (uint32_t)SPAN_BINS) {
@@ -1227,33 +1227,30 @@ __global__ void __launch_bounds__(256, 8) k_span(const PsTri* __restrict__ tris,
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         } else if (in_wide) {
-            // 32 of a span's tiles at a time, without those that the spans
-            // before it in the same tile row cover.  (In rounds a wave across
-            // a 1080p screen makes 540: 68 us for two triangles, now 13.)
-            int ln = lane;
-            asm volatile("" : "+v"(ln));   // nothing of this is kept in registers outside
-            uint64_t before = 0;
+            // Tile row by tile row, 64 tiles at a time: each span marks in LDS
+            // where it begins and ends, and sums along the row tell the tiles
+            // that some span covers.  (In rounds a wave across a 1080p screen
+            // makes 540: 68 us for two triangles, now 11.  Each span looking
+            // through the others of its row took 84 us where this takes 37,
+            // 1080p terrain in tiles of 1x64, and 243 against 32, the demo
+            // scene in them.)
+            const uint32_t base_t = st.g0 - (uint32_t)st.tx0;
+            const int first_t = st.tx0, last_t = st.tx0 + (int)(st.g1 - st.g0);
             for (uint64_t todo = __ballot(has); todo;) {
-                const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)(st.g0 - (uint32_t)st.tx0), __builtin_ctzll(todo));
-                const uint64_t m = __ballot(has && st.g0 - (uint32_t)st.tx0 == r);
-                if ((m >> ln) & 1ull) before = m & ((1ull << ln) - 1ull);
-                todo &= ~m;
-            }
-            const int most = (int)ps_wave_max((uint32_t)__popcll(before));
-            const int nt = has ? (int)(st.g1 - st.g0) + 1 : 0, tiles = (int)ps_wave_max((uint32_t)nt);
-            const uint32_t cols = (uint32_t)st.tx0 | (uint32_t)(st.tx0 + nt - 1) << 16;   // below 2^16 each
-            for (int q0 = 0; q0 < tiles; q0 += 32) {
-                uint32_t bits = nt - q0 >= 32 ? ~0u : nt > q0 ? (1u << (nt - q0)) - 1u : 0u;
-                uint64_t m = before;
-                for (int k = 0; k < most; k++) {   // the same for every lane: all of them are read
-                    const uint32_t c = (uint32_t)__shfl((int)cols, m ? __builtin_ctzll(m) : lane, PS_WAVE);
-                    const int lo = (int)(c & 0xffffu) - st.tx0 - q0, hi = (int)(c >> 16) - st.tx0 - q0;
-                    if (m && lo < 32 && hi >= 0) bits &= ~((~0u << max(lo, 0)) & (~0u >> (31 - min(hi, 31))));
-                    m &= m - 1ull;
-                }
-                while (bits) {
-                    atomicAdd(&tcnt[st.g0 + (uint32_t)(q0 + __builtin_ctz(bits))], PS_TC_RUN);
-                    bits &= bits - 1u;
+                const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)base_t, __builtin_ctzll(todo));
+                const bool in_row = has && base_t == r;
+                todo &= ~__ballot(in_row);
+                const int from = (int)ps_wave_min(in_row ? (uint32_t)first_t : 0xffffffffu), to = (int)ps_wave_max(in_row ? (uint32_t)last_t : 0u);
+                for (int w0 = from; w0 <= to; w0 += PS_WAVE) {
+                    bins[lane] = 0;
+                    ps_lds_turn();
+                    if (in_row && first_t < w0 + PS_WAVE && last_t >= w0) {
+                        atomicAdd(&bins[max(first_t - w0, 0)], 1u);
+                        if (last_t + 1 < w0 + PS_WAVE) atomicAdd(&bins[last_t + 1 - w0], 0xffffffffu);
+                    }
+                    ps_lds_turn();
+                    if (ps_wave_incl_scan(bins[lane])) atomicAdd(&tcnt[r + (uint32_t)(w0 + lane)], PS_TC_RUN);
+                    ps_lds_turn();
                 }
             }
         } else {
